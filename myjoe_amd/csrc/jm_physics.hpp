@@ -234,9 +234,17 @@ __device__ __forceinline__ void jac_a(double A[5][5], const double *vel, double 
 // which = 0 computes A_L (d F / d U_L), which = 1 computes A_R. The reference
 // computes the two independently (calcSubSonicJacobeanHLLC uses only the
 // matching dSMdU/dpsdU), so evaluating one at a time gives the same bits.
-__device__ __forceinline__ void jac_hllc(double J[5][5], int which, double rhoL, const double *uL, double pL, double rhoR,
-                                      const double *uR, double pR, double gam, double area, const double *nVec,
-                                      double kL = 0.0, double kR = 0.0) {
+// out(5 i + j, J[i][j]) is called once per entry, row by row. The side and
+// the star side are chosen by selecting values, not by branching: the
+// reference's two forms of a row differ by a leading term that only the star
+// side's own matrix has (its place takes -0.0, and -0.0 + x is x) and, for
+// R, by the sign of dSM, so one straight row serves both. With the branches,
+// all 25 entries were live where they met (256 registers and more, one wave
+// per SIMD).
+template <class Out>
+__device__ __forceinline__ void jac_hllc_rows(Out out, int which, double rhoL, const double *uL, double pL,
+                                              double rhoR, const double *uR, double pR, double gam, double area,
+                                              const double *nVec, double kL = 0.0, double kR = 0.0) {
   const double gammaL = gam, gammaR = gam;
   double unL = dot3(uL, nVec);
   double uLuL = dot3(uL, uL);
@@ -266,129 +274,109 @@ __device__ __forceinline__ void jac_hllc(double J[5][5], int which, double rhoL,
   // fully supersonic to one side: F = F(U_L) or F(U_R)
   bool left_sup = (sM >= 0.0) && (sL > 0.0);
   bool right_sup = (sM < 0.0) && !(sR >= 0.0);
+  const bool W0 = which == 0;
+  // the requested side
+  const double rhoW = W0 ? rhoL : rhoR, pW = W0 ? pL : pR, unW = W0 ? unL : unR, uuW = W0 ? uLuL : uRuR;
+  const double sW = W0 ? sL : sR;
+  const double uW[3] = {W0 ? uL[0] : uR[0], W0 ? uL[1] : uR[1], W0 ? uL[2] : uR[2]};
   if (left_sup || right_sup) {
-    bool active = left_sup ? (which == 0) : (which == 1);
+    const bool active = left_sup ? W0 : !W0;
     if (active) {
       double nVecArea[3] = {nVec[0] * area, nVec[1] * area, nVec[2] * area};
-      if (which == 0)
-        jac_a(J, uL, pL, rhoL, nVecArea, gAvg);
-      else
-        jac_a(J, uR, pR, rhoR, nVecArea, gAvg);
+      double J[5][5];
+      jac_a(J, uW, pW, rhoW, nVecArea, gAvg);
+#pragma unroll
+      for (int k = 0; k < 25; k++) out(k, J[k / 5][k % 5]);
     } else {
 #pragma unroll
-      for (int i = 0; i < 5; i++)
-#pragma unroll
-        for (int j = 0; j < 5; j++) J[i][j] = 0.0;
+      for (int k = 0; k < 25; k++) out(k, 0.0);
     }
     return;
   }
   // star region on the side of the contact: K = L (sM >= 0) or R (sM < 0)
   const bool K_is_L = (sM >= 0.0);
-  double rhoK = K_is_L ? rhoL : rhoR;
-  const double *uK = K_is_L ? uL : uR;
-  double pK = K_is_L ? pL : pR, eK = K_is_L ? eL : eR, unK = K_is_L ? unL : unR;
-  double uKuK = K_is_L ? uLuL : uRuR, sK = K_is_L ? sL : sR;
-  double invSKmSs = 1.0 / (sK - sM);
-  double sKmuK = sK - unK;
-  double rhoSK = rhoK * sKmuK * invSKmSs;
+  const double rhoK = K_is_L ? rhoL : rhoR;
+  const double uK[3] = {K_is_L ? uL[0] : uR[0], K_is_L ? uL[1] : uR[1], K_is_L ? uL[2] : uR[2]};
+  const double pK = K_is_L ? pL : pR, eK = K_is_L ? eL : eR, unK = K_is_L ? unL : unR;
+  const double uKuK = K_is_L ? uLuL : uRuR, sK = K_is_L ? sL : sR;
+  const double invSKmSs = 1.0 / (sK - sM);
+  const double sKmuK = sK - unK;
+  const double rhoSK = rhoK * sKmuK * invSKmSs;
   double rhouSK[3];
 #pragma unroll
   for (int i = 0; i < 3; i++) rhouSK[i] = (rhoK * uK[i] * sKmuK + (pStar - pK) * nVec[i]) * invSKmSs;
-  double eSK = (sKmuK * eK - pK * unK + pStar * sM) * invSKmSs;
-  double invrhotld = 1.0 / (rhoR * (sR - unR) - rhoL * (sL - unL));
-  // derivative of sM and p* with respect to the requested side
+  const double eSK = (sKmuK * eK - pK * unK + pStar * sM) * invSKmSs;
+  const double invrhotld = 1.0 / (rhoR * (sR - unR) - rhoL * (sL - unL));
+  // derivative of sM and p* with respect to the requested side (R: negated)
   double dSM[5], dps[5];
-  if (which == 0) {
-    double gammaLM1 = (gammaL - 1.0);
-    dSM[0] = -unL * unL + uLuL * gammaLM1 / 2.0 + sM * sL;
-    dSM[1] = nVec[0] * (2.0 * unL - sL - sM) - gammaLM1 * uL[0];
-    dSM[2] = nVec[1] * (2.0 * unL - sL - sM) - gammaLM1 * uL[1];
-    dSM[3] = nVec[2] * (2.0 * unL - sL - sM) - gammaLM1 * uL[2];
-    dSM[4] = gammaLM1;
+  {
+    const double gm1 = (gam - 1.0), inv = W0 ? invrhotld : -invrhotld;
+    const double pre = W0 ? rhoR * (sR - unR) : rhoL * (sL - unL);
+    dSM[0] = -unW * unW + uuW * gm1 / 2.0 + sM * sW;
+#pragma unroll
+    for (int i = 0; i < 3; i++) dSM[1 + i] = nVec[i] * (2.0 * unW - sW - sM) - gm1 * uW[i];
+    dSM[4] = gm1;
 #pragma unroll
     for (int i = 0; i < 5; i++) {
-      dSM[i] *= invrhotld;
-      dps[i] = rhoR * (sR - unR) * dSM[i];
-    }
-  } else {
-    double gammaRM1 = (gammaR - 1.0);
-    dSM[0] = unR * unR - uRuR * gammaRM1 / 2.0 - sM * sR;
-    dSM[1] = -nVec[0] * (2.0 * unR - sR - sM) + gammaRM1 * uR[0];
-    dSM[2] = -nVec[1] * (2.0 * unR - sR - sM) + gammaRM1 * uR[1];
-    dSM[3] = -nVec[2] * (2.0 * unR - sR - sM) + gammaRM1 * uR[2];
-    dSM[4] = -gammaRM1;
-#pragma unroll
-    for (int i = 0; i < 5; i++) {
-      dSM[i] *= invrhotld;
-      dps[i] = rhoL * (sL - unL) * dSM[i];
+      dSM[i] *= inv;
+      dps[i] = pre * dSM[i];
     }
   }
   // calcSubSonicJacobeanHLLC (UgpWithCvCompFlow.cpp:605-659) called with the
   // star side K first: the requested matrix is its "AL" when it is side K
-  // (own-state terms), its "AR" otherwise.
+  // (own-state terms, x below), its "AR" otherwise; then back in
+  // calcEulerFluxMatrices_HLLC (:361-383 / :492-514 and :415-437 / :523-545)
   const double gamma = gAvg, gammaMinus1 = (gAvg - 1.0);
   const double *nV = nVec;
-  double omL = 1.0 / (sK - sM);
-  const bool own = (which == 0) == K_is_L;
-  if (own) {
-    const double qL = unK, psiL = uKuK, SL = sK, SM = sM, pS = pStar;
-    const double *dSMdUL = dSM, *dpsdUL = dps;
-    J[0][0] = SL + rhoSK * dSMdUL[0];
-    J[0][1] = -nV[0] + rhoSK * dSMdUL[1];
-    J[0][2] = -nV[1] + rhoSK * dSMdUL[2];
-    J[0][3] = -nV[2] + rhoSK * dSMdUL[3];
-    J[0][4] = +rhoSK * dSMdUL[4];
-    J[1][0] = qL * uK[0] - nV[0] * psiL * gammaMinus1 / 2.0 + nV[0] * dpsdUL[0] + rhouSK[0] * dSMdUL[0];
-    J[1][1] = SL - qL + nV[0] * (gamma - 2.0) * uK[0] + nV[0] * dpsdUL[1] + rhouSK[0] * dSMdUL[1];
-    J[1][2] = -uK[0] * nV[1] + nV[0] * gammaMinus1 * uK[1] + nV[0] * dpsdUL[2] + rhouSK[0] * dSMdUL[2];
-    J[1][3] = -uK[0] * nV[2] + nV[0] * gammaMinus1 * uK[2] + nV[0] * dpsdUL[3] + rhouSK[0] * dSMdUL[3];
-    J[1][4] = -gammaMinus1 * nV[0] + nV[0] * dpsdUL[4] + rhouSK[0] * dSMdUL[4];
-    J[2][0] = qL * uK[1] - nV[1] * psiL * gammaMinus1 / 2.0 + nV[1] * dpsdUL[0] + rhouSK[1] * dSMdUL[0];
-    J[2][1] = -uK[1] * nV[0] + nV[1] * gammaMinus1 * uK[0] + nV[1] * dpsdUL[1] + rhouSK[1] * dSMdUL[1];
-    J[2][2] = SL - qL + nV[1] * (gamma - 2.0) * uK[1] + nV[1] * dpsdUL[2] + rhouSK[1] * dSMdUL[2];
-    J[2][3] = -uK[1] * nV[2] + nV[1] * gammaMinus1 * uK[2] + nV[1] * dpsdUL[3] + rhouSK[1] * dSMdUL[3];
-    J[2][4] = -gammaMinus1 * nV[1] + nV[1] * dpsdUL[4] + rhouSK[1] * dSMdUL[4];
-    J[3][0] = qL * uK[2] - nV[2] * psiL * gammaMinus1 / 2.0 + nV[2] * dpsdUL[0] + rhouSK[2] * dSMdUL[0];
-    J[3][1] = -uK[2] * nV[0] + nV[2] * gammaMinus1 * uK[0] + nV[2] * dpsdUL[1] + rhouSK[2] * dSMdUL[1];
-    J[3][2] = -uK[2] * nV[1] + nV[2] * gammaMinus1 * uK[1] + nV[2] * dpsdUL[2] + rhouSK[2] * dSMdUL[2];
-    J[3][3] = SL - qL + nV[2] * (gamma - 2.0) * uK[2] + nV[2] * dpsdUL[3] + rhouSK[2] * dSMdUL[3];
-    J[3][4] = -gammaMinus1 * nV[2] + nV[2] * dpsdUL[4] + rhouSK[2] * dSMdUL[4];
-    J[4][0] = qL * (eK + pK) / rhoK - qL * psiL * (gamma - 1.0) / 2.0 + SM * dpsdUL[0] + (pS + eSK) * dSMdUL[0];
-    J[4][1] = -nV[0] * (eK + pK) / rhoK + gammaMinus1 * uK[0] * qL + SM * dpsdUL[1] + (pS + eSK) * dSMdUL[1];
-    J[4][2] = -nV[1] * (eK + pK) / rhoK + gammaMinus1 * uK[1] * qL + SM * dpsdUL[2] + (pS + eSK) * dSMdUL[2];
-    J[4][3] = -nV[2] * (eK + pK) / rhoK + gammaMinus1 * uK[2] * qL + SM * dpsdUL[3] + (pS + eSK) * dSMdUL[3];
-    J[4][4] = SL - qL * gamma + SM * dpsdUL[4] + (pS + eSK) * dSMdUL[4];
+  const double omL = 1.0 / (sK - sM);
+  const bool own = W0 == K_is_L;
+  const double q = unK, psi = uKuK, none = -0.0;
+  {
+    const double x[4] = {sK, -nV[0], -nV[1], -nV[2]};
 #pragma unroll
-    for (int i = 0; i < 5; i++)
-#pragma unroll
-      for (int j = 0; j < 5; j++) J[i][j] *= omL;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 5; i++) J[0][i] = omL * rhoSK * dSM[i];
-#pragma unroll
-    for (int i = 0; i < 5; i++) J[1][i] = omL * (nV[0] * dps[i] + rhouSK[0] * dSM[i]);
-#pragma unroll
-    for (int i = 0; i < 5; i++) J[2][i] = omL * (nV[1] * dps[i] + rhouSK[1] * dSM[i]);
-#pragma unroll
-    for (int i = 0; i < 5; i++) J[3][i] = omL * (nV[2] * dps[i] + rhouSK[2] * dSM[i]);
-#pragma unroll
-    for (int i = 0; i < 5; i++) J[4][i] = omL * (dps[i] * sM + (pStar + eSK) * dSM[i]);
+    for (int i = 0; i < 5; i++) {
+      const double star = rhoSK * dSM[i];
+      const double j = own ? (i < 4 ? x[i < 4 ? i : 0] + star : star) * omL : omL * rhoSK * dSM[i];
+      out(i, (j * sM + dSM[i] * rhoSK) * area);
+    }
   }
-  // back in calcEulerFluxMatrices_HLLC (:361-383 / :492-514 and :415-437 / :523-545)
 #pragma unroll
-  for (int i = 0; i < 5; i++) J[0][i] = J[0][i] * sM + dSM[i] * rhoSK;
+  for (int r = 0; r < 3; r++) {
 #pragma unroll
-  for (int i = 0; i < 5; i++) J[1][i] = J[1][i] * sM + dSM[i] * rhouSK[0] + dps[i] * nVec[0];
+    for (int i = 0; i < 5; i++) {
+      double x;
+      if (i == 0)
+        x = q * uK[r] - nV[r] * psi * gammaMinus1 / 2.0;
+      else if (i == r + 1)
+        x = sK - q + nV[r] * (gamma - 2.0) * uK[r];
+      else if (i < 4)
+        x = -uK[r] * nV[i < 4 ? i - 1 : 0] + nV[r] * gammaMinus1 * uK[i < 4 ? i - 1 : 0];
+      else
+        x = -gammaMinus1 * nV[r];
+      const double j = omL * ((own ? x : none) + nV[r] * dps[i] + rhouSK[r] * dSM[i]);
+      out(5 * (r + 1) + i, (j * sM + dSM[i] * rhouSK[r] + dps[i] * nVec[r]) * area);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
-  for (int i = 0; i < 5; i++) J[2][i] = J[2][i] * sM + dSM[i] * rhouSK[1] + dps[i] * nVec[1];
-#pragma unroll
-  for (int i = 0; i < 5; i++) J[3][i] = J[3][i] * sM + dSM[i] * rhouSK[2] + dps[i] * nVec[2];
-#pragma unroll
-  for (int i = 0; i < 5; i++) J[4][i] = (J[4][i] + dps[i]) * sM + (eSK + pStar) * dSM[i];
-#pragma unroll
-  for (int i = 0; i < 5; i++)
-#pragma unroll
-    for (int j = 0; j < 5; j++) J[i][j] *= area;
+  for (int i = 0; i < 5; i++) {
+    double x;
+    if (i == 0)
+      x = q * (eK + pK) / rhoK - q * psi * (gamma - 1.0) / 2.0;
+    else if (i < 4)
+      x = -nV[i < 4 ? i - 1 : 0] * (eK + pK) / rhoK + gammaMinus1 * uK[i < 4 ? i - 1 : 0] * q;
+    else
+      x = sK - q * gamma;
+    const double j = omL * ((own ? x : none) + sM * dps[i] + (pStar + eSK) * dSM[i]);
+    out(20 + i, ((j + dps[i]) * sM + (eSK + pStar) * dSM[i]) * area);
+  }
+}
+
+__device__ __forceinline__ void jac_hllc(double J[5][5], int which, double rhoL, const double *uL, double pL, double rhoR,
+                                      const double *uR, double pR, double gam, double area, const double *nVec,
+                                      double kL = 0.0, double kR = 0.0) {
+  jac_hllc_rows([&](int k, double v) { J[k / 5][k % 5] = v; }, which, rhoL, uL, pL, rhoR, uR, pR, gam, area, nVec, kL,
+                kR);
 }
 
 // Scalar row of one side of the HLLC Jacobian pair (A_L_Scal / A_R_Scal,
@@ -719,9 +707,12 @@ __device__ __forceinline__ void jac_coupled_super(double A[5][5], const double *
 // kine = 0. In every subsonic case the side's own dSM/dU is used with the
 // other side's rho (S - u_n), the star state is the upwind side's, and the
 // supersonic part and diagonal term belong to the upwind side only.
-__device__ __forceinline__ void jac_hllc_coupled(double J[5][5], int which, double rhoL, const double *uL, double pL,
-                                              double h0, double rhoR, const double *uR, double pR, double h1,
-                                              double gam, double area, const double *nVec) {
+// out(5 i + j, J[i][j]) is called once per entry, row by row, so that no more
+// than a row is live.
+template <class Out>
+__device__ __forceinline__ void jac_hllc_coupled_rows(Out out, int which, double rhoL, const double *uL, double pL,
+                                                      double h0, double rhoR, const double *uR, double pR, double h1,
+                                                      double gam, double area, const double *nVec) {
   const double gammaL = gam, gammaR = gam;
   double unL = dot3(uL, nVec);
   double uLuL = dot3(uL, uL);
@@ -756,15 +747,6 @@ __device__ __forceinline__ void jac_hllc_coupled(double J[5][5], int which, doub
   // this side's state (values selected, not a pointer: see flux_hllc_coupled)
   const double u[3] = {which == 0 ? uL[0] : uR[0], which == 0 ? uL[1] : uR[1], which == 0 ? uL[2] : uR[2]};
   const double p = which == 0 ? pL : pR, rho = which == 0 ? rhoL : rhoR, h = which == 0 ? hL : hR;
-  if (own) {
-    jac_coupled_super(J, u, p, rho, h, nVecArea, gam);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 5; i++)
-#pragma unroll
-      for (int j = 0; j < 5; j++) J[i][j] = 0.0;
-  }
-  if (sup) return;
   // the upwind side's star state
   const double uu[3] = {left ? uL[0] : uR[0], left ? uL[1] : uR[1], left ? uL[2] : uR[2]};
   const double Su = left ? sL : sR, unu = left ? unL : unR, rhou_ = left ? rhoL : rhoR, pu = left ? pL : pR;
@@ -793,17 +775,29 @@ __device__ __forceinline__ void jac_hllc_coupled(double J[5][5], int which, doub
   const double rhoSmq = which == 0 ? rhoR * (sR - unR) : rhoL * (sL - unL);
   double OmSM = Omega * sM;
   double OmSMp1 = OmSM + 1.0;
+  double B[5][5];  // the supersonic part, the upwind side's only
+  jac_coupled_super(B, u, p, rho, h, nVecArea, gam);
+  const double dg = area * Omega * sM * S;
 #pragma unroll
-  for (int i = 0; i < 5; i++) {
-    J[0][i] = -OmSM * J[0][i] + area * OmSMp1 * d[i] * rhoS;
-    J[1][i] = -OmSM * J[1][i] + area * OmSMp1 * d[i] * (rhouS[0] + rhoSmq * nVec[0]);
-    J[2][i] = -OmSM * J[2][i] + area * OmSMp1 * d[i] * (rhouS[1] + rhoSmq * nVec[1]);
-    J[3][i] = -OmSM * J[3][i] + area * OmSMp1 * d[i] * (rhouS[2] + rhoSmq * nVec[2]);
-    J[4][i] = -OmSM * J[4][i] + area * OmSMp1 * d[i] * (rhoeS + pStar + rhoSmq * sM);
+  for (int r = 0; r < 5; r++) {
+    const double x = r == 0 ? rhoS : (r < 4 ? rhouS[r < 4 && r > 0 ? r - 1 : 0] + rhoSmq * nVec[r < 4 && r > 0 ? r - 1 : 0]
+                                            : rhoeS + pStar + rhoSmq * sM);
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      const double b = own ? B[r][i] : 0.0;
+      double v = r == 0 ? -OmSM * b + area * OmSMp1 * d[i] * rhoS : -OmSM * b + area * OmSMp1 * d[i] * x;
+      if (r == i) v = own ? v + dg : v;
+      out(5 * r + i, sup ? b : v);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  if (own)
-#pragma unroll
-    for (int i = 0; i < 5; i++) J[i][i] += area * Omega * sM * S;
+}
+
+__device__ __forceinline__ void jac_hllc_coupled(double J[5][5], int which, double rhoL, const double *uL, double pL,
+                                              double h0, double rhoR, const double *uR, double pR, double h1,
+                                              double gam, double area, const double *nVec) {
+  jac_hllc_coupled_rows([&](int k, double v) { J[k / 5][k % 5] = v; }, which, rhoL, uL, pL, h0, rhoR, uR, pR, h1, gam,
+                        area, nVec);
 }
 
 // The transported scalar's row of the coupled HLLC Jacobian of one face side

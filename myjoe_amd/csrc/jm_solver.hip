@@ -53,6 +53,7 @@ struct DMesh {
   const int *cfl_i;       // [ncv+1]
   const int2 *cfl;        // [entries]
   const int *cfl_noc;     // [entries] off-diagonal block; bit 30 = accumulate
+  const int *cfl_tnoc;    // [entries] the block of this cell's column in the neighbour's row (-1: boundary face)
   const int *nbocv_i;     // [ncv+1]
   const int *nbocv_v;     // [nnz]
   const double *lsg;      // [nnz][3]
@@ -1399,6 +1400,20 @@ __device__ __forceinline__ void face_jac(int scheme, double J[5][5], int which, 
     jac_hllc(J, which, L.rho, L.u, L.p, R.rho, R.u, R.p, gam, area, n, kL, kR);
 }
 
+// the same, entry by entry
+template <class Out>
+__device__ __forceinline__ void face_jac_rows(int scheme, Out out, int which, const Side &L, const Side &R, double gam,
+                                              double area, const double *n, double kL, double kR) {
+  if (scheme == kRoe) {
+    double J[5][5];
+    jac_roe(J, which, L.rho, L.u, L.p, R.rho, R.u, R.p, gam, area, n);
+#pragma unroll
+    for (int k = 0; k < 25; k++) out(k, J[k / 5][k % 5]);
+  } else {
+    jac_hllc_rows(out, which, L.rho, L.u, L.p, R.rho, R.u, R.p, gam, area, n, kL, kR);
+  }
+}
+
 template <typename T, int SCHEME, bool VISC, int NB = 5>
 __device__ __forceinline__ void d_jac(const Blk &B, DMesh m, DParams P, const double *__restrict__ prim,
                                                 const double *__restrict__ bfa, T *__restrict__ A, int step_mode,
@@ -1673,18 +1688,32 @@ __global__ void __launch_bounds__(kBlock) k_jac(DMesh m, DParams P, const double
 
 // ---------------------------------------------------------------------------
 // The same Jacobian assembly with one lane per cell-face entry (the flux
-// kernel's wave table: whole cells per wavefront). Each lane evaluates its
-// face's two blocks once: the off-diagonal one goes straight to A, the
-// diagonal contribution (signed: D -= J is D + (-J) exactly) to the lane's LDS
-// slot. The lanes of a cell then sum the diagonal block component-wise in the
-// cell's entry order (lane pos owns components pos, pos + nent, ...), which is
-// the reference's accumulation order, so the blocks are the same bits as
-// k_jac's. The segregated viscous blocks are a second pass over the same
-// slots (the reference adds them after every Euler block); the coupled loop
-// adds each face's viscous block right after its Euler block, so there the
-// slot also keeps the viscous block's eleven possibly nonzero entries.
-// Duplicate neighbour pairs (two faces between one pair of cells) need their
+// kernel's wave table: whole cells per wavefront). Each lane evaluates one
+// matrix, J = dF/dU of its own cell: signed, it is what the face adds to the
+// cell's diagonal block (D -= J is D + (-J) exactly), and with the opposite
+// sign it is the off-diagonal block of the cell's column in the neighbour's
+// row (icv0's entry gives A[noc00] += Apl and A[noc10] = -Apl, icv1's
+// A[noc11] -= Ami and A[noc01] = +Ami), so the two entries of a face share
+// its two matrices and none is evaluated twice. The diagonal contribution
+// goes to the lane's LDS slot; the lanes of a cell sum the diagonal block
+// component-wise in the cell's entry order (lane pos owns components pos,
+// pos + nent, ...), which is the reference's accumulation order, so the
+// blocks are the same bits as k_jac's. The off-diagonal blocks are written
+// from the slots by the wavefront together, consecutive lanes on consecutive
+// values: a lane writing its own block touches 64 cache lines per store.
+// The segregated viscous blocks are a second pass over the same slots (the
+// reference adds them after every Euler block); the coupled loop adds each
+// face's viscous block right after its Euler block, so there the slot also
+// keeps the viscous block's eleven possibly nonzero entries. Duplicate
+// neighbour pairs (two faces between one pair of cells) need their
 // off-diagonal block accumulated in entry order and use k_jac.
+// What bounds it is the latency of its dependent loads and FP64 chains at the
+// few waves its registers allow, so one matrix per lane, formed row by row
+// straight into LDS (jac_hllc_rows), is worth more than the arithmetic it
+// saves: 146-160 registers and three waves per SIMD where two matrices held
+// whole took 256 and one. 386k-cell split box, FP64: 392 -> 208 us; 687k-cell
+// SST plate: 1531 -> 696 us; the 6x6 form (200 registers, 18.8 KB of LDS per
+// wavefront, two waves) 454 -> 386 us at 250k cells.
 // ---------------------------------------------------------------------------
 // the entries of a coupled viscous block (visc_coupled_jac) that may be
 // nonzero: [1+i][0], [1+i][1+i] for i < 3 and row 4; -1 for the others
@@ -1721,6 +1750,7 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
   constexpr int NS = CV ? 25 + kVcN : 25;
   __shared__ double lds[64 * W * NS];
   __shared__ signed char vsg[64 * W];  // the entry's viscous block: 0 none, +1 added, -1 subtracted
+  __shared__ int toff[64 * W];         // the entry's off-diagonal block, -1 without one
   double *slot = lds + NS * threadIdx.x;
   const EntryLane L = entry_lane<W>(m, B);
   const double gam = P.gamma;
@@ -1736,36 +1766,80 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
     const double *geo = m.fgeo + 8 * (size_t)f;
     const double n[3] = {geo[0], geo[1], geo[2]};
     const double area = geo[3];
-    signed char vs = 0;
-    if (en.y >= 0) {
-      const double *pn = prim + 8 * (size_t)en.y;
+    const bool internal = en.y >= 0;
+    // the face's two sides: this cell and its neighbour as (icv0, icv1), or
+    // the boundary state on one side or both; then one evaluation of this
+    // cell's matrix (Apl, which 0, for icv0 and on boundary faces; Ami, which
+    // 1, for icv1), so a wavefront that mixes them runs the code once
+    const bool s0 = !internal || en.x >= 0;
+    const double *pn = prim + 8 * (size_t)(internal ? en.y : c);
+    const double *bb = bfa + 8 * (size_t)(internal ? 0 : f);
+    const ZoneDev *z = m.zones + (internal ? 0 : -en.y - 1);
+    bool pressure_only = false, both = false;  // SYMM_BC = ANALYTICAL; NEW_NUMERIC: Apl + Ami
+    Side l, r;
+    double kl = 0.0, kr = 0.0, hl = 0.0, hr = 0.0;
+    if (internal) {
       Side nb;
       nb.rho = pn[0]; nb.u[0] = pn[1]; nb.u[1] = pn[2]; nb.u[2] = pn[3]; nb.p = pn[4];
-      const bool s0 = en.x >= 0;
-      const Side l = s0 ? own : nb, r = s0 ? nb : own;
-      const double kcl = SST ? P.sst_phi[s0 ? c : en.y] : 0.0, kcr = SST ? P.sst_phi[s0 ? en.y : c] : 0.0;
-      double hl = 0.0, hr = 0.0;
+      l = s0 ? own : nb;
+      r = s0 ? nb : own;
+      if (SST) {
+        kl = P.sst_phi[s0 ? c : en.y];
+        kr = P.sst_phi[s0 ? en.y : c];
+      }
       if (CPL) {
         hl = enthalpy_of(P, l.rho, l.p);
         hr = enthalpy_of(P, r.rho, r.p);
       }
-      // t = 0: the diagonal's block (icv0 adds Apl, which 0; icv1 subtracts
-      // Ami, which 1); t = 1: the off-diagonal block (icv0's A[noc01] = +Ami,
-      // icv1's A[noc10] = -Apl). One loop, so one copy of the Jacobian code.
-      T *off = A + NB * NB * (size_t)(m.cfl_noc[L.e] & 0x3fffffff);
-#pragma unroll 1
-      for (int t = 0; t < 2; t++) {
-        const int which = (t == 0) == s0 ? 0 : 1;
-        if (CPL) jac_hllc_coupled(J, which, l.rho, l.u, l.p, hl, r.rho, r.u, r.p, hr, gam, area, n);
-        else face_jac(SCHEME, J, which, l, r, gam, area, n, kcl, kcr);
-        if (t == 0) {
-          for (int i = 0; i < 5; i++)
-            for (int j = 0; j < 5; j++) slot[5 * i + j] = s0 ? J[i][j] : -J[i][j];
-        } else {
-          store_block<T, NB>(off, J, !s0, false);
-        }
+    } else {
+      r.rho = bb[0]; r.u[0] = bb[1]; r.u[1] = bb[2]; r.u[2] = bb[3]; r.p = bb[4];
+      if (CPL) hr = bb[6];
+      if (SST) kr = P.sst_bfa[2 * (size_t)f];
+      l = r;
+      hl = hr;
+      kl = kr;
+      if (z->bc == kBcSymmetry || z->bc == kBcWall || (CPL && z->bc == kBcNeumann)) {
+        // walls take the first side's matrix in the segregated loop
+        // (JoeWithModels.cpp:3196-3277) and follow SYMM_BC in the coupled one
+        // (:5150-5470; NEUMANN faces only its NEW_NUMERIC)
+        const bool symm = CPL || z->bc == kBcSymmetry;
+        pressure_only = symm && P.symm_bc == kSymmAnalytical && z->bc != kBcNeumann;
+        both = symm && P.symm_bc == kSymmNew;
+      } else {  // cell-centre state against the boundary state
+        l = own;
+        if (SST) kl = P.sst_phi[c];
+        if (CPL) hl = enthalpy_of(P, own.rho, own.p);
       }
-      if (CV) {  // the same face's viscous blocks next (JoeWithModels.cpp:5096-5104)
+    }
+    if (!pressure_only) {
+      auto put = [&](int k, double v) { slot[k] = s0 ? v : -v; };
+      if (CPL) jac_hllc_coupled_rows(put, s0 ? 0 : 1, l.rho, l.u, l.p, hl, r.rho, r.u, r.p, hr, gam, area, n);
+      else face_jac_rows(SCHEME, put, s0 ? 0 : 1, l, r, gam, area, n, kl, kr);
+      if (both) {
+        auto add = [&](int k, double v) { slot[k] = slot[k] + v; };
+        if (CPL) jac_hllc_coupled_rows(add, 1, l.rho, l.u, l.p, hl, r.rho, r.u, r.p, hr, gam, area, n);
+        else face_jac_rows(SCHEME, add, 1, l, r, gam, area, n, kl, kr);
+      }
+    } else if (CPL) {  // calcFluxCoupled's ONLY_PRESSURE matrix
+      jac_only_pressure(J, r.rho, r.u, r.p, hr, gam, area, n);
+#pragma unroll
+      for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5];
+    } else {  // ANALYTICAL, JoeWithModels.cpp:3243-3269
+      const double a2 = gam - 1.0;
+      const double phi2 = 0.5 * a2 * (r.u[0] * r.u[0] + r.u[1] * r.u[1] + r.u[2] * r.u[2]);
+      for (int j = 0; j < 5; j++) {
+        slot[j] = 0.0;
+        slot[20 + j] = 0.0;
+      }
+      for (int i = 0; i < 3; i++) {
+        slot[5 * (i + 1)] = phi2 * n[i] * area;
+        for (int j = 0; j < 3; j++) slot[5 * (i + 1) + j + 1] = -a2 * r.u[j] * n[i] * area;
+        slot[5 * (i + 1) + 4] = a2 * n[i] * area;
+      }
+    }
+    signed char vs = 0;
+    if (CV) {  // the same face's viscous block next (JoeWithModels.cpp:5096-5104)
+      if (internal) {
         const VSide vo = vside_cell(P, pc, gradv + 12 * (size_t)c);
         const VSide vn = vside_cell(P, pn, gradv + 12 * (size_t)en.y);
         const VSide a = vsel(s0, vo, vn), b = vsel(s0, vn, vo);
@@ -1783,102 +1857,37 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         const double ufa[3] = {0.5 * (a.u[0] + b.u[0]), 0.5 * (a.u[1] + b.u[1]), 0.5 * (a.u[2] + b.u[2])};
         double VF[5], tau[3], keff;
         visc_coupled(P, a, b, mul, mut, ufa, area, n, smag, sV, alpha, VF, tau, keff, P.sa != 0);
-#pragma unroll 1
-        for (int t = 0; t < 2; t++) {
-          // t = 0: the diagonal's block from this cell's side; t = 1: the other side's, off the diagonal
-          visc_coupled_jac(P, J, (t == 0) == s0 ? 0 : 1, vsel((t == 0) == s0, a, b), mul + mut, keff, tau, ufa, area,
-                           alpha, smag);
-          if (t == 0) {
-            for (int k = 0; k < 25; k++) {
-              const int vi = vc_index(k);
-              if (vi >= 0) slot[25 + vi] = s0 ? J[k / 5][k % 5] : -J[k / 5][k % 5];
-            }
-          } else {
-            for (int i = 0; i < 5; i++)
-              for (int j = 0; j < 5; j++)
-                off[NB * i + j] =
-                    (T)(s0 ? (double)off[NB * i + j] + J[i][j] : (double)off[NB * i + j] - J[i][j]);
-          }
+        visc_coupled_jac(P, J, s0 ? 0 : 1, vsel(s0, a, b), mul + mut, keff, tau, ufa, area, alpha, smag);
+        for (int k = 0; k < 25; k++) {
+          const int vi = vc_index(k);
+          if (vi >= 0) slot[25 + vi] = s0 ? J[k / 5][k % 5] : -J[k / 5][k % 5];
         }
         vs = s0 ? 1 : -1;
-      }
-    } else {
-      const ZoneDev &z = m.zones[-en.y - 1];
-      const double *bb = bfa + 8 * (size_t)f;
-      Side sb;
-      sb.rho = bb[0]; sb.u[0] = bb[1]; sb.u[1] = bb[2]; sb.u[2] = bb[3]; sb.p = bb[4];
-      if (CPL) {  // calcFluxCoupled boundary Jacobians (JoeWithModels.cpp:5150-5740)
-        const double hb = bb[6];
-        if (z.bc == kBcSymmetry || z.bc == kBcWall || z.bc == kBcNeumann) {
-          if (z.bc != kBcNeumann && P.symm_bc == kSymmAnalytical) {
-            jac_only_pressure(J, sb.rho, sb.u, sb.p, hb, gam, area, n);
-            for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5];
-          } else if (P.symm_bc == kSymmNew) {
-            double K[5][5];
-            jac_hllc_coupled(J, 0, sb.rho, sb.u, sb.p, hb, sb.rho, sb.u, sb.p, hb, gam, area, n);
-            jac_hllc_coupled(K, 1, sb.rho, sb.u, sb.p, hb, sb.rho, sb.u, sb.p, hb, gam, area, n);
-            for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5] + K[k / 5][k % 5];
-          } else {
-            jac_hllc_coupled(J, 0, sb.rho, sb.u, sb.p, hb, sb.rho, sb.u, sb.p, hb, gam, area, n);
-            for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5];
-          }
-        } else {  // cell-centre state against the boundary state
-          jac_hllc_coupled(J, 0, own.rho, own.u, own.p, enthalpy_of(P, own.rho, own.p), sb.rho, sb.u, sb.p, hb, gam,
-                           area, n);
-          for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5];
+      } else if (z->bc != kBcSymmetry) {  // none on symmetry faces
+        const double *gvo = gradv + 12 * (size_t)c;
+        const VSide vo = vside_cell(P, pc, gvo);
+        const VSide vb = vside_bfa(bb, gvo);
+        const double xfa[3] = {geo[4], geo[5], geo[6]};
+        double sArg[3], smag, alpha;
+        visc_coupled_bgeom(z->bc, xfa, pc + 5, n, sArg, smag, alpha);
+        const double mul = mu_lam(P, bb[5]);
+        const double mut = (P.sa && z->bc != kBcWall)
+                               ? sa_mut(pc[0] * P.sa_phi[c], P.sa_aux[kAuxN * (size_t)c + kAuxMue])
+                               : 0.0;
+        const VSide lv = vsel(z->bc == kBcNeumann, vb, vo);
+        double VF[5], tau[3], keff;
+        visc_coupled(P, lv, vb, mul, mut, vb.u, area, n, smag, sArg, alpha, VF, tau, keff, P.sa != 0);
+        visc_coupled_jac(P, J, 0, lv, mul + mut, keff, tau, vb.u, area, alpha, smag);
+        for (int k = 0; k < 25; k++) {
+          const int vi = vc_index(k);
+          if (vi >= 0) slot[25 + vi] = J[k / 5][k % 5];
         }
-        if (CV && z.bc != kBcSymmetry) {  // the face's viscous block (none on symmetry faces)
-          const double *gvo = gradv + 12 * (size_t)c;
-          const VSide vo = vside_cell(P, pc, gvo);
-          const VSide vb = vside_bfa(bb, gvo);
-          const double xfa[3] = {geo[4], geo[5], geo[6]};
-          double sArg[3], smag, alpha;
-          visc_coupled_bgeom(z.bc, xfa, pc + 5, n, sArg, smag, alpha);
-          const double mul = mu_lam(P, bb[5]);
-          const double mut = (P.sa && z.bc != kBcWall)
-                                 ? sa_mut(pc[0] * P.sa_phi[c], P.sa_aux[kAuxN * (size_t)c + kAuxMue])
-                                 : 0.0;
-          const VSide lv = vsel(z.bc == kBcNeumann, vb, vo);
-          double VF[5], tau[3], keff;
-          visc_coupled(P, lv, vb, mul, mut, vb.u, area, n, smag, sArg, alpha, VF, tau, keff, P.sa != 0);
-          visc_coupled_jac(P, J, 0, lv, mul + mut, keff, tau, vb.u, area, alpha, smag);
-          for (int k = 0; k < 25; k++) {
-            const int vi = vc_index(k);
-            if (vi >= 0) slot[25 + vi] = J[k / 5][k % 5];
-          }
-          vs = 1;
-        }
-      } else if (z.bc == kBcSymmetry || z.bc == kBcWall) {
-        const double kb = SST ? P.sst_bfa[2 * (size_t)f] : 0.0;
-        if (z.bc == kBcWall || P.symm_bc == kSymmOriginal) {
-          face_jac(SCHEME, J, 0, sb, sb, gam, area, n, kb, kb);
-          for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5];
-        } else if (P.symm_bc == kSymmNew) {
-          double K[5][5];
-          face_jac(SCHEME, J, 0, sb, sb, gam, area, n, kb, kb);
-          face_jac(SCHEME, K, 1, sb, sb, gam, area, n, kb, kb);
-          for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5] + K[k / 5][k % 5];
-        } else {  // ANALYTICAL, JoeWithModels.cpp:3243-3269
-          const double a2 = gam - 1.0;
-          const double phi2 = 0.5 * a2 * (sb.u[0] * sb.u[0] + sb.u[1] * sb.u[1] + sb.u[2] * sb.u[2]);
-          for (int j = 0; j < 5; j++) {
-            slot[j] = 0.0;
-            slot[20 + j] = 0.0;
-          }
-          for (int i = 0; i < 3; i++) {
-            slot[5 * (i + 1)] = phi2 * n[i] * area;
-            for (int j = 0; j < 3; j++) slot[5 * (i + 1) + j + 1] = -a2 * sb.u[j] * n[i] * area;
-            slot[5 * (i + 1) + 4] = a2 * n[i] * area;
-          }
-        }
-      } else {
-        if (SST) face_jac(SCHEME, J, 0, own, sb, gam, area, n, P.sst_phi[c], P.sst_bfa[2 * (size_t)f]);
-        else face_jac(SCHEME, J, 0, own, sb, gam, area, n);
-        for (int k = 0; k < 25; k++) slot[k] = J[k / 5][k % 5];
+        vs = 1;
       }
     }
     vsg[threadIdx.x] = vs;
   }
+  toff[threadIdx.x] = L.e >= 0 ? m.cfl_tnoc[L.e] : -1;
   __syncthreads();
   // the cell's diagonal block, summed in entry order by the cell's lanes
   double Dk[kMaxOwned];
@@ -1933,17 +1942,16 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         }
         const double ufa[3] = {0.5 * (a.u[0] + b.u[0]), 0.5 * (a.u[1] + b.u[1]), 0.5 * (a.u[2] + b.u[2])};
         visc_face<SST>(P, a, b, mul, mut, ufa, area, n, smag, sV, Fu, FE, vf, kine_fa);
-        T *off = A + NB * NB * (size_t)(m.cfl_noc[L.e] & 0x3fffffff);
-        // icv0: A[noc00] -= A0, A[noc01] -= A1; icv1: A[noc11] += A1, A[noc10] += A0
-        if (s0) visc_jac<SST>(P, J, 1.0, b, mul, mut, vf, ufa, area, smag);  // A1 -> off
-        else visc_jac<SST>(P, J, -1.0, a, mul, mut, vf, ufa, area, smag);    // A0 -> off
+        // icv0: A[noc00] -= A0, A[noc10] += A0; icv1: A[noc11] += A1, A[noc01] -= A1
+        visc_jac<SST>(P, J, s0 ? -1.0 : 1.0, vsel(s0, a, b), mul, mut, vf, ufa, area, smag);
+#pragma unroll
         for (int i = 1; i < 5; i++)
-          for (int j = 0; j < 5; j++)
-            off[NB * i + j] = (T)(s0 ? (double)off[NB * i + j] - J[i][j] : (double)off[NB * i + j] + J[i][j]);
-        if (s0) visc_jac<SST>(P, J, -1.0, a, mul, mut, vf, ufa, area, smag);  // A0 -> diagonal, subtracted
-        else visc_jac<SST>(P, J, 1.0, b, mul, mut, vf, ufa, area, smag);     // A1 -> diagonal, added
-        for (int i = 1; i < 5; i++)
-          for (int j = 0; j < 5; j++) slot[5 * i + j] = s0 ? -J[i][j] : J[i][j];
+#pragma unroll
+          for (int j = 0; j < 5; j++) {
+            const double inv = slot[5 * i + j], v = s0 ? -J[i][j] : J[i][j];
+            slot[5 * i + j] = v;
+            J[i][j] = (double)(T)((double)(T)(0.0 - inv) - v);  // the off-diagonal value
+          }
         vs = 1;
       } else {
         const ZoneDev &z = m.zones[-en.y - 1];
@@ -1988,6 +1996,43 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         for (int j = 0; j < nent; j++)
           if (vsg[first + j]) d += lds[NS * (first + j) + k];
         Dk[q] = d;
+      }
+    }
+  }
+  // the off-diagonal blocks: the slots' values negated, less the viscous ones
+  if (VISC) {
+    __syncthreads();
+    if (L.e >= 0 && toff[threadIdx.x] >= 0) {
+#pragma unroll
+      for (int k = 0; k < 25; k++) {
+        if (CPL) {
+          const int vi = vc_index(k);
+          if (vi >= 0) slot[k] = -(double)(T)((double)(T)(0.0 - slot[k]) - slot[25 + vi]);
+        } else if (k >= 5) {
+          slot[k] = -J[k / 5][k % 5];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  {
+    constexpr int NR = 5 * NB;  // the flow rows of a block; with the scalar their sixth column is zero
+    const int lane = threadIdx.x & 63, wb = threadIdx.x - lane;
+    int en = lane / NR, k = lane % NR;
+    for (int it = 0; it < NR; it++) {
+      const int tn = toff[wb + en];
+      if (tn >= 0) {
+        const double *sj = lds + NS * (wb + en);
+        T v;
+        if (NB == 6) v = k % 6 == 5 ? (T)0.0 : (T)(0.0 - sj[k - k / 6]);
+        else v = (T)(0.0 - sj[k]);
+        A[NB * NB * (size_t)tn + k] = v;
+      }
+      k += 64 % NR;
+      en += 64 / NR;
+      if (k >= NR) {
+        k -= NR;
+        en++;
       }
     }
   }
@@ -5222,6 +5267,23 @@ __global__ void __launch_bounds__(kBlock) k_wall_dist(int ncv, const double *__r
 }
 
 
+// for every cell-face entry the block of its cell's column in the
+// neighbour's row (set-up; the rows are symmetric in their pattern)
+__global__ void __launch_bounds__(kBlock) k_tnoc(int ncv, const int *__restrict__ cfl_i, const int2 *__restrict__ cfl,
+                                                 const int *__restrict__ nbocv_i, const int *__restrict__ nbocv_v,
+                                                 int *__restrict__ tnoc) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= ncv) return;
+  for (int e = cfl_i[c]; e < cfl_i[c + 1]; e++) {
+    const int nb = cfl[e].y;
+    int t = -1;
+    if (nb >= 0)
+      for (int k = nbocv_i[nb] + 1; k < nbocv_i[nb + 1]; k++)
+        if (nbocv_v[k] == c) t = k;
+    tnoc[e] = t;
+  }
+}
+
 template <typename T>
 struct DBuf {
   T *p = nullptr;
@@ -5610,7 +5672,7 @@ struct Ctx::Impl {
   bool have_state = false;
   // mesh buffers
   DBuf<double> fgeo, fnorm, lsg, bfa_lsg, vol;
-  DBuf<int> cfl_i, cfl_noc, nbocv_i, nbocv_v, bfa_cell, bfa_zone;
+  DBuf<int> cfl_i, cfl_noc, cfl_tnoc, nbocv_i, nbocv_v, bfa_cell, bfa_zone;
   DBuf<int2> cfl_e;
   DBuf<int2> ecp;
   DBuf<int> wave_e0;
@@ -6047,6 +6109,7 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
     d.ecp.upload(ecp.data(), ecp.size());
     d.wave_e0.upload(we.data(), we.size());
     d.cfl_noc.upload(noc.data(), noc.size());
+    d.cfl_tnoc.alloc(std::max<size_t>(1, dcf.size()));
   }
   std::vector<int> bcell(std::max(1, nfa_b), 0);
   for (int f = 0; f < nfa_b; f++) bcell[f] = inv[m.cvofa[2 * (size_t)f]];
@@ -6184,6 +6247,10 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
   d.dm.cfl_i = d.cfl_i.p;
   d.dm.cfl = d.cfl_e.p;
   d.dm.cfl_noc = d.cfl_noc.p;
+  hipLaunchKernelGGL(k_tnoc, dim3(nblk(ncv)), dim3(kBlock), 0, d.stream, ncv, d.cfl_i.p, d.cfl_e.p, d.nbocv_i.p,
+                     d.nbocv_v.p, d.cfl_tnoc.p);
+  HIPCHECK(hipGetLastError());
+  d.dm.cfl_tnoc = d.cfl_tnoc.p;
   d.dm.nbocv_i = d.nbocv_i.p;
   d.dm.nbocv_v = d.nbocv_v.p;
   d.dm.lsg = d.lsg.p;
@@ -6262,7 +6329,7 @@ size_t Ctx::footprint(const Mesh &m, int precision) {
   b += nfa * (8 + 3) * 8;                          // fgeo, fnorm
   b += nnz * (3 * 8 + 4) + nfa_b * (3 * 8 + 4 + 4);  // lsg, nbocv_v, bfa_lsg, bfa_cell, bfa_zone
   b += (ncv + 1) * 4 * 2 + ncv * 4;                // cfl_i, nbocv_i, wave table
-  b += ent * (8 + 4 + 8 + 24);                     // entries, their blocks, their cells and positions, limiter offsets
+  b += ent * (8 + 8 + 8 + 24);                     // entries, their two blocks, their cells and positions, limiter offsets
   b += ncv * (5 + 8 + 16 + 5 + 1 + 1) * 8;         // q, prim, grad, rhs, dt, vol
   b += nfa_b * (8 + 5) * 8;                        // bfa, hook
   b += (nnz + ncv) * 25 * sJ + 10 * ncv * 5 * sJ;  // A, LU, Krylov vectors
