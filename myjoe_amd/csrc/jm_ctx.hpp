@@ -103,15 +103,17 @@ void parse_params(const std::string &joe_in, const Mesh &m, SolverParams &p, std
 // precision, and its solver scalars.
 struct KrylovJob {
   int ncv = 0, maxiter = 0;
+  // the iterations' residual by its recurrence; FP64: the stop test confirmed
+  // on the true residual
+  bool rec = false, confirm = false;
   const int *nbocv_i = nullptr, *nbocv_v = nullptr;
   const void *A = nullptr;
   void *LU = nullptr;
   void *v[10] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   void *S = nullptr;
   // first block and block count of this solve in each launch shape of the
-  // batch (5 lanes per cell, a thread per cell, a thread per unknown);
-  // filled by setup_krylov_batch
-  int b5 = 0, nb5 = 0, b1 = 0, nb1 = 0, bx = 0, nbx = 0;
+  // batch (5 lanes per cell, a thread per cell); filled by setup_krylov_batch
+  int b5 = 0, nb5 = 0, b1 = 0, nb1 = 0;
 };
 
 // device buffers of the batched BiCGStab, grown on demand
@@ -121,7 +123,9 @@ struct KrylovBatchBuf {
   double *partials_d = nullptr;
   int *flag_h = nullptr, *flag_d = nullptr;
   size_t cap_jobs = 0, cap_map = 0, cap_partials = 0;
-  int njobs = 0, g5 = 0, g1 = 0, gx = 0, max_it = 0;  // the batch set up last
+  // the batch set up last
+  int njobs = 0, g5 = 0, g1 = 0, max_it = 0;
+  bool any_true = false, any_confirm = false;  // whether a solve takes the true residual, a confirmation
   int last_launched = 0;  // iterations the last run launched before every solve stopped
   KrylovBatchBuf() = default;
   KrylovBatchBuf(const KrylovBatchBuf &) = delete;

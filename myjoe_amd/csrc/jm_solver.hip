@@ -113,7 +113,10 @@ struct SolverScalars {
   double resid_l2[5];  // L2 norms of the same residual
   double resid_s;  // L1 of the transported scalar's residual (Spalart-Allmaras; SST's kine)
   double resid_s2;  // SST: omega's
-  int iter, done, maxiter, pad;
+  // done: 0 running, 1 converged, 2 iteration limit, 3 the recurrence's
+  // residual has met the stop test and the true residual is to confirm it
+  // (confirm: FP64 block solves)
+  int iter, done, maxiter, confirm;
   double zero_abs, zero_rel;
   // pseudo-time step counter and CFL of the device-driven (graph) step
   int step_no, stop;  // stop: the host-polled loop's launch budget is spent
@@ -3521,7 +3524,8 @@ enum FinOp {
   kFinDt = 0, kFinL1 = 1, kFinAlpha = 2, kFinOmega = 3, kFinResid0 = 4, kFinResid = 5,
   kFinResid0J = 6,  // kFinResid0 of the Jacobi (scalar) solver, which stops at once if already converged
   kFinL1S = 7,      // L1 of the scalar residual
-  kFinL1S2 = 8      // L1 of the second scalar's residual (SST omega)
+  kFinL1S2 = 8,     // L1 of the second scalar's residual (SST omega)
+  kFinConfirm = 9   // kFinResid on the true residual, for solves that wait for it (done 3)
 };
 
 // one block: finishes a reduction and applies the scalar update of its owner
@@ -3530,6 +3534,7 @@ constexpr int kFinBlock = 1024;
 __device__ void fin_body(int nb, int op, const double *__restrict__ partials, size_t stride, SolverScalars *S,
                          double *sh) {
   if ((op == kFinAlpha || op == kFinOmega || op == kFinResid) && (S->done || S->stop)) return;
+  if (op == kFinConfirm && S->done != 3) return;
   const bool t0 = threadIdx.x == 0;
   if (op == kFinDt) {
     double m = fin_slot(partials, nb, kMin, sh);
@@ -3574,13 +3579,13 @@ __device__ void fin_body(int nb, int op, const double *__restrict__ partials, si
       } else {
         S->res_max = mxv;
         if ((mxv <= S->zero_abs) || (mxv / (S->res0_max + 1.0E-12) <= S->zero_rel))
-          S->done = 1;
-        else if (S->iter > S->maxiter)
-          S->done = 2;
+          S->done = op == kFinResid && S->confirm ? 3 : 1;
+        else
+          S->done = S->iter > S->maxiter ? 2 : 0;
       }
       // the host-polled loop launches at most max_launch iterations; a
       // device-driven step stops at the same point (iter counts them)
-      if (op == kFinResid && !S->done && S->iter + 1 >= S->max_launch) S->stop = 1;
+      if ((op == kFinResid || op == kFinConfirm) && !S->done && S->iter + 1 >= S->max_launch) S->stop = 1;
       if (!S->done) {
         S->iter += 1;
         double rho_prime = -S->omega * S->rho;
@@ -4205,12 +4210,14 @@ __global__ void k_set_step(SolverScalars *S, int step, double cfl) {
 }
 
 // BiCGStab scalars at the start of a solve (leaves dt_min, residuals, step)
-__device__ __forceinline__ void d_solver_init(const Blk &B, SolverScalars *S, int maxiter, double zero_abs, double zero_rel) {
+__device__ __forceinline__ void d_solver_init(const Blk &B, SolverScalars *S, int maxiter, double zero_abs, double zero_rel,
+                                              int confirm) {
   if (threadIdx.x != 0) return;
   S->rho = S->rho_prime = S->alpha = S->omega = S->beta = S->gamma = 0.0;
   S->res0_max = S->res_max = 0.0;
   S->iter = 0;
   S->done = 0;
+  S->confirm = confirm;
   S->stop = 0;
   S->max_launch = maxiter + 1;
   S->maxiter = maxiter;
@@ -4218,8 +4225,8 @@ __device__ __forceinline__ void d_solver_init(const Blk &B, SolverScalars *S, in
   S->zero_rel = zero_rel;
 }
 
-__global__ void k_solver_init(SolverScalars *S, int maxiter, double zero_abs, double zero_rel) {
-  d_solver_init(hw_blk(), S, maxiter, zero_abs, zero_rel);
+__global__ void k_solver_init(SolverScalars *S, int maxiter, double zero_abs, double zero_rel, int confirm) {
+  d_solver_init(hw_blk(), S, maxiter, zero_abs, zero_rel, confirm);
 }
 
 template <typename T>
@@ -4256,10 +4263,13 @@ __global__ void k_publish(const SolverScalars *S, StepMail *out) {
 // matrix-vector products keep the reference's per-row order (blocks in
 // nbocv order, columns ascending) using NB lanes per cell.
 // ---------------------------------------------------------------------------
+// start of a solve, one thread per cell: the LU of the cell's diagonal block
+// and p = v = 0
 template <typename T, int NB>
-__global__ void __launch_bounds__(kBlock) k_lu(int ncv, const int *__restrict__ nbocv_i, const T *__restrict__ A,
-                                               T *__restrict__ LU) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void d_start(const Blk &B, int ncv, const int *__restrict__ nbocv_i,
+                                        const T *__restrict__ A, T *__restrict__ LU, T *__restrict__ p,
+                                        T *__restrict__ v) {
+  const int c = B.id * blockDim.x + threadIdx.x;
   if (c >= ncv) return;
   T a[NB][NB];
   const T *s = A + NB * NB * (size_t)nbocv_i[c];
@@ -4269,6 +4279,16 @@ __global__ void __launch_bounds__(kBlock) k_lu(int ncv, const int *__restrict__ 
   T *d = LU + NB * NB * (size_t)c;
   for (int i = 0; i < NB; i++)
     for (int j = 0; j < NB; j++) d[NB * i + j] = a[i][j];
+  for (int k = 0; k < NB; k++) {
+    p[NB * (size_t)c + k] = (T)0;
+    v[NB * (size_t)c + k] = (T)0;
+  }
+}
+
+template <typename T, int NB>
+__global__ void __launch_bounds__(kBlock) k_start(int ncv, const int *__restrict__ nbocv_i, const T *__restrict__ A,
+                                                  T *__restrict__ LU, T *__restrict__ p, T *__restrict__ v) {
+  d_start<T, NB>(hw_blk(), ncv, nbocv_i, A, LU, p, v);
 }
 
 // y = A x for row component (c, i) = (tid / NB, tid % NB)
@@ -4291,24 +4311,32 @@ constexpr int cells_per_block() {
 }
 constexpr int kCellsPerBlock = cells_per_block<5>();
 
-// res = rhs - A phi; init: res0 = res. Partials: res.res0 (slot 0) and
-// max |LU^-1 res| (slot 1), finished by k_fin kFinResid0 / kFinResid.
+// res = rhs - A phi. Partials: res.res0 (slot 0) and max |LU^-1 res| (slot 1),
+// finished by k_fin.
+enum ResidMode {
+  kResidIter = 0,     // each iteration's residual (kFinResid)
+  kResidFirst = 1,    // the first: also res0 = res (kFinResid0)
+  kResidZero = 2,     // the first of a zero guess: res0 = res = rhs, no product with A
+  kResidConfirm = 3   // the true residual of a solve whose recurrence has met the stop test (kFinConfirm)
+};
 template <typename T, int NB>
-__global__ void __launch_bounds__(kBlock) k_resid(int ncv, const int *__restrict__ nbocv_i,
-                                                  const int *__restrict__ nbocv_v, const T *__restrict__ A,
-                                                  const T *__restrict__ LU, const T *__restrict__ phi,
-                                                  const T *__restrict__ rhs, T *__restrict__ res, T *__restrict__ res0,
-                                                  int init, double *partials, const SolverScalars *S) {
+__device__ __forceinline__ void d_resid(const Blk &B, int ncv, const int *__restrict__ nbocv_i,
+                                        const int *__restrict__ nbocv_v, const T *__restrict__ A,
+                                        const T *__restrict__ LU, const T *__restrict__ phi,
+                                        const T *__restrict__ rhs, T *__restrict__ res, T *__restrict__ res0,
+                                        int mode, double *partials, size_t stride, const SolverScalars *S) {
   constexpr int CPB = cells_per_block<NB>();
   __shared__ double sh[32];
   __shared__ T cellv[CPB][NB];
-  if (!init && (S->done || S->stop)) return;
+  const bool init = mode == kResidFirst || mode == kResidZero;
+  if (mode == kResidConfirm ? S->done != 3 : (!init && (S->done || S->stop))) return;
   const int lc = threadIdx.x / NB, i = threadIdx.x % NB;
-  const int c = blockIdx.x * CPB + lc;
+  const int c = B.id * CPB + lc;
   const bool active = (lc < CPB) && (c < ncv);
   T r = (T)0.0;
   if (active) {
-    T ax = spmv_row<T, NB>(nbocv_i, nbocv_v, A, phi, c, i);
+    T ax = (T)0.0;
+    if (mode != kResidZero) ax = spmv_row<T, NB>(nbocv_i, nbocv_v, A, phi, c, i);
     r = rhs[NB * (size_t)c + i] - ax;
     res[NB * (size_t)c + i] = r;
     if (init) res0[NB * (size_t)c + i] = r;
@@ -4328,49 +4356,64 @@ __global__ void __launch_bounds__(kBlock) k_resid(int ncv, const int *__restrict
   __syncthreads();
   block_reduce<1>(vm, sh + 16, kMax);
   if (threadIdx.x == 0) {
-    partials[blockIdx.x] = vs[0];
-    partials[gridDim.x + blockIdx.x] = vm[0];
+    partials[B.id] = vs[0];
+    partials[stride + B.id] = vm[0];
   }
 }
 
-// res = s - omega t: the residual by the BiCGStab recurrence instead of
-// rhs - A phi (no product with A), for the FP32 solve when asked
-// (GPU_KRYLOV_RESIDUAL = RECURRENCE); partials as k_resid's
 template <typename T, int NB>
-__global__ void __launch_bounds__(kBlock) k_resid_rec(int ncv, const T *__restrict__ LU, const T *__restrict__ s,
-                                                      const T *__restrict__ t, T *__restrict__ res,
-                                                      const T *__restrict__ res0, double *partials,
-                                                      const SolverScalars *S) {
-  constexpr int CPB = cells_per_block<NB>();
-  __shared__ double sh[32];
-  __shared__ T cellv[CPB][NB];
-  if (S->done || S->stop) return;
-  const int lc = threadIdx.x / NB, i = threadIdx.x % NB;
-  const int c = blockIdx.x * CPB + lc;
-  const bool active = (lc < CPB) && (c < ncv);
-  T r = (T)0.0;
-  if (active) {
-    const size_t o = NB * (size_t)c + i;
-    r = s[o] - (T)S->omega * t[o];
-    res[o] = r;
-    cellv[lc][i] = r;
-  }
-  __syncthreads();
+__global__ void __launch_bounds__(kBlock) k_resid(int ncv, const int *__restrict__ nbocv_i,
+                                                  const int *__restrict__ nbocv_v, const T *__restrict__ A,
+                                                  const T *__restrict__ LU, const T *__restrict__ phi,
+                                                  const T *__restrict__ rhs, T *__restrict__ res, T *__restrict__ res0,
+                                                  int mode, double *partials, const SolverScalars *S) {
+  d_resid<T, NB>(hw_blk(), ncv, nbocv_i, nbocv_v, A, LU, phi, rhs, res, res0, mode, partials, gridDim.x, S);
+}
+
+// phi += alpha phat + omega shat, and the residual by the BiCGStab's own
+// recurrence, res = s - omega t (FP32: GPU_KRYLOV_RESIDUAL = RECURRENCE;
+// FP64: kRecMinBytes), where the reference recomputes rhs - A phi
+// (UgpWithCv.cpp:2812-2846): one product with A fewer per iteration. One
+// thread per cell; partials as k_resid's, per block of kBlock cells.
+template <typename T, int NB>
+__device__ __forceinline__ void d_x_rec(const Blk &B, int ncv, const T *__restrict__ LU, T *__restrict__ phi,
+                                        const T *__restrict__ phat, const T *__restrict__ shat,
+                                        const T *__restrict__ s, const T *__restrict__ t, T *__restrict__ res,
+                                        const T *__restrict__ res0, T alpha, T omega, double *partials,
+                                        size_t stride, double *sh) {
+  const int c = B.id * blockDim.x + threadIdx.x;
   double vs[1] = {0.0}, vm[1] = {0.0};
-  if (active) {
-    vs[0] = (double)r * (double)res0[NB * (size_t)c + i];
-    T tmp[NB];
-    for (int k = 0; k < NB; k++) tmp[k] = cellv[lc][k];
-    lusolv_n<T, NB>(LU + NB * NB * (size_t)c, tmp);
-    vm[0] = fabs((double)tmp[i]);
+  if (c < ncv) {
+    T r[NB];
+    for (int k = 0; k < NB; k++) {
+      const size_t o = NB * (size_t)c + k;
+      phi[o] += alpha * phat[o] + omega * shat[o];
+      r[k] = s[o] - omega * t[o];
+      res[o] = r[k];
+      vs[0] += (double)r[k] * (double)res0[o];
+    }
+    lusolv_n<T, NB>(LU + NB * NB * (size_t)c, r);
+    for (int k = 0; k < NB; k++) vm[0] = Dev::mx(vm[0], fabs((double)r[k]));
   }
   block_reduce<1>(vs, sh, kSum);
   __syncthreads();
   block_reduce<1>(vm, sh + 16, kMax);
   if (threadIdx.x == 0) {
-    partials[blockIdx.x] = vs[0];
-    partials[gridDim.x + blockIdx.x] = vm[0];
+    partials[B.id] = vs[0];
+    partials[stride + B.id] = vm[0];
   }
+}
+
+template <typename T, int NB>
+__global__ void __launch_bounds__(kBlock) k_x_rec(int ncv, const T *__restrict__ LU, T *__restrict__ phi,
+                                                  const T *__restrict__ phat, const T *__restrict__ shat,
+                                                  const T *__restrict__ s, const T *__restrict__ t,
+                                                  T *__restrict__ res, const T *__restrict__ res0, double *partials,
+                                                  const SolverScalars *S) {
+  __shared__ double sh[32];
+  if (S->done || S->stop) return;
+  d_x_rec<T, NB>(hw_blk(), ncv, LU, phi, phat, shat, s, t, res, res0, (T)S->alpha, (T)S->omega, partials, gridDim.x,
+                 sh);
 }
 
 // p = res - beta (p - omega v); phat = LU^-1 p   (one thread per cell). With
@@ -4614,36 +4657,58 @@ struct BcgSys {
   int ilu_sub = 0;
   void *F = nullptr, *Dinv = nullptr;
   // the residual of each iteration by the recurrence s - omega t instead of
-  // rhs - A phi (FP32 solves only)
-  bool rec_resid = false;
+  // rhs - A phi (FP32 solves unless asked otherwise; FP64 solves of
+  // kRecMinBytes and more); with confirm (FP64) the stop test it meets is
+  // taken again on the true residual, so a solve ends on the reference's own
+  // criterion
+  bool rec_resid = false, confirm = false;
+  bool zero_guess = false;  // phi is zero when the solve starts
 };
+
+// FP64 solves take the recurrence's residual once A is larger than this. It
+// saves a product with A per iteration, at 80-87 % of the card's read rate
+// already, for two launches per chunk of iterations and one product per
+// solve. Implicit step of the split box, true residual against recurrence:
+// 223k cells 1598 -> 1469 us, 115k 901 -> 828, 28k 462 -> 432, 5.9k 377 -> 358.
+// Below 16 MB (14k cells of five-by-five blocks) the product costs no more
+// than its launch and the 20-40 us left are the fused update's; there the
+// solve keeps the reference's form and its bits, which small cases are
+// compared on over hundreds of steps.
+constexpr size_t kRecMinBytes = size_t(16) << 20;
+inline bool krylov_rec64(long long nnz, int nb) { return (size_t)nnz * nb * nb * sizeof(double) >= kRecMinBytes; }
 
 // start of a solve (UgpWithCv.cpp:2660-2735): p = v = 0, block LU of the
 // diagonal, the first residual and its stop test
 template <typename T, int NB>
 void bcg_prologue(const BcgSys &y) {
-  const int ncv = y.ncv, n = NB * ncv;
+  const int ncv = y.ncv;
   const T *A = (const T *)y.A;
   T *LU = (T *)y.LU;
   T *rhs_ = (T *)y.v[0], *phi = (T *)y.v[1], *res = (T *)y.v[2], *res0 = (T *)y.v[3], *p = (T *)y.v[4],
     *vv = (T *)y.v[5];
-  hipLaunchKernelGGL(k_fill<T>, dim3(nblk(n)), dim3(kBlock), 0, y.stream, (size_t)n, p, (T)0);
-  hipLaunchKernelGGL(k_fill<T>, dim3(nblk(n)), dim3(kBlock), 0, y.stream, (size_t)n, vv, (T)0);
-  hipLaunchKernelGGL(k_solver_init, dim3(1), dim3(64), 0, y.stream, y.S, y.maxiter, y.zero_abs, y.zero_rel);
-  hipLaunchKernelGGL((k_lu<T, NB>), dim3(nblk(ncv)), dim3(kBlock), 0, y.stream, ncv, y.nbocv_i, A, LU);
+  const dim3 g(nblk(ncv)), bl(kBlock);
+  hipLaunchKernelGGL(k_solver_init, dim3(1), dim3(64), 0, y.stream, y.S, y.maxiter, y.zero_abs, y.zero_rel,
+                     y.confirm ? 1 : 0);
+  hipLaunchKernelGGL((k_start<T, NB>), g, bl, 0, y.stream, ncv, y.nbocv_i, A, LU, p, vv);
   if (y.ilu_sub > 0) {
     const int nsub = (ncv + y.ilu_sub - 1) / y.ilu_sub;
     hipLaunchKernelGGL((k_ilu_factor<T, NB>), dim3((nsub + 63) / 64), dim3(64), 0, y.stream, ncv, y.ilu_sub,
                        y.nbocv_i, y.nbocv_v, A, (T *)y.F, (T *)y.Dinv);
   }
   const int gb = (ncv + cells_per_block<NB>() - 1) / cells_per_block<NB>();
-  hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), dim3(kBlock), 0, y.stream, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi,
-                     rhs_, res, res0, 1, y.partials, y.S);
+  hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), bl, 0, y.stream, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi, rhs_, res,
+                     res0, y.zero_guess ? (int)kResidZero : (int)kResidFirst, y.partials, y.S);
   hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, y.stream, gb, (int)kFinResid0, y.partials, y.S);
 }
 
 // count BiCGStab iterations (van der Vorst, UgpWithCv.cpp:2725-2856); each
-// returns at once once the device has set the convergence or stop flag
+// returns at once once the device has set the convergence or stop flag. With
+// y.rec_resid the residual comes from its recurrence; an FP64 solve that
+// meets the stop test with it waits (done 3, the remaining iterations are
+// no-ops) for the confirmation at the end of the chunk: the true residual
+// either passes the same test, or replaces the recurrence's and the solve
+// goes on. So a solve of k iterations takes 2 k + 1 products with A where
+// the reference's form takes 3 k, and stops on the same test.
 template <typename T, int NB>
 void bcg_iterations(const BcgSys &y, int count) {
   const int ncv = y.ncv, n = NB * ncv;
@@ -4677,14 +4742,21 @@ void bcg_iterations(const BcgSys &y, int count) {
     hipLaunchKernelGGL((k_spmv_dot<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, shat, t, s,
                        y.partials, y.S);
     hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, gb, (int)kFinOmega, y.partials, y.S);
-    hipLaunchKernelGGL(k_x<T>, dim3(nblk(n)), dim3(kBlock), 0, st, n, phi, phat, shat, y.S);
-    if (y.rec_resid)
-      hipLaunchKernelGGL((k_resid_rec<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, LU, s, t, res, res0, y.partials,
-                         y.S);
-    else
+    if (y.rec_resid) {
+      hipLaunchKernelGGL((k_x_rec<T, NB>), dim3(nblk(ncv)), dim3(kBlock), 0, st, ncv, LU, phi, phat, shat, s, t, res,
+                         res0, y.partials, y.S);
+    } else {
+      hipLaunchKernelGGL(k_x<T>, dim3(nblk(n)), dim3(kBlock), 0, st, n, phi, phat, shat, y.S);
       hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi,
-                         rhs_, res, res0, 0, y.partials, y.S);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, gb, (int)kFinResid, y.partials, y.S);
+                         rhs_, res, res0, (int)kResidIter, y.partials, y.S);
+    }
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, y.rec_resid ? nblk(ncv) : gb, (int)kFinResid,
+                       y.partials, y.S);
+  }
+  if (y.confirm) {
+    hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi, rhs_,
+                       res, res0, (int)kResidConfirm, y.partials, y.S);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, gb, (int)kFinConfirm, y.partials, y.S);
   }
 }
 
@@ -4719,68 +4791,22 @@ void bcg_solve(const BcgSys &y, SolverScalars *hs, int &iters, int &status) {
 // same bits as the per-solve solver's.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void __launch_bounds__(kBlock) kb_lu(const KrylovJob *__restrict__ jobs, const int *__restrict__ map1) {
+__global__ void __launch_bounds__(kBlock) kb_start(const KrylovJob *__restrict__ jobs, const int *__restrict__ map1) {
   const KrylovJob &J = jobs[map1[blockIdx.x]];
-  const int c = (blockIdx.x - J.b1) * blockDim.x + threadIdx.x;
-  if (c >= J.ncv) return;
-  T a[5][5];
-  const T *src = (const T *)J.A + 25 * (size_t)J.nbocv_i[c];
-  for (int i = 0; i < 5; i++)
-    for (int j = 0; j < 5; j++) a[i][j] = src[5 * i + j];
-  ludeco5<T>(a);
-  T *d = (T *)J.LU + 25 * (size_t)c;
-  for (int i = 0; i < 5; i++)
-    for (int j = 0; j < 5; j++) d[5 * i + j] = a[i][j];
-  for (int k = 0; k < 5; k++) {  // p = v = 0
-    ((T *)J.v[4])[5 * (size_t)c + k] = (T)0;
-    ((T *)J.v[5])[5 * (size_t)c + k] = (T)0;
-  }
+  d_start<T, 5>(Blk{(int)blockIdx.x - J.b1, J.nb1}, J.ncv, J.nbocv_i, (const T *)J.A, (T *)J.LU, (T *)J.v[4],
+                (T *)J.v[5]);
 }
 
-// REC: the residual by the recurrence s - omega t, as k_resid_rec (the FP32
-// solves; omega is stored by kb_x)
-template <typename T, bool REC = false>
+// k_resid; an iteration's residual only of the solves that do not take it
+// from the recurrence
+template <typename T>
 __global__ void __launch_bounds__(kBlock) kb_resid(const KrylovJob *__restrict__ jobs, const int *__restrict__ map5,
-                                                   int init, double *partials) {
-  __shared__ double sh[32];
-  __shared__ T cellv[kCellsPerBlock][5];
+                                                   int mode, double *partials) {
   const KrylovJob &J = jobs[map5[blockIdx.x]];
-  const SolverScalars *S = (const SolverScalars *)J.S;
-  if (!init && (S->done || S->stop)) return;
-  const T *A = (const T *)J.A, *LU = (const T *)J.LU, *phi = (const T *)J.v[1], *rhs = (const T *)J.v[0];
-  T *res = (T *)J.v[2], *res0 = (T *)J.v[3];
-  const int lc = threadIdx.x / 5, i = threadIdx.x % 5;
-  const int c = (blockIdx.x - J.b5) * kCellsPerBlock + lc;
-  const bool active = (lc < kCellsPerBlock) && (c < J.ncv);
-  T r = (T)0.0;
-  if (active && REC && !init) {
-    const size_t o = 5 * (size_t)c + i;
-    r = ((const T *)J.v[7])[o] - (T)S->omega * ((const T *)J.v[9])[o];
-    res[o] = r;
-    cellv[lc][i] = r;
-  } else if (active) {
-    T ax = spmv_row<T, 5>(J.nbocv_i, J.nbocv_v, A, phi, c, i);
-    r = rhs[5 * (size_t)c + i] - ax;
-    res[5 * (size_t)c + i] = r;
-    if (init) res0[5 * (size_t)c + i] = r;
-    cellv[lc][i] = r;
-  }
-  __syncthreads();
-  double vs[1] = {0.0}, vm[1] = {0.0};
-  if (active) {
-    T r0v = init ? r : res0[5 * (size_t)c + i];
-    vs[0] = (double)r * (double)r0v;
-    T tmp[5] = {cellv[lc][0], cellv[lc][1], cellv[lc][2], cellv[lc][3], cellv[lc][4]};
-    lusolv5<T>(LU + 25 * (size_t)c, tmp);
-    vm[0] = fabs((double)tmp[i]);
-  }
-  block_reduce<1>(vs, sh, kSum);
-  __syncthreads();
-  block_reduce<1>(vm, sh + 16, kMax);
-  if (threadIdx.x == 0) {
-    partials[blockIdx.x] = vs[0];
-    partials[gridDim.x + blockIdx.x] = vm[0];
-  }
+  if (mode == kResidIter && J.rec) return;
+  d_resid<T, 5>(Blk{(int)blockIdx.x - J.b5, J.nb5}, J.ncv, J.nbocv_i, J.nbocv_v, (const T *)J.A, (const T *)J.LU,
+                (const T *)J.v[1], (const T *)J.v[0], (T *)J.v[2], (T *)J.v[3], mode, partials + J.b5, gridDim.x,
+                (const SolverScalars *)J.S);
 }
 
 // which = 0: p = res - beta (p - omega v), phat = LU^-1 p; 1: s = res - alpha v, shat = LU^-1 s
@@ -4853,32 +4879,49 @@ __global__ void __launch_bounds__(kBlock) kb_spmv_dot(const KrylovJob *__restric
   block_partials<2>(v, partials, sh, kSum);
 }
 
-// phi += alpha phat + omega shat, with omega = (s.t) / (t.t + 1e-20) finished
-// from kb_spmv_dot's partials in every block as k_fin kFinOmega does (the
-// solve's first block stores it)
+// k_x_rec (or, for a solve with the true residual, k_x) with omega = (s.t) /
+// (t.t + 1e-20) finished from kb_spmv_dot's partials in every block as k_fin
+// kFinOmega does (the solve's first block stores it); its own partials go to
+// partials1
 template <typename T>
-__global__ void __launch_bounds__(kBlock) kb_x(const KrylovJob *__restrict__ jobs, const int *__restrict__ mapx,
-                                               const double *__restrict__ partials, int grid5) {
-  __shared__ double sh[16];
-  const KrylovJob &J = jobs[mapx[blockIdx.x]];
+__global__ void __launch_bounds__(kBlock) kb_x_rec(const KrylovJob *__restrict__ jobs, const int *__restrict__ map1,
+                                                   const double *__restrict__ partials, int grid5,
+                                                   double *__restrict__ partials1, int grid1) {
+  __shared__ double sh[32];
+  const KrylovJob &J = jobs[map1[blockIdx.x]];
   SolverScalars *S = (SolverScalars *)J.S;
   if (S->done || S->stop) return;
   const double st = fin_slot_v(partials + J.b5, J.nb5, kSum, sh);  // UgpWithCv.cpp:2808-2810
   const double tt = fin_slot_v(partials + J.b5 + grid5, J.nb5, kSum, sh);
   const double omega = st / (tt + 1.0E-20);
-  if ((int)blockIdx.x == J.bx && threadIdx.x == 0) S->omega = omega;
-  const int k = (blockIdx.x - J.bx) * blockDim.x + threadIdx.x;
-  if (k >= 5 * J.ncv) return;
-  T *phi = (T *)J.v[1];
-  phi[k] += (T)S->alpha * ((const T *)J.v[6])[k] + (T)omega * ((const T *)J.v[8])[k];
+  if ((int)blockIdx.x == J.b1 && threadIdx.x == 0) S->omega = omega;
+  __syncthreads();
+  if (!J.rec) {
+    const int c = (blockIdx.x - J.b1) * blockDim.x + threadIdx.x;
+    if (c >= J.ncv) return;
+    T *phi = (T *)J.v[1];
+    for (int i = 0; i < 5; i++) {
+      const size_t k = 5 * (size_t)c + i;
+      phi[k] += (T)S->alpha * ((const T *)J.v[6])[k] + (T)omega * ((const T *)J.v[8])[k];
+    }
+    return;
+  }
+  d_x_rec<T, 5>(Blk{(int)blockIdx.x - J.b1, J.nb1}, J.ncv, (const T *)J.LU, (T *)J.v[1], (const T *)J.v[6],
+                (const T *)J.v[8], (const T *)J.v[7], (const T *)J.v[9], (T *)J.v[2], (const T *)J.v[3], (T)S->alpha,
+                (T)omega, partials1 + J.b1, grid1, sh);
 }
 
-// one block per solve: finish its partials (at its first block, stride = the whole grid)
+// one block per solve: finish its partials, at its first block of the launch
+// shape that wrote them (the recurrence's residual: one thread per cell)
 __global__ void __launch_bounds__(kFinBlock) kb_fin(const KrylovJob *__restrict__ jobs, int op,
-                                                    const double *__restrict__ partials, int grid5) {
+                                                    const double *__restrict__ partials, int grid5,
+                                                    const double *__restrict__ partials1, int grid1) {
   __shared__ double sh[16];
   const KrylovJob &J = jobs[blockIdx.x];
-  fin_body(J.nb5, op, partials + J.b5, (size_t)grid5, (SolverScalars *)J.S, sh);
+  if (op == kFinResid && J.rec)
+    fin_body(J.nb1, op, partials1 + J.b1, (size_t)grid1, (SolverScalars *)J.S, sh);
+  else
+    fin_body(J.nb5, op, partials + J.b5, (size_t)grid5, (SolverScalars *)J.S, sh);
 }
 
 // *flag = 1 when every solve of the batch has converged or spent its launches
@@ -5005,7 +5048,7 @@ struct StepJob {
   DtArgs dta;
   size_t nA;
   double gamma, relax, cfl_factor, cfl_max, ls_abs, ls_rel;
-  int ncv, cfl_after, cfl_interval, ls_maxiter;
+  int ncv, cfl_after, cfl_interval, ls_maxiter, confirm;
   int b[kShapes], n[kShapes];  // first block and block count in each launch shape
 };
 
@@ -5021,7 +5064,7 @@ __global__ void ks_ramp(const StepJob *__restrict__ jobs) {
 
 __global__ void ks_solver_init(const StepJob *__restrict__ jobs) {
   const StepJob &J = jobs[blockIdx.x];
-  d_solver_init(Blk{0, 1}, J.scal, J.ls_maxiter, J.ls_abs, J.ls_rel);
+  d_solver_init(Blk{0, 1}, J.scal, J.ls_maxiter, J.ls_abs, J.ls_rel, J.confirm);
 }
 
 __global__ void ks_publish(const StepJob *__restrict__ jobs) {
@@ -6450,32 +6493,32 @@ KrylovBatchBuf::~KrylovBatchBuf() {
 // block -> solve maps, and the job table on the device.
 void setup_krylov_batch(KrylovJob *jobs_h, int njobs, void *stream, KrylovBatchBuf &buf) {
   hipStream_t st = (hipStream_t)stream;
-  int g5 = 0, g1 = 0, gx = 0, max_it = 0;
+  int g5 = 0, g1 = 0, max_it = 0;
   for (int j = 0; j < njobs; j++) {
     KrylovJob &J = jobs_h[j];
     J.b5 = g5;
     J.nb5 = (J.ncv + kCellsPerBlock - 1) / kCellsPerBlock;
     J.b1 = g1;
     J.nb1 = nblk(J.ncv);
-    J.bx = gx;
-    J.nbx = nblk(5 * (long long)J.ncv);
     g5 += J.nb5;
     g1 += J.nb1;
-    gx += J.nbx;
     max_it = std::max(max_it, J.maxiter + 1);
+  }
+  buf.any_true = buf.any_confirm = false;
+  for (int j = 0; j < njobs; j++) {
+    buf.any_true = buf.any_true || !jobs_h[j].rec;
+    buf.any_confirm = buf.any_confirm || jobs_h[j].confirm;
   }
   buf.njobs = njobs;
   buf.g5 = g5;
   buf.g1 = g1;
-  buf.gx = gx;
   buf.max_it = max_it;
   if (njobs <= 0) return;
-  std::vector<int> map((size_t)g5 + g1 + gx);
+  std::vector<int> map((size_t)g5 + g1);
   for (int j = 0; j < njobs; j++) {
     const KrylovJob &J = jobs_h[j];
     for (int b = 0; b < J.nb5; b++) map[J.b5 + b] = j;
     for (int b = 0; b < J.nb1; b++) map[(size_t)g5 + J.b1 + b] = j;
-    for (int b = 0; b < J.nbx; b++) map[(size_t)g5 + g1 + J.bx + b] = j;
   }
   if (buf.cap_jobs < (size_t)njobs) {
     if (buf.jobs_d) HIPCHECK(hipFree(buf.jobs_d));
@@ -6487,9 +6530,10 @@ void setup_krylov_batch(KrylovJob *jobs_h, int njobs, void *stream, KrylovBatchB
     buf.cap_map = std::max(map.size(), 2 * buf.cap_map);
     HIPCHECK(hipMalloc((void **)&buf.map_d, sizeof(int) * buf.cap_map));
   }
-  if (buf.cap_partials < 2 * (size_t)g5 + 8) {
+  const size_t npart = 2 * ((size_t)g5 + g1) + 8;  // two slots per block of either shape
+  if (buf.cap_partials < npart) {
     if (buf.partials_d) HIPCHECK(hipFree(buf.partials_d));
-    buf.cap_partials = std::max<size_t>(2 * (size_t)g5 + 8, 2 * buf.cap_partials);
+    buf.cap_partials = std::max<size_t>(npart, 2 * buf.cap_partials);
     HIPCHECK(hipMalloc((void **)&buf.partials_d, sizeof(double) * buf.cap_partials));
   }
   if (!buf.flag_h) {
@@ -6504,30 +6548,31 @@ void setup_krylov_batch(KrylovJob *jobs_h, int njobs, void *stream, KrylovBatchB
 template <typename T>
 static void krylov_batch_prologue(hipStream_t st, const KrylovBatchBuf &buf) {
   const int *m5 = buf.map_d, *m1 = buf.map_d + buf.g5;
-  hipLaunchKernelGGL(kb_lu<T>, dim3(buf.g1), dim3(kBlock), 0, st, buf.jobs_d, m1);
-  hipLaunchKernelGGL(kb_resid<T>, dim3(buf.g5), dim3(kBlock), 0, st, buf.jobs_d, m5, 1, buf.partials_d);
-  hipLaunchKernelGGL(kb_fin, dim3(buf.njobs), dim3(kFinBlock), 0, st, buf.jobs_d, (int)kFinResid0, buf.partials_d,
-                     buf.g5);
+  double *pt = buf.partials_d, *pt1 = pt + 2 * (size_t)buf.g5;
+  hipLaunchKernelGGL(kb_start<T>, dim3(buf.g1), dim3(kBlock), 0, st, buf.jobs_d, m1);
+  hipLaunchKernelGGL(kb_resid<T>, dim3(buf.g5), dim3(kBlock), 0, st, buf.jobs_d, m5, (int)kResidZero, pt);
+  hipLaunchKernelGGL(kb_fin, dim3(buf.njobs), dim3(kFinBlock), 0, st, buf.jobs_d, (int)kFinResid0, pt, buf.g5, pt1,
+                     buf.g1);
 }
 
 template <typename T>
 static void krylov_batch_iterations(hipStream_t st, const KrylovBatchBuf &buf, int count) {
-  const int *m5 = buf.map_d, *m1 = buf.map_d + buf.g5, *mx = buf.map_d + buf.g5 + buf.g1;
+  const int *m5 = buf.map_d, *m1 = buf.map_d + buf.g5;
   const KrylovJob *jd = buf.jobs_d;
-  double *pt = buf.partials_d;
-  const int g5 = buf.g5, g1 = buf.g1, gx = buf.gx, nj = buf.njobs;
-  for (int k = 0; k < count; k++) {  // seven launches: alpha and omega are finished in kb_ps and kb_x
+  double *pt = buf.partials_d, *pt1 = pt + 2 * (size_t)buf.g5;
+  const int g5 = buf.g5, g1 = buf.g1, nj = buf.njobs;
+  for (int k = 0; k < count; k++) {  // six launches: alpha and omega are finished in kb_ps and kb_x_rec
     hipLaunchKernelGGL(kb_ps<T>, dim3(g1), dim3(kBlock), 0, st, jd, m1, 0, pt, g5);
     hipLaunchKernelGGL(kb_spmv_dot<T>, dim3(g5), dim3(kBlock), 0, st, jd, m5, 0, pt);
     hipLaunchKernelGGL(kb_ps<T>, dim3(g1), dim3(kBlock), 0, st, jd, m1, 1, pt, g5);
     hipLaunchKernelGGL(kb_spmv_dot<T>, dim3(g5), dim3(kBlock), 0, st, jd, m5, 1, pt);
-    hipLaunchKernelGGL(kb_x<T>, dim3(gx), dim3(kBlock), 0, st, jd, mx, pt, g5);
-    // FP32 solves take the residual by the recurrence (GPU_KRYLOV_RESIDUAL = RECURRENCE, the server's rule)
-    if (std::is_same<T, float>::value)
-      hipLaunchKernelGGL((kb_resid<T, true>), dim3(g5), dim3(kBlock), 0, st, jd, m5, 0, pt);
-    else
-      hipLaunchKernelGGL(kb_resid<T>, dim3(g5), dim3(kBlock), 0, st, jd, m5, 0, pt);
-    hipLaunchKernelGGL(kb_fin, dim3(nj), dim3(kFinBlock), 0, st, jd, (int)kFinResid, pt, g5);
+    hipLaunchKernelGGL(kb_x_rec<T>, dim3(g1), dim3(kBlock), 0, st, jd, m1, pt, g5, pt1, g1);
+    if (buf.any_true) hipLaunchKernelGGL(kb_resid<T>, dim3(g5), dim3(kBlock), 0, st, jd, m5, (int)kResidIter, pt);
+    hipLaunchKernelGGL(kb_fin, dim3(nj), dim3(kFinBlock), 0, st, jd, (int)kFinResid, pt, g5, pt1, g1);
+  }
+  if (buf.any_confirm) {  // as bcg_iterations
+    hipLaunchKernelGGL(kb_resid<T>, dim3(g5), dim3(kBlock), 0, st, jd, m5, (int)kResidConfirm, pt);
+    hipLaunchKernelGGL(kb_fin, dim3(nj), dim3(kFinBlock), 0, st, jd, (int)kFinConfirm, pt, g5, pt1, g1);
   }
 }
 
@@ -6636,6 +6681,7 @@ void StepBatch::set(Ctx *const *ctxs, int n, void *stream) {
     J.cfl_after = d.par.cfl_after;
     J.cfl_interval = d.par.cfl_interval;
     J.ls_maxiter = d.par.ls_maxiter;
+    J.confirm = d.precision == 0 && krylov_rec64(d.nnz, 5);
     // the grids of the solve's own launches (launch_grad, launch_flux,
     // launch_jac, launch_state_bc)
     const bool grad = d.par.second_order || d.dp.visc;
@@ -6816,6 +6862,8 @@ void Ctx::batch_job(KrylovJob &job) {
   Impl &d = *d_;
   job.ncv = d.ncv;
   job.maxiter = d.par.ls_maxiter;
+  job.confirm = d.precision == 0 && krylov_rec64(d.nnz, 5);
+  job.rec = d.precision != 0 || job.confirm;  // FP32 solves: the server takes no other form
   job.nbocv_i = d.nbocv_i.p;
   job.nbocv_v = d.nbocv_v.p;
   job.S = d.scal.p;
@@ -7167,7 +7215,7 @@ void Ctx::Impl::scalar_step(const T *dq) {
                      AS.p, dq, b, x);
   hipLaunchKernelGGL(k_fill<double>, g, bl, 0, stream, (size_t)ncv, p, 0.0);
   hipLaunchKernelGGL(k_fill<double>, g, bl, 0, stream, (size_t)ncv, vv, 0.0);
-  hipLaunchKernelGGL(k_solver_init, dim3(1), dim3(64), 0, stream, scal_s.p, kSaMaxIter, kSaPhiZero, kSaPhiZeroRel);
+  hipLaunchKernelGGL(k_solver_init, dim3(1), dim3(64), 0, stream, scal_s.p, kSaMaxIter, kSaPhiZero, kSaPhiZeroRel, 0);
   const int nb = nblk(ncv);
   hipLaunchKernelGGL(k_sc_resid, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, AS.p, x, b, res, res0, 1, partials.p,
                      scal_s.p);
@@ -7218,7 +7266,7 @@ void Ctx::Impl::sst_scalar_step(const T *dq) {
     hipLaunchKernelGGL(k_fill<double>, g, bl, 0, stream, (size_t)ncv, p, 0.0);
     hipLaunchKernelGGL(k_fill<double>, g, bl, 0, stream, (size_t)ncv, vv, 0.0);
     hipLaunchKernelGGL(k_solver_init, dim3(1), dim3(64), 0, stream, scal_s.p, kSstMaxIter, kSstPhiZero,
-                       kSstPhiZeroRel);
+                       kSstPhiZeroRel, 0);
     hipLaunchKernelGGL(k_sc_resid, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, as, x, b, res, res0, 1, partials.p,
                        scal_s.p);
     hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinResid0J, partials.p, scal_s.p);
@@ -7324,7 +7372,9 @@ BcgSys Ctx::Impl::bcg_sys() {
   y.partials = partials.p;
   y.S = scal.p;
   y.stream = stream;
-  y.rec_resid = par.krylov_recurrence && !std::is_same<T, double>::value;
+  y.confirm = std::is_same<T, double>::value && krylov_rec64(nnz, nbs);
+  y.rec_resid = y.confirm || (par.krylov_recurrence && !std::is_same<T, double>::value);
+  y.zero_guess = true;  // the Jacobian kernels (or k_time_term) leave phi = 0 with the right-hand side
   if (par.ilu_sub > 0) {
     y.ilu_sub = par.ilu_sub;
     if constexpr (std::is_same<T, double>::value) {
@@ -7483,6 +7533,7 @@ std::string Ctx::time_step_kernels(int reps, double *ms) {
     y.maxiter = 1 << 30;
     y.zero_abs = 0.0;
     y.zero_rel = 0.0;
+    y.confirm = false;  // the iteration alone
     const int nb = d.nbs;
     ms[2] = timed([&] {
       if (nb == 6) bcg_prologue<T, 6>(y);
@@ -8098,6 +8149,9 @@ BcgSys bcg_on_workspace(const BlockSolve &bs, double *ws, hipStream_t stream) {
   y.A = bs.A;
   y.v[0] = (void *)bs.rhs;
   y.v[1] = bs.phi;
+  // the row pointers are on the device: six blocks a row, a mean of hexahedra
+  // and tetrahedra, stand for A's size
+  y.rec_resid = y.confirm = krylov_rec64(6LL * bs.ncv, 5);
   size_t o = 0;
   y.S = (SolverScalars *)(ws + o);  // first, so it keeps the buffer's alignment
   o += (sizeof(SolverScalars) + 7) / 8 + 32;

@@ -43,3 +43,56 @@ def test_jacobian_per_entry_equals_per_cell(n, frac, precision, scheme, kind):
     a = values(mesh, joe + "GPU_JAC_KERNEL = ENTRY\n", ["A"], precision)["A"]
     b = values(mesh, joe + "GPU_JAC_KERNEL = CELL\n", ["A"], precision)["A"]
     assert np.array_equal(a, b, equal_nan=True)
+
+
+# the block BiCGStab against its own stop test: 1 cell .. several blocks of
+# either launch shape with the true residual, and on both sides of the size
+# from which it takes the recurrence's and confirms it (14k cells); a zero and
+# a near guess, tolerances it reaches and one it cannot
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 1, 1), (7, 3, 2), (4, 13, 1), (8, 8, 8), (23, 23, 23), (25, 25, 25),
+                                  (3, 71, 73)])
+def test_block_solver_true_residual_at_the_stop(dims):
+    print(f"block solver {dims}", flush=True)
+    n = int(np.prod(dims))
+    idx = np.arange(n).reshape(dims)
+    r, c = [np.arange(n)], [np.arange(n)]
+    for ax in range(3):
+        a = np.moveaxis(idx, ax, 0)
+        for x, y in ((a[:-1], a[1:]), (a[1:], a[:-1])):
+            r.append(x.ravel())
+            c.append(y.ravel())
+    row, nv = np.concatenate(r), np.concatenate(c)
+    order = np.argsort(row, kind="stable")  # the diagonal stays first in its row
+    row, nv = row[order], nv[order].astype(np.int32)
+    ni = np.searchsorted(row, np.arange(n + 1)).astype(np.int32)
+    g = np.random.default_rng(n)
+    A = 0.1 * g.standard_normal((len(nv), 5, 5)) - 0.6 * np.eye(5)
+    A[ni[:-1]] += 5.0 * np.eye(5)
+    inv = np.linalg.inv(A[ni[:-1]])
+
+    def mul(x):
+        return np.add.reduceat(np.einsum("kij,kj->ki", A, x[nv]), ni[:-1], axis=0)
+
+    x = g.standard_normal((n, 5))
+    rhs = mul(x)
+    t = joemi.DeviceArray
+    d = [t(v) for v in (ni, nv, A, rhs)]
+
+    def resid(phi):  # the reference's stop measure
+        return np.max(np.abs(np.einsum("cij,cj->ci", inv, rhs - mul(phi))))
+
+    # from the near guess 1e-10 would be a residual below 1e-12, where the
+    # solver's absolute guards (t.t + 1e-20) stall it
+    zero, near = np.zeros((n, 5)), x + 1e-3 * g.standard_normal((n, 5))
+    for guess, rels in ((zero, (1e-2, 1e-6, 1e-10)), (near, (1e-2, 1e-6))):
+        for rel in rels:
+            phi = t(guess)
+            it, st = joemi.block_bcgstab(*d, phi, zero_abs=1e-300, zero_rel=rel, max_iter=60)
+            assert st == 1 and it >= 1
+            # the device's test is taken on this residual up to its rounding
+            # (a few dozen sums of terms of size 5: 1e-13)
+            assert resid(phi.numpy()) <= rel * (resid(guess) + 1e-12) * (1 + 1e-6) + 1e-13
+        phi = t(guess)
+        it, st = joemi.block_bcgstab(*d, phi, zero_abs=0.0, zero_rel=1e-30, max_iter=60)
+        # stalled by those guards, |t| near 1e-10: at the solution to ten times that
+        assert st in (0, 1, 2) and np.max(np.abs(phi.numpy() - x)) <= 1e-9 * np.max(np.abs(x))
