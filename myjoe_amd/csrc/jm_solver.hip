@@ -92,6 +92,10 @@ struct DParams {
   // when set, the viscous per-entry flux kernel writes each face's laminar
   // and eddy viscosity [nfa][2] (device face order), as it used them
   double *vdump;
+  // laminar and eddy viscosity of every face [nfa][2] (device face order),
+  // evaluated once per residual: k_face_visc, and the flux kernel for the
+  // eddy viscosities that need the cells' model fields
+  double *muf;
 };
 
 // per-cell Spalart-Allmaras fields in DParams::sa_aux
@@ -1202,15 +1206,18 @@ __device__ __forceinline__ VSide vside_bfa(const double *bb, const double *gv) {
   return s;
 }
 
-// geometry of an internal face for the viscous terms: icv0 -> icv1 unit
-// vector and distance, and the distance-weighted face temperature's mul
-// (calcMaterialProperties, UgpWithCvCompFlow.h:1700-1750)
-__device__ __forceinline__ void visc_internal_geom(const DParams &P, const double *x0, const double *x1,
-                                                   const double *xfa, double T0, double T1, double sVec[3],
-                                                   double &smag, double &mul, double &w0, double &w1) {
+// geometry of an internal face for the viscous terms: the icv0 -> icv1 unit
+// vector and distance
+__device__ __forceinline__ void visc_dir(const double *x0, const double *x1, double sVec[3], double &smag) {
   for (int i = 0; i < 3; i++) sVec[i] = x1[i] - x0[i];
   smag = sqrt(dot3(sVec, sVec));
   for (int i = 0; i < 3; i++) sVec[i] /= smag;
+}
+
+// and the distances of its centroid from the two cells (the weights of face
+// values, calcMaterialProperties, UgpWithCvCompFlow.h:1700-1750)
+__device__ __forceinline__ void visc_weights(const double *x0, const double *x1, const double *xfa, double &w0,
+                                             double &w1) {
   double dx0[3], dx1[3];
   for (int i = 0; i < 3; i++) {
     dx0[i] = xfa[i] - x0[i];
@@ -1218,6 +1225,14 @@ __device__ __forceinline__ void visc_internal_geom(const DParams &P, const doubl
   }
   w0 = sqrt(dot3(dx0, dx0));
   w1 = sqrt(dot3(dx1, dx1));
+}
+
+// all of it, and the distance-weighted face temperature's mul
+__device__ __forceinline__ void visc_internal_geom(const DParams &P, const double *x0, const double *x1,
+                                                   const double *xfa, double T0, double T1, double sVec[3],
+                                                   double &smag, double &mul, double &w0, double &w1) {
+  visc_dir(x0, x1, sVec, smag);
+  visc_weights(x0, x1, xfa, w0, w1);
   mul = mu_lam(P, (w1 * T0 + w0 * T1) / (w0 + w1));
 }
 
@@ -1373,6 +1388,45 @@ __device__ __forceinline__ double sa_mut_face(double w0, double w1, double rho0,
   double rho_fa = (w1 * rho0 + w0 * rho1) / (w0 + w1);
   double nuSA_fa = (w1 * nu0 + w0 * nu1) / (w0 + w1);
   return sa_mut(rho_fa * nuSA_fa, mul);
+}
+
+// The faces' viscosities once per residual, one thread per face: mul of every
+// face, mut of the SA model's internal faces, mut = 0 elsewhere (SST's, and
+// boundary faces', need the cells' model fields: the flux kernel writes
+// them). The cells' averages, the flux, the Jacobian and the scalar rows
+// each evaluated them from both sides of the face, two or three pow() calls
+// in each. On the 2M-cell SA plate (FP32 Jacobian): this kernel 148 us, the
+// cells' averages 951 -> 672, the flux 930 -> 788, the Jacobian 2705 -> 2497.
+__global__ void __launch_bounds__(kBlock) k_face_visc(DMesh m, DParams P, const int2 *__restrict__ fcell,
+                                                      const double *__restrict__ prim,
+                                                      const double *__restrict__ bfa) {
+  const int f = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (f >= m.nfa) return;
+  double mul, mut = 0.0;
+  if (f < m.nfa_b) {
+    mul = mu_lam(P, bfa[8 * (size_t)f + 5]);
+  } else {
+    const int2 cc = fcell[f - m.nfa_b];
+    const double *p0 = prim + 8 * (size_t)cc.x, *p1 = prim + 8 * (size_t)cc.y;
+    const double *xf = m.fgeo + 8 * (size_t)f + 4;
+    double w0, w1;
+    visc_weights(p0 + 5, p1 + 5, xf, w0, w1);
+    const double T0 = p0[4] / (p0[0] * P.R), T1 = p1[4] / (p1[0] * P.R);
+    mul = mu_lam(P, (w1 * T0 + w0 * T1) / (w0 + w1));
+    if (P.sa) mut = sa_mut_face(w0, w1, p0[0], p1[0], P.sa_phi[cc.x], P.sa_phi[cc.y], mul);
+  }
+  *reinterpret_cast<double2 *>(P.muf + 2 * (size_t)f) = make_double2(mul, mut);
+}
+
+// the two cells of every internal face (set-up)
+__global__ void __launch_bounds__(kBlock) k_face_cells(int ncv, int nfa_b, const int *__restrict__ cfl_i,
+                                                       const int2 *__restrict__ cfl, int2 *__restrict__ fcell) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= ncv) return;
+  for (int e = cfl_i[c]; e < cfl_i[c + 1]; e++) {
+    const int2 en = cfl[e];
+    if (en.y >= 0 && en.x >= 0) fcell[en.x - nfa_b] = make_int2(c, en.y);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1848,15 +1902,11 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         const VSide a = vsel(s0, vo, vn), b = vsel(s0, vn, vo);
         const double xa[3] = {s0 ? pc[5] : pn[5], s0 ? pc[6] : pn[6], s0 ? pc[7] : pn[7]};
         const double xb[3] = {s0 ? pn[5] : pc[5], s0 ? pn[6] : pc[6], s0 ? pn[7] : pc[7]};
-        const double xfa[3] = {geo[4], geo[5], geo[6]};
-        double sV[3], smag, mul, w0, w1;
-        visc_internal_geom(P, xa, xb, xfa, a.T, b.T, sV, smag, mul, w0, w1);
+        double sV[3], smag;
+        visc_dir(xa, xb, sV, smag);
         const double alpha = dot3(n, sV);
-        double mut = 0.0;
-        if (P.sa) {
-          const double nuo = P.sa_phi[c], nun = P.sa_phi[en.y];
-          mut = sa_mut_face(w0, w1, a.rho, b.rho, s0 ? nuo : nun, s0 ? nun : nuo, mul);
-        }
+        const double2 mu = ld2(P.muf + 2 * (size_t)f);
+        const double mul = mu.x, mut = mu.y;
         const double ufa[3] = {0.5 * (a.u[0] + b.u[0]), 0.5 * (a.u[1] + b.u[1]), 0.5 * (a.u[2] + b.u[2])};
         double VF[5], tau[3], keff;
         visc_coupled(P, a, b, mul, mut, ufa, area, n, smag, sV, alpha, VF, tau, keff, P.sa != 0);
@@ -1873,10 +1923,8 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         const double xfa[3] = {geo[4], geo[5], geo[6]};
         double sArg[3], smag, alpha;
         visc_coupled_bgeom(z->bc, xfa, pc + 5, n, sArg, smag, alpha);
-        const double mul = mu_lam(P, bb[5]);
-        const double mut = (P.sa && z->bc != kBcWall)
-                               ? sa_mut(pc[0] * P.sa_phi[c], P.sa_aux[kAuxN * (size_t)c + kAuxMue])
-                               : 0.0;
+        const double2 mu = ld2(P.muf + 2 * (size_t)f);
+        const double mul = mu.x, mut = mu.y;
         const VSide lv = vsel(z->bc == kBcNeumann, vb, vo);
         double VF[5], tau[3], keff;
         visc_coupled(P, lv, vb, mul, mut, vb.u, area, n, smag, sArg, alpha, VF, tau, keff, P.sa != 0);
@@ -1933,15 +1981,15 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         if (SST) vn.k = P.sst_phi[en.y];
         const bool s0 = en.x >= 0;
         const VSide &a = s0 ? vo : vn, &b = s0 ? vn : vo;
-        double sV[3], smag, mul, w0, w1;
-        visc_internal_geom(P, s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, a.T, b.T, sV, smag, mul, w0, w1);
-        double mut = 0.0, kine_fa = 0.0;
+        double sV[3], smag;
+        visc_dir(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, sV, smag);
+        const double2 mu = ld2(P.muf + 2 * (size_t)f);
+        const double mul = mu.x, mut = mu.y;
+        double kine_fa = 0.0;
         if (SST) {
-          mut = sst_mut_face(P, m.ncv, w0, w1, a.rho, b.rho, s0 ? c : en.y, s0 ? en.y : c);
+          double w0, w1;
+          visc_weights(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, w0, w1);
           kine_fa = (w1 * a.k + w0 * b.k) / (w0 + w1);
-        } else if (P.sa) {
-          const double nuo = P.sa_phi[c], nun = P.sa_phi[en.y];
-          mut = sa_mut_face(w0, w1, a.rho, b.rho, s0 ? nuo : nun, s0 ? nun : nuo, mul);
         }
         const double ufa[3] = {0.5 * (a.u[0] + b.u[0]), 0.5 * (a.u[1] + b.u[1]), 0.5 * (a.u[2] + b.u[2])};
         visc_face<SST>(P, a, b, mul, mut, ufa, area, n, smag, sV, Fu, FE, vf, kine_fa);
@@ -1960,7 +2008,8 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         const ZoneDev &z = m.zones[-en.y - 1];
         if (z.bc != kBcSymmetry) {
           const double *bb = bfa + 8 * (size_t)f;
-          const double mul = mu_lam(P, bb[5]);
+          const double2 mu = ld2(P.muf + 2 * (size_t)f);
+          const double mul = mu.x, mut = mu.y;
           VSide vb = vside_bfa(bb, gradv + 12 * (size_t)c);
           double kine_fa = 0.0;
           if (SST) {  // walls: kine1 = kine_fa = 0; other zones phi_bfa
@@ -1977,10 +2026,6 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
             smag = sqrt(dot3(sV, sV));
             for (int i = 0; i < 3; i++) sArg[i] = sV[i] / smag;
           }
-          const double mut = z.bc == kBcWall ? 0.0
-                             : SST       ? sst_mut_cell(P, m.ncv, pc[0], c)
-                             : P.sa      ? sa_mut(pc[0] * P.sa_phi[c], P.sa_aux[kAuxN * (size_t)c + kAuxMue])
-                                         : 0.0;
           visc_face<SST>(P, vo, vb, mul, mut, vb.u, area, n, smag, sArg, Fu, FE, vf, kine_fa);
           visc_jac<SST>(P, J, -1.0, vo, mul, mut, vf, vb.u, area, smag);
           for (int i = 1; i < 5; i++)
@@ -2179,25 +2224,11 @@ __global__ void __launch_bounds__(kBlock) k_sa_cell(DMesh m, DParams P, const do
     }
   }
   // face-averaged laminar viscosity over the faocv list
-  const double Tc = pc[4] / (pc[0] * P.R);
   const int nf = e1 - e0;
   double mue = 0.0;
   for (int k = 0; k < nf; k++) {
-    const int e = e0 + m.foc[e0 + k];
-    const int2 en = m.cfl[e];
-    const int f = en.x & 0x7fffffff;
-    double mul;
-    if (en.y >= 0) {
-      const double *pn = prim + 8 * (size_t)en.y;
-      const double Tn = pn[4] / (pn[0] * P.R);
-      const bool s0 = (en.x >= 0);
-      double sV[3], smag, w0, w1;
-      visc_internal_geom(P, s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, m.fgeo + 8 * (size_t)f + 4, s0 ? Tc : Tn,
-                         s0 ? Tn : Tc, sV, smag, mul, w0, w1);
-    } else {
-      mul = mu_lam(P, bfa[8 * (size_t)f + 5]);
-    }
-    mue += mul;
+    const int f = m.cfl[e0 + m.foc[e0 + k]].x & 0x7fffffff;
+    mue += P.muf[2 * (size_t)f];
   }
   mue /= (double)nf;
   // strain and vorticity magnitudes (pow(x, 2.0) is x * x)
@@ -2361,25 +2392,11 @@ __global__ void __launch_bounds__(kBlock) k_sst_cell(DMesh m, DParams P, const d
   sst_grad<LS>(m, P, prim, P.sst_phi + m.ncv, 1, c, gw);
   // face-averaged laminar viscosity over the faocv list
   const int e0 = m.cfl_i[c], e1 = m.cfl_i[c + 1];
-  const double Tc = pc[4] / (pc[0] * P.R);
   const int nf = e1 - e0;
   double mue = 0.0;
   for (int k = 0; k < nf; k++) {
-    const int e = e0 + m.foc[e0 + k];
-    const int2 en = m.cfl[e];
-    const int f = en.x & 0x7fffffff;
-    double mul;
-    if (en.y >= 0) {
-      const double *pn = prim + 8 * (size_t)en.y;
-      const double Tn = pn[4] / (pn[0] * P.R);
-      const bool s0 = (en.x >= 0);
-      double sV[3], smag, w0, w1;
-      visc_internal_geom(P, s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, m.fgeo + 8 * (size_t)f + 4, s0 ? Tc : Tn,
-                         s0 ? Tn : Tc, sV, smag, mul, w0, w1);
-    } else {
-      mul = mu_lam(P, bfa[8 * (size_t)f + 5]);
-    }
-    mue += mul;
+    const int f = m.cfl[e0 + m.foc[e0 + k]].x & 0x7fffffff;
+    mue += P.muf[2 * (size_t)f];
   }
   mue /= (double)nf;
   const double *gu = grad + 16 * (size_t)c + 6;
@@ -2922,14 +2939,14 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
         off1[k] = s0 ? 0.0 + S1[k] : 0.0 - S1[k];
       }
       // diffusion (the cell's second pass)
-      const double Tc = pc[4] / (pc[0] * P.R), Tn = pn[4] / (pn[0] * P.R);
-      double sV[3], smag, mul, w0, w1;
-      visc_internal_geom(P, s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, s0 ? Tc : Tn, s0 ? Tn : Tc, sV, smag,
-                         mul, w0, w1);
+      double sV[3], smag, w0, w1;
+      visc_dir(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, sV, smag);
+      visc_weights(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, w0, w1);
+      const double2 mu = ld2(P.muf + 2 * (size_t)f);
+      const double mul = mu.x, mut = mu.y;
       const int c0 = s0 ? c : nb, c1 = s0 ? nb : c;
       const double rho0 = s0 ? pc[0] : pn[0], rho1 = s0 ? pn[0] : pc[0];
       const double *a0 = P.sst_aux + kSstN * (size_t)c0, *a1 = P.sst_aux + kSstN * (size_t)c1;
-      const double mut = sst_mut_face(P, ncv, w0, w1, rho0, rho1, c0, c1);
       const double f1_fa = (w1 * a0[kSF1] + w0 * a1[kSF1]) / (w0 + w1);
       const double alpha = dot3(n, sV);
       const double nmag = area;
@@ -2975,8 +2992,8 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
         slot[8 + k] = S1[k];
       }
       if (z.skind || z.skind2) {
-        const double mul = mu_lam(P, bb[5]);
-        const double mutb = z.bc != kBcWall ? sst_mut_cell(P, ncv, pc[0], c) : 0.0;
+        const double2 mu = ld2(P.muf + 2 * (size_t)f);
+        const double mul = mu.x, mutb = mu.y;
         const double s_half[3] = {xfa[0] - pc[5], xfa[1] - pc[6], xfa[2] - pc[7]};
         const double smag_half = fabs(dot3(s_half, n));
         const double nmag = area;
@@ -3085,7 +3102,7 @@ __global__ void __launch_bounds__(kBlock) k_sc_update_b(int ncv, const double *_
 // The cell's own values every entry of the scalar row reads.
 struct ScalOwn {
   const double *pc, *gc, *gpc;
-  double ph, hown, Tc;
+  double ph, hown;
   Side own;
 };
 
@@ -3098,7 +3115,6 @@ __device__ __forceinline__ ScalOwn scal_own(const DParams &P, const double *__re
   o.ph = P.sa_phi[c];
   o.own.rho = o.pc[0]; o.own.u[0] = o.pc[1]; o.own.u[1] = o.pc[2]; o.own.u[2] = o.pc[3]; o.own.p = o.pc[4];
   o.hown = enthalpy_of(P, o.own.rho, o.own.p);
-  o.Tc = o.pc[4] / (o.pc[0] * P.R);
   return o;
 }
 
@@ -3176,10 +3192,10 @@ __device__ __forceinline__ void scal_c_entry(const DMesh &m, const DParams &P, c
       }
     }
     {  // the face's scalar diffusion (:5076-5105)
-      const double Tn = pn[4] / (pn[0] * P.R);
-      double sV[3], smag, mul, w0, w1;
-      visc_internal_geom(P, s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, s0 ? o.Tc : Tn, s0 ? Tn : o.Tc, sV,
-                         smag, mul, w0, w1);
+      double sV[3], smag, w0, w1;
+      visc_dir(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, sV, smag);
+      visc_weights(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, w0, w1);
+      const double mul = P.muf[2 * (size_t)f];
       const double rho0 = s0 ? pc[0] : pn[0], rho1 = s0 ? pn[0] : pc[0];
       const double nu0 = s0 ? ph : phn, nu1 = s0 ? phn : ph;
       const double *g0 = s0 ? gpc : gpn, *g1 = s0 ? gpn : gpc;
@@ -3212,7 +3228,7 @@ __device__ __forceinline__ void scal_c_entry(const DMesh &m, const DParams &P, c
     // a zone without a nuSA value carries no diffusive scalar flux
     // (DiffTerm = 0, :5453-5461, 5599-5607); NEUMANN zones keep it (:5293-5296)
     const double DiffTerm = (z.bc == kBcNeumann || z.skind) ? 1.0 : 0.0;
-    const double mul = mu_lam(P, bb[5]);
+    const double mul = P.muf[2 * (size_t)f];
     const double diff = z.bc == kBcWall ? invSigma * mul : invSigma * (mul + rb * phb);
     if (z.bc == kBcSymmetry || z.bc == kBcWall || z.bc == kBcNeumann) {
       const bool op = z.bc != kBcNeumann && P.symm_bc == kSymmAnalytical;  // ONLY_PRESSURE (:1910-1917)
@@ -3669,7 +3685,9 @@ __global__ void __launch_bounds__(kBlock) k_flux(DMesh m, DParams P, const doubl
 // order), applies the gravity source, and writes the residual and local dt.
 // SST: the sides' turbulent kinetic energy in the HLLC flux (kineFA, JoeWithModels.cpp:2924-2930,
 // 3140-3147, 3466-3471), the kinetic-energy viscous terms and the SST eddy viscosity
-template <int SCHEME, bool SND, bool VISC, int W = kWaves, bool SST = false>
+// MUF: the faces' viscosities are in DParams::muf (see k_face_visc); a batched
+// solve evaluates them here
+template <int SCHEME, bool SND, bool VISC, int W = kWaves, bool SST = false, bool MUF = false>
 __device__ __forceinline__ void d_flux_e(const Blk &B, DMesh m, DParams P, const double *__restrict__ prim,
                                                    const double *__restrict__ grad, const double *__restrict__ bfa,
                                                    const double *__restrict__ q, double *__restrict__ rhs,
@@ -3791,13 +3809,22 @@ __device__ __forceinline__ void d_flux_e(const Blk &B, DMesh m, DParams P, const
           vn.k = kn;
         }
         const VSide &a = s0 ? vo : vn, &b = s0 ? vn : vo;
-        double sV[3], smag, w0, w1;
-        visc_internal_geom(P, s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, xfa, a.T, b.T, sV, smag, mul, w0, w1);
+        double sV[3], smag, w0 = 0.0, w1 = 0.0;
+        const double *xa = s0 ? pc + 5 : pn + 5, *xb = s0 ? pn + 5 : pc + 5;
+        if (MUF) {
+          visc_dir(xa, xb, sV, smag);
+          if (SST) visc_weights(xa, xb, xfa, w0, w1);
+          const double2 mu = ld2(P.muf + 2 * (size_t)f);
+          mul = mu.x;
+          mut = mu.y;
+        } else {
+          visc_internal_geom(P, xa, xb, xfa, a.T, b.T, sV, smag, mul, w0, w1);
+        }
         double kine_fa = 0.0;
         if (SST) {
           mut = sst_mut_face(P, m.ncv, w0, w1, a.rho, b.rho, s0 ? L.c : en.y, s0 ? en.y : L.c);
           kine_fa = (w1 * a.k + w0 * b.k) / (w0 + w1);
-        } else if (P.sa) {
+        } else if (!MUF && P.sa) {
           const double nuo = P.sa_phi[L.c], nun = P.sa_phi[en.y];
           mut = sa_mut_face(w0, w1, a.rho, b.rho, s0 ? nuo : nun, s0 ? nun : nuo, mul);
         }
@@ -3847,7 +3874,7 @@ __device__ __forceinline__ void d_flux_e(const Blk &B, DMesh m, DParams P, const
         if (SCHEME == kHllcC) hl = enthalpy_of(P, so.rho, so.p);
       }
       if (VISC && CPL) {  // calcFluxCoupled boundary faces; mul from T_bfa
-        mul = mu_lam(P, bb[5]);
+        mul = MUF ? P.muf[2 * (size_t)f] : mu_lam(P, bb[5]);
         if (P.sa && z.bc != kBcWall)  // mut_fa of calcRansTurbViscMuet (TurbModel_SA.h:112-120)
           mut = sa_mut(pc[0] * P.sa_phi[L.c], P.sa_aux[kAuxN * (size_t)L.c + kAuxMue]);
         const double *gvo = gradv + 12 * (size_t)L.c;
@@ -3865,7 +3892,7 @@ __device__ __forceinline__ void d_flux_e(const Blk &B, DMesh m, DParams P, const
           for (int k = 0; k < 5; k++) vcc[k] = -VF[k];
         }
       } else if (VISC) {  // boundary faces (:3714-3851); boundary mul from T_bfa (ComputeBCProperties_T)
-        mul = mu_lam(P, bb[5]);
+        mul = MUF ? P.muf[2 * (size_t)f] : mu_lam(P, bb[5]);
         if (SST && z.bc != kBcWall)  // mut of every non-wall boundary face, symmetry included (calcDt reads it)
           mut = sst_mut_cell(P, m.ncv, pc[0], L.c);
         else if (P.sa && z.bc != kBcWall)
@@ -3915,6 +3942,7 @@ __device__ __forceinline__ void d_flux_e(const Blk &B, DMesh m, DParams P, const
     }
     if (P.fdump && en.x >= 0)
       for (int k = 0; k < 5; k++) P.fdump[5 * (size_t)f + k] = F[k];
+    if (VISC && MUF && (SST ? en.x >= 0 : en.y < 0)) P.muf[2 * (size_t)f + 1] = mut;
     if (VISC && P.vdump && en.x >= 0) {
       P.vdump[2 * (size_t)f] = mul;
       P.vdump[2 * (size_t)f + 1] = mut;
@@ -4005,7 +4033,7 @@ __global__ void __launch_bounds__(64 * kFluxWaves) k_flux_e(DMesh m, DParams P, 
                                                             int *__restrict__ nfirst, DtArgs dta,
                                                             double *__restrict__ dt, double *__restrict__ partials,
                                                             const double *__restrict__ gradv) {
-  d_flux_e<SCHEME, SND, VISC, kFluxWaves, SST>(hw_blk(), m, P, prim, grad, bfa, q, rhs, nfirst, dta, dt, partials,
+  d_flux_e<SCHEME, SND, VISC, kFluxWaves, SST, VISC>(hw_blk(), m, P, prim, grad, bfa, q, rhs, nfirst, dta, dt, partials,
                                                gradv);
 }
 
@@ -5734,7 +5762,8 @@ struct Ctx::Impl {
   // state
   DBuf<double> q, prim, grad, bfa, rhs, dt, hook;
   DBuf<double> gradv;  // [ncv][12] velocity and enthalpy gradients of the viscous flux
-  DBuf<int2> fcell;    // [nfa_i] device cells (icv0, icv1) of each internal face (face form of the flux)
+  DBuf<int2> fcell;    // [nfa_i] device cells (icv0, icv1) of each internal face (face form of the flux, k_face_visc)
+  DBuf<double> muf;    // [nfa][2] the faces' viscosities (k_face_visc)
   DBuf<double> fflux;  // [nfa_i][5] face fluxes of the face form
   bool face_form() const { return par.flux_kernel == kResidFace && !dp.visc; }
   DBuf<int> counters;  // [0] negative pressure, [1] first-order fallbacks
@@ -6294,6 +6323,13 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
                      d.nbocv_v.p, d.cfl_tnoc.p);
   HIPCHECK(hipGetLastError());
   d.dm.cfl_tnoc = d.cfl_tnoc.p;
+  if (d.par.mu_ref > 0.0) {
+    d.muf.alloc(2 * (size_t)std::max(1, nfa));
+    d.fcell.alloc(std::max(1, nfa - nfa_b));
+    hipLaunchKernelGGL(k_face_cells, dim3(nblk(ncv)), dim3(kBlock), 0, d.stream, ncv, nfa_b, d.cfl_i.p, d.cfl_e.p,
+                       d.fcell.p);
+    HIPCHECK(hipGetLastError());
+  }
   d.dm.nbocv_i = d.nbocv_i.p;
   d.dm.nbocv_v = d.nbocv_v.p;
   d.dm.lsg = d.lsg.p;
@@ -6335,6 +6371,7 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
   d.dp.sa_prof = d.sa_prof.p;
   d.dp.fdump = nullptr;
   d.dp.vdump = nullptr;
+  d.dp.muf = d.muf.p;
   d.dp.sa_aux = d.sa_aux.p;
   d.dp.sst = d.par.sst ? 1 : 0;
   d.dp.sst_limit_pk = d.par.sst_limit_pk;
@@ -6369,10 +6406,10 @@ size_t Ctx::footprint(const Mesh &m, int precision) {
   const size_t ent = 2 * (nfa - nfa_b) + nfa_b;
   const size_t sJ = precision == 0 ? 8 : 4;
   size_t b = 0;
-  b += nfa * (8 + 3) * 8;                          // fgeo, fnorm
+  b += nfa * (8 + 3) * 8;  // fgeo; fnorm, or without it muf, fcell and cfl_tnoc
   b += nnz * (3 * 8 + 4) + nfa_b * (3 * 8 + 4 + 4);  // lsg, nbocv_v, bfa_lsg, bfa_cell, bfa_zone
   b += (ncv + 1) * 4 * 2 + ncv * 4;                // cfl_i, nbocv_i, wave table
-  b += ent * (8 + 8 + 8 + 24);                     // entries, their two blocks, their cells and positions, limiter offsets
+  b += ent * (8 + 4 + 8 + 24);                     // entries, their blocks, their cells and positions, limiter offsets
   b += ncv * (5 + 8 + 16 + 5 + 1 + 1) * 8;         // q, prim, grad, rhs, dt, vol
   b += nfa_b * (8 + 5) * 8;                        // bfa, hook
   b += (nnz + ncv) * 25 * sJ + 10 * ncv * 5 * sJ;  // A, LU, Krylov vectors
@@ -7014,6 +7051,7 @@ void Ctx::Impl::launch_grad(hipStream_t s) {
       else hipLaunchKernelGGL((k_grad<false, false>), g, dim3(kBlock), 0, s, dm, dp, prim.p, bfa.p, grad.p, gradv.p);
     }
   }
+  if (dp.visc) hipLaunchKernelGGL(k_face_visc, dim3(nblk(nfa)), dim3(kBlock), 0, s, dm, dp, fcell.p, prim.p, bfa.p);
   if (par.sa) {  // nuSA gradient, face-averaged mul, strain and vorticity
     if (par.grad_ls)
       hipLaunchKernelGGL(k_sa_cell<true>, dim3(nblk(ncv)), dim3(kBlock), 0, s, dm, dp, prim.p, bfa.p, grad.p, sa_aux.p);
