@@ -2853,14 +2853,18 @@ __global__ void __launch_bounds__(kBlock) k_sst_scal(DMesh m, DParams P, const d
 }
 
 // The same rows per cell-face entry: a lane evaluates its entry's face for
-// both scalars, writes the off-diagonal AScal entries it owns, and leaves its
-// contributions to the cell's sums in LDS: the convective acc (2) and
+// both scalars, its own cell's side of the face's matrices only (negated they
+// are the entries of the cell's column in the neighbour's row, written from
+// LDS by the wavefront: see k_jac_e), and leaves its contributions to the
+// cell's sums in LDS: the convective acc (2) and
 // diagonal entries (2 x 6, signed for the cell: d - s == d + (-s)), then the
 // diffusive acc (2) and diagonal [5] (2), -0.0 where it adds nothing. The
 // owner lane sums the convective terms of the cell's entries in entry order,
 // then the diffusive ones, then adds the sources, as k_sst_scal does; so the
 // bits are k_sst_scal's. Each off-diagonal block has one writer (the SST path
 // requires a mesh without duplicate neighbour pairs).
+// One side's matrices per lane and one evaluation for internal and boundary
+// entries: 687k-cell SST plate 703 -> 608 us.
 constexpr int kSstScalWaves = 1;
 
 __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DParams P, const double *__restrict__ prim,
@@ -2869,6 +2873,7 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
                                                                   double *__restrict__ rhs_s, double *__restrict__ AS) {
   constexpr int NS = 18;
   __shared__ double lds[64 * kSstScalWaves * NS];
+  __shared__ int toff[64 * kSstScalWaves];  // the entry's off-diagonal block, -1 without one
   double *slot = lds + NS * threadIdx.x;
   const EntryLane L = entry_lane<kSstScalWaves>(m, hw_blk());
   const int ncv = m.ncv;
@@ -2879,6 +2884,7 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
   const double *pc = prim + 8 * (size_t)c;
   const double *auxc = P.sst_aux + kSstN * (size_t)c;
   const double kc = kin[c], wc = omg[c];
+  toff[threadIdx.x] = L.e >= 0 ? m.cfl_tnoc[L.e] : -1;
   if (L.e >= 0) {
     const double gam = P.gamma;
     const bool snd = P.second_order != 0;
@@ -2893,51 +2899,65 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
     const double area = geo[3];
     const double xfa[3] = {geo[4], geo[5], geo[6]};
     double dacc0 = -0.0, dacc1 = -0.0, dd0 = -0.0, dd1 = -0.0;  // diffusive terms
-    if (en.y >= 0) {
-      const int nb = en.y;
-      const double *pn = prim + 8 * (size_t)nb;
-      const double *auxn = P.sst_aux + kSstN * (size_t)nb;
-      const double kn = kin[nb], wn = omg[nb];
-      Side nbs;
-      nbs.rho = pn[0]; nbs.u[0] = pn[1]; nbs.u[1] = pn[2]; nbs.u[2] = pn[3]; nbs.p = pn[4];
-      Side so = own, sn = nbs;
-      double kfo = kc, kfn = kn, wfo = wc, wfn = wn;
-      if (snd) {
-        if (reconstruct(so, pc, gc, xfa)) {
-          const double r[3] = {xfa[0] - pc[5], xfa[1] - pc[6], xfa[2] - pc[7]};
-          kfo = kfo + dot3(r, auxc + kSGradK);
-          wfo = wfo + dot3(r, auxc + kSGradW);
-        }
-        if (reconstruct(sn, pn, grad + 16 * (size_t)nb, xfa)) {
-          const double r[3] = {xfa[0] - pn[5], xfa[1] - pn[6], xfa[2] - pn[7]};
-          kfn = kfn + dot3(r, auxn + kSGradK);
-          wfn = wfn + dot3(r, auxn + kSGradW);
-        }
+    const bool internal = en.y >= 0;
+    const bool s0 = !internal || en.x >= 0;
+    const int nb = internal ? en.y : c;
+    const double *pn = prim + 8 * (size_t)nb;
+    const double *bb = bfa + 8 * (size_t)(internal ? 0 : f);
+    const ZoneDev *z = m.zones + (internal ? 0 : -en.y - 1);
+    const bool reflect = !internal && (z->bc == kBcSymmetry || z->bc == kBcWall);
+    const double kb = internal ? 0.0 : P.sst_bfa[2 * (size_t)f], wb = internal ? 0.0 : P.sst_bfa[2 * (size_t)f + 1];
+    // the face's two sides (the boundary's: its state, on both sides of a wall
+    // or symmetry face), for the flux and for the matrices; then one
+    // evaluation of each
+    Side fo = own, fn, jn, jo = own;  // this cell's side and the other
+    double kfo = kc, wfo = wc, kfn, wfn, kjo = kc, wjo = wc, kjn, wjn;
+    if (snd && !reflect && reconstruct(fo, pc, gc, xfa)) {
+      const double r[3] = {xfa[0] - pc[5], xfa[1] - pc[6], xfa[2] - pc[7]};
+      kfo = kfo + dot3(r, auxc + kSGradK);
+      wfo = wfo + dot3(r, auxc + kSGradW);
+    }
+    if (internal) {
+      kfn = kjn = kin[nb];
+      wfn = wjn = omg[nb];
+      jn.rho = pn[0]; jn.u[0] = pn[1]; jn.u[1] = pn[2]; jn.u[2] = pn[3]; jn.p = pn[4];
+      fn = jn;
+      if (snd && reconstruct(fn, pn, grad + 16 * (size_t)nb, xfa)) {
+        const double *auxn = P.sst_aux + kSstN * (size_t)nb;
+        const double r[3] = {xfa[0] - pn[5], xfa[1] - pn[6], xfa[2] - pn[7]};
+        kfn = kfn + dot3(r, auxn + kSGradK);
+        wfn = wfn + dot3(r, auxn + kSGradW);
       }
-      const bool s0 = en.x >= 0;
-      const int noc = m.cfl_noc[L.e] & 0x3fffffff;
-      double *off0 = AS + 6 * (size_t)noc, *off1 = AS1 + 6 * (size_t)noc;
-      const Side fl = s0 ? so : sn, fr = s0 ? sn : so;
-      const Side jl = s0 ? own : nbs, jr = s0 ? nbs : own;
-      const double kl = s0 ? kfo : kfn, kr = s0 ? kfn : kfo, kjl = s0 ? kc : kn, kjr = s0 ? kn : kc;
-      const double wl = s0 ? wfo : wfn, wr = s0 ? wfn : wfo, wjl = s0 ? wc : wn, wjr = s0 ? wn : wc;
+    } else {
+      jn.rho = bb[0]; jn.u[0] = bb[1]; jn.u[1] = bb[2]; jn.u[2] = bb[3]; jn.p = bb[4];
+      fn = jn;
+      kfn = kjn = kb;
+      wfn = wjn = wb;
+      if (reflect) {
+        fo = jn;
+        jo = jn;
+        kfo = kjo = kb;
+        wfo = wjo = wb;
+      }
+    }
+    {
+      const Side fl = s0 ? fo : fn, fr = s0 ? fn : fo;
+      const double kl = s0 ? kfo : kfn, kr = s0 ? kfn : kfo, wl = s0 ? wfo : wfn, wr = s0 ? wfn : wfo;
       flux_hllc(F, fl.rho, fl.u, fl.p, fr.rho, fr.u, fr.p, gam, area, n, kl, kr, &Fs0, kl, kr, &Fs1, wl, wr);
       slot[0] = s0 ? -Fs0 : Fs0;
       slot[1] = s0 ? -Fs1 : Fs1;
+    }
+    {
       // the diagonal's side (icv0 adds A_L's rows, icv1 subtracts A_R's)
-      jac_hllc_scal2(S0, S1, s0 ? 0 : 1, jl.rho, jl.u, jl.p, jr.rho, jr.u, jr.p, gam, area, n, kjl, kjr, wjl, wjr, kjl,
-                     kjr);
+      const Side jl = s0 ? jo : jn, jr = s0 ? jn : jo;
+      const double kl = s0 ? kjo : kjn, kr = s0 ? kjn : kjo, wl = s0 ? wjo : wjn, wr = s0 ? wjn : wjo;
+      jac_hllc_scal2(S0, S1, s0 ? 0 : 1, jl.rho, jl.u, jl.p, jr.rho, jr.u, jr.p, gam, area, n, kl, kr, wl, wr, kl, kr);
       for (int k = 0; k < 6; k++) {
         slot[2 + k] = s0 ? S0[k] : -S0[k];
         slot[8 + k] = s0 ? S1[k] : -S1[k];
       }
-      // the off-diagonal block (icv0's = +A_R's rows, icv1's = -A_L's)
-      jac_hllc_scal2(S0, S1, s0 ? 1 : 0, jl.rho, jl.u, jl.p, jr.rho, jr.u, jr.p, gam, area, n, kjl, kjr, wjl, wjr, kjl,
-                     kjr);
-      for (int k = 0; k < 6; k++) {
-        off0[k] = s0 ? 0.0 + S0[k] : 0.0 - S0[k];
-        off1[k] = s0 ? 0.0 + S1[k] : 0.0 - S1[k];
-      }
+    }
+    if (internal) {
       // diffusion (the cell's second pass)
       double sV[3], smag, w0, w1;
       visc_dir(s0 ? pc + 5 : pn + 5, s0 ? pn + 5 : pc + 5, sV, smag);
@@ -2950,7 +2970,7 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
       const double f1_fa = (w1 * a0[kSF1] + w0 * a1[kSF1]) / (w0 + w1);
       const double alpha = dot3(n, sV);
       const double nmag = area;
-      auto face = [&](double sg1, double sg2, const double *phi, int gS, double &dacc, double &dd, double *off) {
+      auto face = [&](double sg1, double sg2, const double *phi, int gS, double &dacc, double &dd) {
         const double coeff = sg1 * f1_fa + (1. - f1_fa) * sg2;
         const double diff = mul + coeff * mut;
         const double phi0 = phi[c0], phi1 = phi[c1];
@@ -2962,36 +2982,11 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
         const double a = diff * nmag * alpha / smag;
         dacc = s0 ? viscFlux : -viscFlux;
         dd = s0 ? a / rho0 : a / rho1;
-        off[5] = off[5] + -(s0 ? a / rho1 : a / rho0);
       };
-      face(kSstSigmaK1, kSstSigmaK2, kin, kSGradK, dacc0, dd0, off0);
-      face(kSstSigmaW1, kSstSigmaW2, omg, kSGradW, dacc1, dd1, off1);
+      face(kSstSigmaK1, kSstSigmaK2, kin, kSGradK, dacc0, dd0);
+      face(kSstSigmaW1, kSstSigmaW2, omg, kSGradW, dacc1, dd1);
     } else {
-      const ZoneDev &z = m.zones[-en.y - 1];
-      const double *bb = bfa + 8 * (size_t)f;
-      const double kb = P.sst_bfa[2 * (size_t)f], wb = P.sst_bfa[2 * (size_t)f + 1];
-      const double ub[3] = {bb[1], bb[2], bb[3]};
-      if (z.bc == kBcSymmetry || z.bc == kBcWall) {
-        flux_hllc(F, bb[0], ub, bb[4], bb[0], ub, bb[4], gam, area, n, kb, kb, &Fs0, kb, kb, &Fs1, wb, wb);
-        jac_hllc_scal2(S0, S1, 0, bb[0], ub, bb[4], bb[0], ub, bb[4], gam, area, n, kb, kb, wb, wb, kb, kb);
-      } else {
-        Side so = own;
-        double kfo = kc, wfo = wc;
-        if (snd && reconstruct(so, pc, gc, xfa)) {
-          const double r[3] = {xfa[0] - pc[5], xfa[1] - pc[6], xfa[2] - pc[7]};
-          kfo = kfo + dot3(r, auxc + kSGradK);
-          wfo = wfo + dot3(r, auxc + kSGradW);
-        }
-        flux_hllc(F, so.rho, so.u, so.p, bb[0], ub, bb[4], gam, area, n, kfo, kb, &Fs0, kfo, kb, &Fs1, wfo, wb);
-        jac_hllc_scal2(S0, S1, 0, own.rho, own.u, own.p, bb[0], ub, bb[4], gam, area, n, kc, kb, wc, wb, kc, kb);
-      }
-      slot[0] = -Fs0;
-      slot[1] = -Fs1;
-      for (int k = 0; k < 6; k++) {
-        slot[2 + k] = S0[k];
-        slot[8 + k] = S1[k];
-      }
-      if (z.skind || z.skind2) {
+      if (z->skind || z->skind2) {
         const double2 mu = ld2(P.muf + 2 * (size_t)f);
         const double mul = mu.x, mutb = mu.y;
         const double s_half[3] = {xfa[0] - pc[5], xfa[1] - pc[6], xfa[2] - pc[7]};
@@ -2999,15 +2994,15 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
         const double nmag = area;
         auto bface = [&](double sg1, double sg2, double phb, double ph, double &dacc, double &dd) {
           double diff = mul;
-          if (z.bc != kBcWall) {
+          if (z->bc != kBcWall) {
             const double coeff = sg1 * auxc[kSF1] + (1. - auxc[kSF1]) * sg2;
             diff = mul + coeff * mutb;
           }
           dacc = diff * nmag * (phb - ph) / smag_half;
           dd = diff * nmag / smag_half / pc[0];
         };
-        if (z.skind) bface(kSstSigmaK1, kSstSigmaK2, kb, kc, dacc0, dd0);
-        if (z.skind2) bface(kSstSigmaW1, kSstSigmaW2, wb, wc, dacc1, dd1);
+        if (z->skind) bface(kSstSigmaK1, kSstSigmaK2, kb, kc, dacc0, dd0);
+        if (z->skind2) bface(kSstSigmaW1, kSstSigmaW2, wb, wc, dacc1, dd1);
       }
     }
     slot[14] = dacc0;
@@ -3016,6 +3011,18 @@ __global__ void __launch_bounds__(64 * kSstScalWaves) k_sst_scal_e(DMesh m, DPar
     slot[17] = dd1;
   }
   __syncthreads();
+  {
+    const int wb = threadIdx.x & ~63;
+    for (int it = 0; it < 12; it++) {
+      const int q = it < 6 ? 0 : 1, idx = (it - 6 * q) * 64 + (threadIdx.x & 63), en = idx / 6, k = idx - 6 * en;
+      const int tn = toff[wb + en];
+      if (tn < 0) continue;
+      const double *sj = lds + NS * (wb + en);
+      double v = 0.0 - sj[2 + 6 * q + k];
+      if (k == 5) v = v + -sj[16 + q];
+      (q ? AS1 : AS)[6 * (size_t)tn + k] = v;
+    }
+  }
   if (L.e < 0 || L.pos != 0) return;
   const int nent = m.cfl_i[c + 1] - m.cfl_i[c];
   double acc0 = 0.0, acc1 = 0.0;
@@ -3124,8 +3131,10 @@ __device__ __forceinline__ ScalOwn scal_own(const DParams &P, const double *__re
 // diffusion (out[8] to [5][0], out[9] to [5][5]); -0.0 where the entry adds
 // nothing (x + -0.0 is x, signed zeros included), and subtractions stored
 // negated (a - b is a + (-b)). With A, row 5 of the entry's off-diagonal
-// block is written (internal faces).
-template <typename T, bool SND>
+// block is written (internal faces), unless OWN: then only this cell's side
+// of the face's matrices is evaluated, which negated is the row of the cell's
+// column in the neighbour's block (k_scal_e writes it from the slots).
+template <typename T, bool SND, bool OWN = false>
 __device__ __forceinline__ void scal_c_entry(const DMesh &m, const DParams &P, const double *__restrict__ prim,
                                              const double *__restrict__ grad, const double *__restrict__ bfa,
                                              T *__restrict__ A, const ScalOwn &o, int e, double out[10]) {
@@ -3165,7 +3174,7 @@ __device__ __forceinline__ void scal_c_entry(const DMesh &m, const DParams &P, c
     const bool s0 = en.x >= 0;
     const int noc = m.cfl_noc[e];
     const bool accum = (noc >> 30) & 1;
-    T *off = A ? A + 36 * (size_t)(noc & 0x3fffffff) + 30 : nullptr;
+    T *off = A && !OWN ? A + 36 * (size_t)(noc & 0x3fffffff) + 30 : nullptr;
     T ov[6];  // row 5 of the off-diagonal block, kept until its one store
     // the face's (icv0, icv1) sides; the flux and both rows evaluated once,
     // routed by this cell's side
@@ -3178,16 +3187,21 @@ __device__ __forceinline__ void scal_c_entry(const DMesh &m, const DParams &P, c
       const Side jl = s0 ? own : nbs, jr = s0 ? nbs : own;
       const double hjl = enthalpy_of(P, jl.rho, jl.p), hjr = enthalpy_of(P, jr.rho, jr.p);
       const double pjl = s0 ? ph : phn, pjr = s0 ? phn : ph;
-      jac_hllc_coupled_srow(S, 0, jl.rho, jl.u, jl.p, hjl, pjl, jr.rho, jr.u, jr.p, hjr, pjr, gam, area, n);
-      jac_hllc_coupled_srow(R6, 1, jl.rho, jl.u, jl.p, hjl, pjl, jr.rho, jr.u, jr.p, hjr, pjr, gam, area, n);
-      // icv0: A[noc00] += SL, A[noc01] += SR; icv1: A[noc11] -= SR, A[noc10] -= SL
-      for (int k = 0; k < 6; k++) {
-        if (s0) {
-          out[2 + k] = S[k];
-          ov[k] = (T)(accum ? (double)off[k] + R6[k] : 0.0 + R6[k]);
-        } else {
-          out[2 + k] = -R6[k];
-          ov[k] = (T)(accum ? (double)off[k] - S[k] : 0.0 - S[k]);
+      jac_hllc_coupled_srow(S, OWN && !s0 ? 1 : 0, jl.rho, jl.u, jl.p, hjl, pjl, jr.rho, jr.u, jr.p, hjr, pjr, gam,
+                            area, n);
+      if (OWN) {
+        for (int k = 0; k < 6; k++) out[2 + k] = s0 ? S[k] : -S[k];
+      } else {
+        jac_hllc_coupled_srow(R6, 1, jl.rho, jl.u, jl.p, hjl, pjl, jr.rho, jr.u, jr.p, hjr, pjr, gam, area, n);
+        // icv0: A[noc00] += SL, A[noc01] += SR; icv1: A[noc11] -= SR, A[noc10] -= SL
+        for (int k = 0; k < 6; k++) {
+          if (s0) {
+            out[2 + k] = S[k];
+            ov[k] = (T)(accum ? (double)off[k] + R6[k] : 0.0 + R6[k]);
+          } else {
+            out[2 + k] = -R6[k];
+            ov[k] = (T)(accum ? (double)off[k] - S[k] : 0.0 - S[k]);
+          }
         }
       }
     }
@@ -3209,15 +3223,15 @@ __device__ __forceinline__ void scal_c_entry(const DMesh &m, const DParams &P, c
         if (s0) {
           out[8] = a0[0];
           out[9] = a0[1];
-          ov[0] = (T)((double)ov[0] + a1[0]);
-          ov[5] = (T)((double)ov[5] + a1[1]);
         } else {
           out[8] = -a1[0];
           out[9] = -a1[1];
-          ov[0] = (T)((double)ov[0] - a0[0]);
-          ov[5] = (T)((double)ov[5] - a0[1]);
         }
-        for (int k = 0; k < 6; k++) off[k] = ov[k];
+        if (!OWN) {
+          ov[0] = (T)(s0 ? (double)ov[0] + a1[0] : (double)ov[0] - a0[0]);
+          ov[5] = (T)(s0 ? (double)ov[5] + a1[1] : (double)ov[5] - a0[1]);
+          for (int k = 0; k < 6; k++) off[k] = ov[k];
+        }
       }
     }
   } else {
@@ -3383,6 +3397,8 @@ __global__ void __launch_bounds__(kBlock) k_scal_c(DMesh m, DParams P, const dou
   scal_c_finish<T>(m, P, o, c, acc, D, rhs_s, A, step_mode, dt, relax, rhs_ls, x0);
 }
 
+// k_scal_e with only its own side of the face's matrices: 2M-cell SA plate,
+// FP32, 1508 -> 1351 us (120 registers, four waves per SIMD)
 constexpr int kScalWaves = 1;
 
 template <typename T, bool SND>
@@ -3396,16 +3412,31 @@ __global__ void __launch_bounds__(64 * kScalWaves) k_scal_e(DMesh m, DParams P, 
                                                             T *__restrict__ x0) {
   constexpr int NS = 10;
   __shared__ double lds[64 * kScalWaves * NS];
+  __shared__ int toff[64 * kScalWaves];  // the entry's off-diagonal block, -1 without one
   double *slot = lds + NS * threadIdx.x;
   const EntryLane L = entry_lane<kScalWaves>(m, hw_blk());
   ScalOwn o;
+  toff[threadIdx.x] = L.e >= 0 ? m.cfl_tnoc[L.e] : -1;
   if (L.e >= 0) {
     o = scal_own(P, prim, grad, L.c);
     double t10[NS];
-    scal_c_entry<T, SND>(m, P, prim, grad, bfa, A, o, L.e, t10);
+    scal_c_entry<T, SND, true>(m, P, prim, grad, bfa, A, o, L.e, t10);
     for (int k = 0; k < NS; k++) slot[k] = t10[k];
   }
   __syncthreads();
+  if (A) {  // row 5 of the off-diagonal blocks, by the wavefront (see k_jac_e)
+    const int wb = threadIdx.x & ~63;
+    for (int it = 0; it < 6; it++) {
+      const int idx = it * 64 + (threadIdx.x & 63), en = idx / 6, k = idx - 6 * en;
+      const int tn = toff[wb + en];
+      if (tn < 0) continue;
+      const double *sj = lds + NS * (wb + en);
+      T v = (T)(0.0 - sj[2 + k]);
+      if (k == 0) v = (T)((double)v - sj[8]);
+      if (k == 5) v = (T)((double)v - sj[9]);
+      A[36 * (size_t)tn + 30 + k] = v;
+    }
+  }
   if (L.e < 0 || L.pos != 0) return;
   const int c = L.c;
   const int nent = m.cfl_i[c + 1] - m.cfl_i[c];

@@ -96,3 +96,17 @@ def test_block_solver_true_residual_at_the_stop(dims):
         it, st = joemi.block_bcgstab(*d, phi, zero_abs=0.0, zero_rel=1e-30, max_iter=60)
         # stalled by those guards, |t| near 1e-10: at the solution to ten times that
         assert st in (0, 1, 2) and np.max(np.abs(phi.numpy() - x)) <= 1e-9 * np.max(np.abs(x))
+
+
+# the scalar rows per entry (their off-diagonal entries written from the other
+# side of each face) against the per-cell form: the segregated SST rows and
+# row 5 of the coupled SA blocks (the latter in test_jacobian_... too)
+@pytest.mark.parametrize("n,frac", [(1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0)])
+def test_sst_rows_per_entry_equal_per_cell(n, frac):
+    print(f"sst rows n={n} frac={frac}", flush=True)
+    mesh, joe = box(n, frac, "HLLC", "sst")
+    names = ["ASCAL", "RHS_KINE", "RHS_OMEGA", "A"]
+    a = values(mesh, joe + "GPU_SCAL_KERNEL = ENTRY\n", names)
+    b = values(mesh, joe + "GPU_SCAL_KERNEL = CELL\n", names)
+    for k in names:
+        assert np.array_equal(a[k], b[k], equal_nan=True), k
