@@ -46,6 +46,12 @@ struct ZoneDev {
   double sval, sval2;
 };
 
+// a tile's first cell, halo cell, entry, LS coefficient and face evaluation,
+// and how many of each
+struct alignas(16) Tile {
+  int c0, nc, h0, nh, e0, ne, k0, nk, w0, nw, pad0, pad1;
+};
+
 struct DMesh {
   int ncv, nfa, nfa_b, nnz;
   const double *fgeo;     // [nfa][8]
@@ -67,6 +73,16 @@ struct DMesh {
   const int *wave_e0;     // [nwave+1] first entry of each 64-lane wavefront
   int nwave;
   const int *foc;         // [entries] entry offset of the cell's k-th face in faocv order (Spalart-Allmaras)
+  const double *gg;       // [entries][5] Green-Gauss: outward normal, distances of the face's centroid from cell and neighbour
+  // tiles of consecutive cells (build_tiles), their halo cells, each entry's
+  // neighbour as a row of the tile (its cells, then its halo; kNoRow on
+  // boundary faces) and the face evaluations
+  int ntile;
+  const Tile *tile;
+  const int *halo;
+  const unsigned short *lnb;
+  const int4 *eval;
+  const uint2 *tcell;  // [ncv] each tile's cells by entry count
   const int *cell_perm;   // [ncv] cell of each thread of the per-cell gradient, or null (thread t -> cell t)
 };
 
@@ -137,6 +153,17 @@ struct StepMail {
 namespace {
 
 constexpr int kBlock = 256;
+
+// A tile: at most kTileEval faces to evaluate (one per thread), kTileCells
+// cells, kTileRows cells and halo cells, kTileEnt entries. The rows in LDS
+// (208 bytes each in the flux kernel) let four blocks share a CU.
+constexpr int kTileEval = kBlock, kTileCells = 80, kTileRows = 188, kTileEnt = 448;
+// an evaluation: {face | side << 31 (DMesh::cfl's), neighbour cell or -(zone + 1),
+// the cell's row | the neighbour's << 16, the entry | the face's other entry in
+// the tile (or kNoEntry) << 16, counted from the tile's first}
+// a cell in DMesh::tcell: {cell of the tile | entries << 8 | first entry << 16,
+// first LS coefficient | internal entries << 16}
+constexpr unsigned kNoRow = 0xffff, kNoEntry = 0xffff;
 constexpr int kRedSlots = 8;  // partial-sum slots per block for fused reductions
 inline int nblk(long long n, int b = kBlock) { return (int)((n + b - 1) / b); }
 
@@ -361,6 +388,19 @@ __global__ void __launch_bounds__(kBlock) k_bc(DMesh m, DParams P, const double 
   d_bc(hw_blk(), m, P, prim, hook, bfa);
 }
 
+// the larger and the smaller of two values, the other one if one is NaN, in
+// one instruction each (fmax and fmin first quiet their arguments)
+__device__ __forceinline__ double max_num(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double min_num(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // smooth Barth-Jespersen factor of one face (UgpWithCv.h:913-925, BJ undefined)
 __device__ __forceinline__ double bj_face(double alfa, double phi, double phifa, double phiMax, double phiMin,
                                           double eps2) {
@@ -373,18 +413,29 @@ __device__ __forceinline__ double bj_face(double alfa, double phi, double phifa,
 // Gradients of u (vector), rho and p with boundary values, and their smooth
 // Barth-Jespersen limiters: calcCvVectorGrad / calcCvScalarGrad
 // (UgpWithCv.h:803-872), least squares (:1009-1083) or Green-Gauss
-// (:1091-1188), limiters (:881-1000). One thread per cell; the cell's sums
-// follow the reference's order (diagonal, nbocv neighbours, boundary faces).
+// (:1091-1188), limiters (:881-1000). The cell's sums follow the reference's
+// order (diagonal, nbocv neighbours, boundary faces).
+//
+// One thread per cell and field (rho, u, v, w, p; with VISC also the
+// enthalpy): the five or six neighbouring lanes of a cell read consecutive
+// values of each neighbour's row, the coefficient and offset of an entry is
+// one address for all of them, and each lane keeps only its own field's
+// gradient and bounds (44 registers; a thread holding all fields needed 120).
+// The batched server's form, and of meshes with duplicate neighbour pairs; a
+// solve of its own takes k_grad_t. 5.9k cells: 23 us with a thread per cell,
+// 10 so; 3.1M cells: 614 and 670, bound by the vector memory unit.
 // ---------------------------------------------------------------------------
 // enthalpy of a cell state (calcStateVariables: T = p / (rho R),
 // h = gamma R / (gamma - 1) T; UgpWithCvCompFlow.h:1680-1690)
-// entries of a cell whose loads the per-cell gradient issues together
-constexpr int kGradChunk = 4;
-
 __device__ __forceinline__ double enthalpy_of(const DParams &P, double rho, double p) {
   const double T = p / (rho * P.R);
   return P.gamma * P.R / (P.gamma - 1.0) * T;
 }
+
+// entries of a cell whose loads the gradient issues together
+constexpr int kGradChunk = 4;
+// threads per cell
+constexpr int grad_fields(bool visc) { return visc ? 6 : 5; }
 
 // With VISC the kernel also forms the enthalpy gradient and the velocity and
 // enthalpy gradients the viscous flux uses (calcViscousFluxNS,
@@ -394,241 +445,110 @@ template <bool LS, bool VISC>
 __device__ __forceinline__ void d_grad(const Blk &B, DMesh m, DParams P, const double *__restrict__ prim,
                                                  const double *__restrict__ bfa, double *__restrict__ grad,
                                                  double *__restrict__ gradv) {
-  const int t = xcd_block(B.id, B.n) * blockDim.x + threadIdx.x;
-  if (t >= m.ncv) return;
-  const int c = m.cell_perm ? m.cell_perm[t] : t;
+  constexpr int NF = grad_fields(VISC);
+  const unsigned t = (unsigned)xcd_block(B.id, B.n) * blockDim.x + threadIdx.x;
+  const int ct = (int)(t / NF), fld = (int)(t - (unsigned)NF * ct);  // 0 rho, 1-3 velocity, 4 p, 5 enthalpy
+  if (ct >= m.ncv) return;
+  const int c = m.cell_perm ? m.cell_perm[ct] : ct;
+  const bool enth = VISC && fld == 5;
+  const bool vel = fld >= 1 && fld <= 3;
   const double *pc = prim + 8 * (size_t)c;
-  const double rho = pc[0], u[3] = {pc[1], pc[2], pc[3]}, p = pc[4];
-  const double xcv[3] = {pc[5], pc[6], pc[7]};
-  double gr[3], gp[3], gu[3][3], gh[3] = {0.0, 0.0, 0.0};
-  double rmax = rho, rmin = rho, pmax = p, pmin = p;
-  double umax[3] = {u[0], u[1], u[2]}, umin[3] = {u[0], u[1], u[2]};
-  const double h = VISC ? enthalpy_of(P, rho, p) : 0.0;
-  double hmax = h, hmin = h;
+  const double phi = enth ? enthalpy_of(P, pc[0], pc[4]) : pc[enth ? 0 : fld];
+  double g[3], vmax = phi, vmin = phi;
   const int e0 = m.cfl_i[c], e1 = m.cfl_i[c + 1];
   int e_int = e0;  // end of the internal entries (they come first)
-  if (LS) {
-    const int noc_f = m.nbocv_i[c];
-    const double *l0 = m.lsg + 3 * (size_t)noc_f;
-    for (int j = 0; j < 3; j++) {
-      gr[j] = l0[j] * rho;
-      gp[j] = l0[j] * p;
-      if (VISC) gh[j] = l0[j] * h;
-    }
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j < 3; j++) gu[i][j] = l0[j] * u[i];
-    // internal entries (they come first) in chunks of kGradChunk: a chunk's
-    // entries, then its neighbour rows and coefficients, are loaded together
-    // (slots past the internal ones read the cell's own row, always valid)
-    // and added in entry order
-    const int noc_l = m.nbocv_i[c + 1] - 1;
-    bool open = true;
-    for (int eb = e0; open && eb < e1; eb += kGradChunk) {
-      int2 en[kGradChunk];
+  const int noc_f = LS ? m.nbocv_i[c] : 0, noc_l = LS ? m.nbocv_i[c + 1] - 1 : 0;
+  for (int j = 0; j < 3; j++) g[j] = LS ? m.lsg[3 * (size_t)noc_f + j] * phi : 0.0;
+  // internal entries in chunks of kGradChunk: a chunk's entries, then its
+  // neighbour values and coefficients, are loaded together (slots past the
+  // internal ones read the cell's own row, always valid) and added in entry
+  // order
+  bool open = true;
+  for (int eb = e0; open && eb < e1; eb += kGradChunk) {
+    int2 en[kGradChunk];
 #pragma unroll
-      for (int q = 0; q < kGradChunk; q++) en[q] = eb + q < e1 ? m.cfl[eb + q] : make_int2(0, -1);
-      double2 a[kGradChunk], b[kGradChunk];
-      double pv[kGradChunk], l[kGradChunk][3];
+    for (int q = 0; q < kGradChunk; q++) en[q] = eb + q < e1 ? m.cfl[eb + q] : make_int2(0, -1);
+    double v[kGradChunk], l[kGradChunk][3], ws[kGradChunk], wn[kGradChunk];
 #pragma unroll
-      for (int q = 0; q < kGradChunk; q++) {
-        const double *pn = prim + 8 * (size_t)(en[q].y >= 0 ? en[q].y : c);
-        a[q] = ld2(pn);
-        b[q] = ld2(pn + 2);
-        pv[q] = pn[4];
+    for (int q = 0; q < kGradChunk; q++) {
+      const double *pn = prim + 8 * (size_t)(en[q].y >= 0 ? en[q].y : c);
+      v[q] = enth ? pn[4] : pn[enth ? 4 : fld];
+      if (VISC && enth) v[q] = enthalpy_of(P, pn[0], v[q]);
+      if (LS) {
         const double *lq = m.lsg + 3 * (size_t)min(noc_f + 1 + (eb - e0) + q, noc_l);
-        l[q][0] = lq[0];
-        l[q][1] = lq[1];
-        l[q][2] = lq[2];
-      }
-#pragma unroll
-      for (int q = 0; q < kGradChunk; q++) {
-        open = open && en[q].y >= 0;
-        if (!open) break;
-        const double rn = a[q].x, un[3] = {a[q].y, b[q].x, b[q].y}, pnv = pv[q];
-        const double l_0 = l[q][0], l_1 = l[q][1], l_2 = l[q][2];
-        gr[0] += l_0 * rn; gr[1] += l_1 * rn; gr[2] += l_2 * rn;
-        gp[0] += l_0 * pnv; gp[1] += l_1 * pnv; gp[2] += l_2 * pnv;
-        if (VISC) {
-          const double hn = enthalpy_of(P, rn, pnv);
-          gh[0] += l_0 * hn; gh[1] += l_1 * hn; gh[2] += l_2 * hn;
-          hmax = Dev::mx(hmax, hn); hmin = Dev::mn(hmin, hn);
-        }
-        for (int i = 0; i < 3; i++) {
-          gu[i][0] += l_0 * un[i];
-          gu[i][1] += l_1 * un[i];
-          gu[i][2] += l_2 * un[i];
-          umax[i] = Dev::mx(umax[i], un[i]);
-          umin[i] = Dev::mn(umin[i], un[i]);
-        }
-        rmax = Dev::mx(rmax, rn); rmin = Dev::mn(rmin, rn);
-        pmax = Dev::mx(pmax, pnv); pmin = Dev::mn(pmin, pnv);
-        e_int = eb + q + 1;
-      }
-    }
-    for (int e = e0; e < e1; e++) {
-      int2 en = m.cfl[e];
-      if (en.y >= 0) continue;
-      int f = en.x & 0x7fffffff;
-      const double *bl = m.bfa_lsg + 3 * (size_t)f;
-      const double *bb = bfa + 8 * (size_t)f;
-      double b0 = bl[0], b1 = bl[1], b2 = bl[2];
-      double rb = bb[0], ub[3] = {bb[1], bb[2], bb[3]}, pb = bb[4];
-      for (int i = 0; i < 3; i++) {
-        gu[i][0] += b0 * ub[i];
-        gu[i][1] += b1 * ub[i];
-        gu[i][2] += b2 * ub[i];
-      }
-      gr[0] += b0 * rb; gr[1] += b1 * rb; gr[2] += b2 * rb;
-      gp[0] += b0 * pb; gp[1] += b1 * pb; gp[2] += b2 * pb;
-      if (VISC) {
-        const double hb = bb[6];
-        gh[0] += b0 * hb; gh[1] += b1 * hb; gh[2] += b2 * hb;
-      }
-    }
-  } else {
-    for (int j = 0; j < 3; j++) {
-      gr[j] = 0.0;
-      gp[j] = 0.0;
-      gu[0][j] = gu[1][j] = gu[2][j] = 0.0;
-    }
-    for (int e = e0; e < e1; e++) {
-      int2 en = m.cfl[e];
-      int f = en.x & 0x7fffffff;
-      const double *fn = m.fnorm + 3 * (size_t)f;
-      double n[3] = {fn[0], fn[1], fn[2]};
-      if (en.y >= 0) {
-        const double *pn = prim + 8 * (size_t)en.y;
-        double rn = pn[0], un[3] = {pn[1], pn[2], pn[3]}, pnv = pn[4];
-        // distance weights (GG_WITH_DIST, UgpWithCv.h:37, :1104-1110)
-        const double *xf = m.fgeo + 8 * (size_t)f + 4;
-        double ds[3], dn[3];
-        for (int j = 0; j < 3; j++) {
-          ds[j] = xf[j] - xcv[j];
-          dn[j] = xf[j] - pn[5 + j];
-        }
-        const bool s0 = (en.x >= 0);  // side 0: this cell is icv0
-        const double wself = sqrt(dot3(ds, ds)), wnb = sqrt(dot3(dn, dn));
-        const double w0 = s0 ? wself : wnb, w1 = s0 ? wnb : wself;
-        double fr = s0 ? (w1 * rho + w0 * rn) / (w0 + w1) : (w1 * rn + w0 * rho) / (w0 + w1);
-        double fp = s0 ? (w1 * p + w0 * pnv) / (w0 + w1) : (w1 * pnv + w0 * p) / (w0 + w1);
-        for (int j = 0; j < 3; j++) {
-          if (s0) {
-            gr[j] += fr * n[j];
-            gp[j] += fp * n[j];
-          } else {
-            gr[j] -= fr * n[j];
-            gp[j] -= fp * n[j];
-          }
-        }
-        if (VISC) {
-          const double hn = enthalpy_of(P, rn, pnv);
-          const double fh = s0 ? (w1 * h + w0 * hn) / (w0 + w1) : (w1 * hn + w0 * h) / (w0 + w1);
-          for (int j = 0; j < 3; j++) {
-            if (s0)
-              gh[j] += fh * n[j];
-            else
-              gh[j] -= fh * n[j];
-          }
-          hmax = Dev::mx(hmax, hn); hmin = Dev::mn(hmin, hn);
-        }
-        for (int i = 0; i < 3; i++) {
-          double fu = s0 ? (w1 * u[i] + w0 * un[i]) / (w0 + w1) : (w1 * un[i] + w0 * u[i]) / (w0 + w1);
-          for (int j = 0; j < 3; j++) {
-            if (s0)
-              gu[i][j] += fu * n[j];
-            else
-              gu[i][j] -= fu * n[j];
-          }
-          umax[i] = Dev::mx(umax[i], un[i]);
-          umin[i] = Dev::mn(umin[i], un[i]);
-        }
-        rmax = Dev::mx(rmax, rn); rmin = Dev::mn(rmin, rn);
-        pmax = Dev::mx(pmax, pnv); pmin = Dev::mn(pmin, pnv);
-        e_int = e + 1;
+        for (int j = 0; j < 3; j++) l[q][j] = lq[j];
       } else {
-        const double *bb = bfa + 8 * (size_t)f;
-        double rb = bb[0], ub[3] = {bb[1], bb[2], bb[3]}, pb = bb[4];
-        for (int j = 0; j < 3; j++) {
-          gr[j] += rb * n[j];
-          gp[j] += pb * n[j];
-          if (VISC) gh[j] += bb[6] * n[j];
-        }
-        for (int i = 0; i < 3; i++)
-          for (int j = 0; j < 3; j++) gu[i][j] += ub[i] * n[j];
+        const double *gq = m.gg + 5 * (size_t)min(eb + q, e1 - 1);
+        for (int j = 0; j < 3; j++) l[q][j] = gq[j];
+        ws[q] = gq[3];
+        wn[q] = gq[4];
       }
     }
-    const double vol = m.vol[c];
-    for (int j = 0; j < 3; j++) {
-      gr[j] /= vol;
-      gp[j] /= vol;
-      if (VISC) gh[j] /= vol;
+#pragma unroll
+    for (int q = 0; q < kGradChunk; q++) {
+      open = open && en[q].y >= 0;
+      if (!open) break;
+      const double vn = v[q];
+      if (LS) {
+        for (int j = 0; j < 3; j++) g[j] += l[q][j] * vn;
+      } else {
+        // distance weights (GG_WITH_DIST, UgpWithCv.h:37, :1104-1110): the
+        // reference's (w1 phi0 + w0 phi1) / (w0 + w1) from either side
+        const double fv = (wn[q] * phi + ws[q] * vn) / (ws[q] + wn[q]);
+        for (int j = 0; j < 3; j++) g[j] += fv * l[q][j];
+      }
+      vmax = Dev::mx(vmax, vn);
+      vmin = Dev::mn(vmin, vn);
+      e_int = eb + q + 1;
     }
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j < 3; j++) gu[i][j] /= vol;
+  }
+  for (int e = e_int; e < e1; e++) {  // boundary entries
+    const int f = m.cfl[e].x & 0x7fffffff;
+    const double *bl = (LS ? m.bfa_lsg : m.fnorm) + 3 * (size_t)f;
+    const double vb = bfa[8 * (size_t)f + (enth ? 6 : fld)];
+    for (int j = 0; j < 3; j++) g[j] += bl[j] * vb;
+  }
+  if (!LS) {
+    const double vol = m.vol[c];
+    for (int j = 0; j < 3; j++) g[j] /= vol;
   }
 
-  double au[3] = {1.0, 1.0, 1.0}, ar = 1.0, ap = 1.0, ah = 1.0;
-  if (P.limiter) {
-    const double sos = sqrt(P.gamma * p / rho);
-    double e2u = P.eps * sos;
-    e2u = e2u * e2u;
-    double e2r = Dev::mx(P.eps * fabs(rho), 1.0e-8);
-    e2r = e2r * e2r;
-    double e2p = Dev::mx(P.eps * fabs(p), 1.0e-8);
-    e2p = e2p * e2p;
-    bool lu[3] = {(umax[0] - umin[0]) > 1.0e-8, (umax[1] - umin[1]) > 1.0e-8, (umax[2] - umin[2]) > 1.0e-8};
-    bool lr = (rmax - rmin) > 1.0e-12, lp = (pmax - pmin) > 1.0e-12;
-    // face offsets in chunks loaded together (slots past e_int repeat the
-    // last entry and are not applied)
-    for (int eb = e0; eb < e_int; eb += kGradChunk) {
-      double r0[kGradChunk][3];
+  double al = 1.0;
+  if (P.limiter && (!enth || P.visc_limiter)) {
+    // reference values: the speed of sound for the velocity, the field itself
+    // for the others (enthalpy: JoeWithModels.cpp:3619)
+    double e2 = vel ? P.eps * sqrt(P.gamma * pc[4] / pc[0]) : Dev::mx(P.eps * fabs(phi), 1.0e-8);
+    e2 = e2 * e2;
+    if ((vmax - vmin) > (vel ? 1.0e-8 : 1.0e-12)) {
+      // face offsets in chunks loaded together (slots past e_int repeat the
+      // last entry and are not applied)
+      for (int eb = e0; eb < e_int; eb += kGradChunk) {
+        double r0[kGradChunk][3];
 #pragma unroll
-      for (int q = 0; q < kGradChunk; q++) {
-        const double *rr = m.cfl_r0 + 3 * (size_t)min(eb + q, e_int - 1);
-        r0[q][0] = rr[0];
-        r0[q][1] = rr[1];
-        r0[q][2] = rr[2];
-      }
-#pragma unroll
-      for (int q = 0; q < kGradChunk; q++) {
-        if (eb + q >= e_int) break;
-        for (int i = 0; i < 3; i++)
-          if (lu[i]) au[i] = bj_face(au[i], u[i], u[i] + dot3(r0[q], gu[i]), umax[i], umin[i], e2u);
-        if (lr) ar = bj_face(ar, rho, rho + dot3(r0[q], gr), rmax, rmin, e2r);
-        if (lp) ap = bj_face(ap, p, p + dot3(r0[q], gp), pmax, pmin, e2p);
-      }
-    }
-    for (int i = 0; i < 3; i++)
-      if (!lu[i]) au[i] = 0.0;
-    if (!lr) ar = 0.0;
-    if (!lp) ap = 0.0;
-    if (VISC && P.visc_limiter) {  // enthalpy, reference value h (JoeWithModels.cpp:3619)
-      double e2h = Dev::mx(P.eps * fabs(h), 1.0e-8);
-      e2h = e2h * e2h;
-      if ((hmax - hmin) > 1.0e-12) {
-        for (int e = e0; e < e_int; e++) {
-          const double *rr = m.cfl_r0 + 3 * (size_t)e;
-          double r0[3] = {rr[0], rr[1], rr[2]};
-          ah = bj_face(ah, h, h + dot3(r0, gh), hmax, hmin, e2h);
+        for (int q = 0; q < kGradChunk; q++) {
+          const double *rr = m.cfl_r0 + 3 * (size_t)min(eb + q, e_int - 1);
+          for (int j = 0; j < 3; j++) r0[q][j] = rr[j];
         }
-      } else {
-        ah = 0.0;
+#pragma unroll
+        for (int q = 0; q < kGradChunk; q++) {
+          if (eb + q >= e_int) break;
+          al = bj_face(al, phi, phi + dot3(r0[q], g), vmax, vmin, e2);
+        }
       }
+    } else {
+      al = 0.0;
     }
   }
-  if (VISC) {
+  if (VISC && (enth || vel)) {
     const bool lim = P.limiter && P.visc_limiter;
-    double *v = gradv + 12 * (size_t)c;
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j < 3; j++) v[3 * i + j] = lim ? gu[i][j] * au[i] : gu[i][j];
-    for (int j = 0; j < 3; j++) v[9 + j] = lim ? gh[j] * ah : gh[j];
+    double *v = gradv + 12 * (size_t)c + (enth ? 9 : 3 * (fld - 1));
+    for (int j = 0; j < 3; j++) v[j] = lim ? g[j] * al : g[j];
   }
+  if (enth) return;
   double *o = grad + 16 * (size_t)c;
-  o[0] = gr[0] * ar; o[1] = gr[1] * ar; o[2] = gr[2] * ar;
-  o[3] = gp[0] * ap; o[4] = gp[1] * ap; o[5] = gp[2] * ap;
-  for (int i = 0; i < 3; i++)
-    for (int j = 0; j < 3; j++) o[6 + 3 * i + j] = gu[i][j] * au[i];
-  o[15] = ar;
+  double *og = o + (fld == 0 ? 0 : (fld == 4 ? 3 : 3 + 3 * fld));
+  for (int j = 0; j < 3; j++) og[j] = g[j] * al;
+  if (fld == 0) o[15] = al;
 }
 
 template <bool LS, bool VISC>
@@ -636,6 +556,170 @@ __global__ void __launch_bounds__(kBlock) k_grad(DMesh m, DParams P, const doubl
                                                  const double *__restrict__ bfa, double *__restrict__ grad,
                                                  double *__restrict__ gradv) {
   d_grad<LS, VISC>(hw_blk(), m, P, prim, bfa, grad, gradv);
+}
+
+// The same gradient by tiles of cells (DMesh): the tile's and its halo's five
+// fields, the coefficients and then the face offsets of its entries are
+// copied to LDS, each cache line once and by consecutive lanes, and the
+// threads, again one per cell and field, work from there. k_grad's lanes ask
+// the vector memory unit for about seven lines per entry, which is what
+// bounds it on a mesh that fills the card. The cells of a tile are taken by
+// entry count, since a wavefront loops as long as its longest cell: 530 us
+// without, 414 with. 3.1M-cell split box (k_grad with a thread per cell 614
+// us): 414 us, 1.48 GB, 3.6 TB/s; 223k cells 52 -> 36; Green-Gauss, 876k
+// cells, 230 -> 181. Bound now by HBM and latency: VALU 55 % busy.
+constexpr int kGradRow = 6;  // doubles per row: rho, u, v, w, p, enthalpy
+
+template <bool LS, bool VISC>
+__global__ void __launch_bounds__(kBlock) k_grad_t(DMesh m, DParams P, const double *__restrict__ prim,
+                                                   const double *__restrict__ bfa, double *__restrict__ grad,
+                                                   double *__restrict__ gradv) {
+  constexpr int NF = grad_fields(VISC), NC = LS ? 3 : 5;  // doubles of a coefficient
+  constexpr int kCoef = LS ? 3 * (kTileEnt + kTileCells) : 5 * kTileEnt, kOut = (VISC ? 28 : 16) * kTileCells;
+  constexpr int NT = (kTileCells * NF + kBlock - 1) / kBlock;  // cell-field pairs per thread
+  __shared__ __align__(16) double rows[kGradRow * kTileRows];
+  __shared__ __align__(16) double buf[kCoef > kOut ? kCoef : kOut];  // coefficients, then offsets, then results
+  __shared__ unsigned short lnb[kTileEnt];
+  const int tid = threadIdx.x;
+  const Tile T = m.tile[xcd_block(blockIdx.x, gridDim.x)];
+  const int c0 = T.c0, nc = T.nc, h0 = T.h0, nr = nc + T.nh, e0 = T.e0, ne = T.ne;
+  const int k0 = LS ? T.k0 : e0, nk = LS ? T.nk : ne;
+  uint2 tc[NT];  // each pair's cell
+#pragma unroll
+  for (int i = 0; i < NT; i++) tc[i] = m.tcell[c0 + min((i * kBlock + tid) / NF, nc - 1)];
+  // the face offsets, wanted later, are on their way while the gradient is formed
+  constexpr int NR0 = (3 * kTileEnt + kBlock - 1) / kBlock;
+  double r0[NR0];
+  {
+    double2 *r2 = reinterpret_cast<double2 *>(rows);
+    for (int k = tid; k < 3 * nr; k += kBlock) {
+      const int r = k / 3;
+      const int c = r < nc ? c0 + r : m.halo[h0 + r - nc];
+      r2[k] = ld2(prim + 8 * (size_t)c + 2 * (k - 3 * r));
+    }
+    const double *coef = (LS ? m.lsg : m.gg) + NC * (size_t)k0;
+    for (int k = tid; k < NC * nk; k += kBlock) buf[k] = coef[k];
+    for (int k = tid; k < ne; k += kBlock) lnb[k] = m.lnb[e0 + k];
+#pragma unroll
+    for (int i = 0; i < NR0; i++) r0[i] = P.limiter ? m.cfl_r0[3 * (size_t)e0 + min(i * kBlock + tid, 3 * ne - 1)] : 0.0;
+  }
+  __syncthreads();
+  if (VISC) {
+    for (int r = tid; r < nr; r += kBlock) rows[kGradRow * r + 5] = enthalpy_of(P, rows[kGradRow * r], rows[kGradRow * r + 4]);
+    __syncthreads();
+  }
+  double phi[NT], vmax[NT], vmin[NT], g[NT][3], al[NT];
+#pragma unroll
+  for (int i = 0; i < NT; i++) {
+    const int t = i * kBlock + tid, fld = t % NF, cl = tc[i].x & 0xff;
+    if (t >= NF * nc) continue;
+    const bool enth = VISC && fld == 5;
+    const int c = c0 + cl, ks = tc[i].x >> 16, ki = ks + (tc[i].y >> 16), ke = ks + (tc[i].x >> 8 & 0xff);
+    const double ph = rows[kGradRow * cl + fld];
+    // LS: the cell's coefficients start with its own, then one per entry
+    const double *l = buf + (LS ? 3 * (tc[i].y & 0xffff) : 5 * ks);
+    for (int j = 0; j < 3; j++) g[i][j] = LS ? l[j] * ph : 0.0;
+    if (LS) l += 3;
+    double hi = ph, lo = ph;
+    for (int k = ks; k < ki; k++) {
+      const double vn = rows[kGradRow * lnb[k] + fld];
+      if (LS) {
+        for (int j = 0; j < 3; j++) g[i][j] += l[j] * vn;
+      } else {
+        const double fv = (l[4] * ph + l[3] * vn) / (l[3] + l[4]);
+        for (int j = 0; j < 3; j++) g[i][j] += fv * l[j];
+      }
+      l += NC;
+      hi = max_num(hi, vn);
+      lo = min_num(lo, vn);
+    }
+    if (ph != ph) hi = lo = ph;  // the reference's bounds of a NaN stay NaN
+    for (int k = ki; k < ke; k++) {  // boundary entries
+      const int f = m.cfl[e0 + k].x & 0x7fffffff;
+      const double *bl = (LS ? m.bfa_lsg : m.fnorm) + 3 * (size_t)f;
+      const double vb = bfa[8 * (size_t)f + (enth ? 6 : fld)];
+      for (int j = 0; j < 3; j++) g[i][j] += bl[j] * vb;
+    }
+    if (!LS) {
+      const double vol = m.vol[c];
+      for (int j = 0; j < 3; j++) g[i][j] /= vol;
+    }
+    phi[i] = ph;
+    vmax[i] = hi;
+    vmin[i] = lo;
+    al[i] = 1.0;
+  }
+  __syncthreads();
+  if (P.limiter) {  // as d_grad
+#pragma unroll
+    for (int i = 0; i < NR0; i++)
+      if (i * kBlock + tid < 3 * ne) buf[i * kBlock + tid] = r0[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+      const int t = i * kBlock + tid, fld = t % NF, cl = tc[i].x & 0xff, ks = tc[i].x >> 16;
+      if (t >= NF * nc) continue;
+      const bool enth = VISC && fld == 5, vel = fld >= 1 && fld <= 3;
+      if (enth && !P.visc_limiter) continue;
+      const double *pc = rows + kGradRow * cl;
+      double e2 = vel ? P.eps * sqrt(P.gamma * pc[4] / pc[0]) : Dev::mx(P.eps * fabs(phi[i]), 1.0e-8);
+      e2 = e2 * e2;
+      if ((vmax[i] - vmin[i]) > (vel ? 1.0e-8 : 1.0e-12)) {
+        const int ki = ks + (tc[i].y >> 16);
+        for (int k = ks; k < ki; k++)
+          al[i] = bj_face(al[i], phi[i], phi[i] + dot3(buf + 3 * k, g[i]), vmax[i], vmin[i], e2);
+      } else {
+        al[i] = 0.0;
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < NT; i++) {
+    const int t = i * kBlock + tid, fld = t % NF, cl = tc[i].x & 0xff;
+    if (t >= NF * nc) continue;
+    const bool enth = VISC && fld == 5, vel = fld >= 1 && fld <= 3;
+    if (VISC && (enth || vel)) {
+      const bool lim = P.limiter && P.visc_limiter;
+      double *v = buf + 16 * kTileCells + 12 * cl + (enth ? 9 : 3 * (fld - 1));
+      for (int j = 0; j < 3; j++) v[j] = lim ? g[i][j] * al[i] : g[i][j];
+    }
+    if (enth) continue;
+    double *o = buf + 16 * cl, *og = o + (fld == 0 ? 0 : (fld == 4 ? 3 : 3 + 3 * fld));
+    for (int j = 0; j < 3; j++) og[j] = g[i][j] * al[i];
+    if (fld == 0) o[15] = al[i];
+  }
+  __syncthreads();
+  const double2 *o2 = reinterpret_cast<const double2 *>(buf);
+  double2 *g2 = reinterpret_cast<double2 *>(grad + 16 * (size_t)c0);
+  for (int k = tid; k < 8 * nc; k += kBlock) g2[k] = o2[k];
+  if (VISC) {
+    double2 *v2 = reinterpret_cast<double2 *>(gradv + 12 * (size_t)c0);
+    for (int k = tid; k < 6 * nc; k += kBlock) v2[k] = o2[8 * kTileCells + k];
+  }
+}
+
+// Green-Gauss coefficients of every entry (set-up: geometry only)
+__global__ void __launch_bounds__(kBlock) k_gg_coeff(DMesh m, const double *__restrict__ prim,
+                                                     double *__restrict__ gg) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= m.ncv) return;
+  const double *pc = prim + 8 * (size_t)c;
+  for (int e = m.cfl_i[c]; e < m.cfl_i[c + 1]; e++) {
+    const int2 en = m.cfl[e];
+    const int f = en.x & 0x7fffffff;
+    const double *pn = prim + 8 * (size_t)(en.y >= 0 ? en.y : c);
+    const double *xf = m.fgeo + 8 * (size_t)f + 4, *fn = m.fnorm + 3 * (size_t)f;
+    double ds[3], dn[3];
+    for (int j = 0; j < 3; j++) {
+      ds[j] = xf[j] - pc[5 + j];
+      dn[j] = xf[j] - pn[5 + j];
+    }
+    double *o = gg + 5 * (size_t)e;
+    for (int j = 0; j < 3; j++) o[j] = en.x >= 0 ? fn[j] : -fn[j];
+    o[3] = sqrt(dot3(ds, ds));
+    o[4] = sqrt(dot3(dn, dn));
+  }
 }
 
 // Entry-parallel form of k_grad: one lane per cell-face entry, each 64-lane
@@ -3710,6 +3794,199 @@ __global__ void __launch_bounds__(kBlock) k_flux(DMesh m, DParams P, const doubl
   block_partials<1>(v, partials, sh, kMin);
 }
 
+// The inviscid residual by tiles of cells (DMesh): each face between two of a
+// tile's cells is evaluated once, by one thread, and its flux left in the LDS
+// slots of both entries; faces that leave the tile are evaluated from the
+// entry inside (about 0.65 evaluations per entry). The states and gradients
+// of the tile's cells and its halo come to LDS by full cache lines. The
+// cells' sums are k_flux_e's, in entry order, so the bits are the same.
+// k_flux_e evaluates every face twice and its lanes ask the vector memory
+// unit for about twenty lines per entry (75 % busy). Every load that needs
+// only the tile's header, or one more index, is issued first: with each
+// index fetched where it was used the chain of loads made a tile live 18 us
+// and the kernel no faster (705 us). 3.1M-cell split box, HLLC: k_flux_e 617
+// us, this 484 to 500; Roe, 223k cells, 47 -> 37; AUSM, 876k cells, 188 ->
+// 137.
+constexpr int kFluxRow = 26;  // doubles per row: prim 8, gradients 15, rho u (the tile's cells) 3
+
+template <int SCHEME, bool SND>
+__global__ void __launch_bounds__(kBlock) k_flux_t(DMesh m, DParams P, const double *__restrict__ prim,
+                                                   const double *__restrict__ grad, const double *__restrict__ bfa,
+                                                   const double *__restrict__ q, double *__restrict__ rhs,
+                                                   int *__restrict__ nfirst, DtArgs dta, double *__restrict__ dt,
+                                                   double *__restrict__ partials) {
+  constexpr int NS = 6;  // slot: the flux signed for the cell 5, wave speed
+  static_assert(kFluxRow * kTileRows >= NS * kTileEnt, "LDS shared in turn");
+  __shared__ __align__(16) double lds[kFluxRow * kTileRows];  // cell rows, then slots
+  __shared__ double snd[kTileCells], sh[16];
+  const int tid = threadIdx.x;
+  const Tile T = m.tile[xcd_block(blockIdx.x, gridDim.x)];
+  const int c0 = T.c0, nc = T.nc, nr = nc + T.nh;
+  const bool has = tid < T.nw;
+  const double gam = P.gamma;
+  // every load that needs only the tile's header or one more index is issued
+  // before the first is waited for
+  const int4 ev = has ? m.eval[T.w0 + tid] : make_int4(0, 0, 0, 0);
+  constexpr int NP = SND ? 12 : 4, NQ = (NP * kTileRows + kBlock - 1) / kBlock;
+  double2 v[NQ];
+  int rc[NQ], rr[NQ], pp[NQ];  // piece pp of row rr, cell rc: consecutive threads take consecutive pieces
+#pragma unroll
+  for (int i = 0; i < NQ; i++) {
+    rr[i] = i == 0 ? tid / NP : rr[i - (i > 0)] + kBlock / NP;
+    pp[i] = i == 0 ? tid % NP : pp[i - (i > 0)] + kBlock % NP;
+    if (pp[i] >= NP) {
+      pp[i] -= NP;
+      rr[i]++;
+    }
+    const int r = min(rr[i], nr - 1);
+    rc[i] = r < nc ? c0 + r : m.halo[T.h0 + r - nc];
+  }
+  const int cr = tid < nc ? c0 + tid : c0;  // this thread's cell of the last part
+  const int ks = m.cfl_i[cr], nent = m.cfl_i[cr + 1] - ks;
+  const double vol = m.vol[cr];
+  const double2 cp0 = ld2(prim + 8 * (size_t)cr), cp1 = ld2(prim + 8 * (size_t)cr + 2);
+  const double cpp = prim[8 * (size_t)cr + 4];
+  const double pc[4] = {cp0.x, cp0.y, cp1.x, cp1.y};
+  const int qi = min(tid / nc, 2), qr = min(tid - nc * qi, nc - 1);
+  const double ruv = q[(size_t)(1 + qi) * m.ncv + c0 + qr];
+  const int f = ev.x & 0x7fffffff, own = ev.z & 0xffff, nb = (unsigned)ev.z >> 16;
+  const unsigned el = ev.w & 0xffff, ep = (unsigned)ev.w >> 16;
+  const int2 en = make_int2(ev.x, ev.y);
+  double n[3], area, xfa[3];
+  {
+    const double *geo = m.fgeo + 8 * (size_t)f;
+    const double2 a = ld2(geo), b = ld2(geo + 2), cc = ld2(geo + 4);
+    n[0] = a.x; n[1] = a.y; n[2] = b.x; area = b.y;
+    xfa[0] = cc.x; xfa[1] = cc.y; xfa[2] = geo[6];
+  }
+#pragma unroll
+  for (int i = 0; i < NQ; i++) {
+    const int p = pp[i];
+    v[i] = p < 4 ? ld2(prim + 8 * (size_t)rc[i] + 2 * p) : ld2(grad + 16 * (size_t)rc[i] + 2 * (p - 4));
+  }
+#pragma unroll
+  for (int i = 0; i < NQ; i++) {
+    if (rr[i] >= nr) continue;
+    double *o = lds + kFluxRow * rr[i] + 2 * pp[i];
+    if (pp[i] < 11) *reinterpret_cast<double2 *>(o) = v[i];
+    else o[0] = v[i].x;
+  }
+  if (tid < 3 * nc) lds[kFluxRow * qr + 23 + qi] = ruv;
+  if (tid < nc) snd[tid] = sqrt(gam * cpp / pc[0]);
+  __syncthreads();
+  double F[5], lam = 0.0, lamp = 0.0;
+  bool s0 = true;
+  if (has) {
+    Side so, sn, fl, fr;
+    int low = 0;
+    double hl = 0.0, hr = 0.0;  // side enthalpies of the coupled flux
+    bool symm_analytic = false, reflect = false;
+    const double *bb = bfa + 8 * (size_t)(en.y >= 0 ? 0 : f);
+    if (en.y < 0) {
+      const ZoneDev &z = m.zones[-en.y - 1];
+      // the coupled loop treats walls as symmetry faces and NEUMANN faces
+      // with the boundary state on both sides (JoeWithModels.cpp:5150-5470)
+      reflect = z.bc == kBcSymmetry || z.bc == kBcWall || (SCHEME == kHllcC && z.bc == kBcNeumann);
+      if (reflect)
+        symm_analytic = SCHEME == kHllcC ? (z.bc != kBcNeumann && P.symm_bc == kSymmAnalytical)
+                                         : (z.bc == kBcSymmetry && P.symm_bc == kSymmAnalytical);
+    }
+    // one cell's row at a time: its state at the face and its wave speed
+    auto side = [&](int row, Side &s, double &lambda, bool in_tile) {
+      double w[kFluxRow];
+#pragma unroll
+      for (int k = 0; k < kFluxRow; k += 2) {
+        const double2 a = ld2(lds + kFluxRow * row + k);
+        w[k] = a.x;
+        w[k + 1] = a.y;
+      }
+      if (in_tile) lambda = (fabs(dot3(w + 23, n) / w[0]) + snd[row]) * area;
+      if (SND) return reconstruct(s, w, w + 8, xfa);
+      s.rho = w[0]; s.u[0] = w[1]; s.u[1] = w[2]; s.u[2] = w[3]; s.p = w[4];
+      return true;
+    };
+    if (!side(own, so, lam, true) && !reflect) low++;
+    if (en.y >= 0) {
+      s0 = en.x >= 0;
+      __builtin_amdgcn_sched_barrier(0);
+      if (!side(nb, sn, lamp, ep != kNoEntry) && ep != kNoEntry) low++;
+    } else {
+      sn.rho = bb[0]; sn.u[0] = bb[1]; sn.u[1] = bb[2]; sn.u[2] = bb[3]; sn.p = bb[4];
+      if (reflect) so = sn;
+    }
+    fl = s0 ? so : sn;
+    fr = s0 ? sn : so;
+    if (SCHEME == kHllcC) {  // calcThermoProp_p after reconstruction, or the cell's (JoeWithModels.cpp:4920-4928)
+      if (en.y < 0) hr = bb[6];
+      else hr = enthalpy_of(P, fr.rho, fr.p);
+      if (reflect) hl = bb[6];
+      else hl = enthalpy_of(P, fl.rho, fl.p);
+      flux_hllc_coupled(F, fl.rho, fl.u, fl.p, hl, fr.rho, fr.u, fr.p, hr, gam, area, n);
+    } else {
+      face_flux(SCHEME, F, fl, fr, gam, area, n);
+    }
+    if (symm_analytic) {  // the ONLY_PRESSURE flux
+      F[0] = 0.0;
+      for (int i = 0; i < 3; i++) F[1 + i] = fr.p * n[i] * area;
+      F[4] = 0.0;
+    }
+    if (P.fdump && en.x >= 0)
+      for (int k = 0; k < 5; k++) P.fdump[5 * (size_t)f + k] = F[k];
+    if (low) atomicAdd(nfirst, low);
+  }
+  __syncthreads();  // every row has been read
+  if (has) {
+    double *slot = lds + NS * el;
+    for (int k = 0; k < 5; k++) slot[k] = s0 ? -F[k] : F[k];
+    slot[5] = lam;
+    if (ep != kNoEntry) {  // the evaluation's own entry is the face's first side
+      double *sp = lds + NS * ep;
+      for (int k = 0; k < 5; k++) sp[k] = F[k];
+      sp[5] = lamp;
+    }
+  }
+  __syncthreads();
+  double dtc = 1.0e20;
+  if (tid < nc) {  // as k_flux_e's owner lanes
+    const int c = c0 + tid;
+    const double *slot = lds + NS * (ks - T.e0);
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    double lambdaMax = 0.0;
+    for (int j = 0; j < nent; j++) {
+      const double *s = slot + NS * j;
+      for (int k = 0; k < 5; k++) acc[k] += s[k];
+      lambdaMax = Dev::mx(lambdaMax, s[5]);
+    }
+    if (P.gravity_on) {  // sourceHook (JoeWithModels.h:111-129)
+      const double ru[3] = {q[m.ncv + c], q[2 * m.ncv + c], q[3 * m.ncv + c]};
+      acc[1] += vol * pc[0] * P.g[0];
+      acc[2] += vol * pc[0] * P.g[1];
+      acc[3] += vol * pc[0] * P.g[2];
+      acc[4] += vol * (P.g[0] * ru[0] + P.g[1] * ru[1] + P.g[2] * ru[2]);
+    } else {
+      acc[1] += 0.0;
+      acc[2] += 0.0;
+      acc[3] += 0.0;
+      bool allneg = signbit(pc[1]) && signbit(pc[2]) && signbit(pc[3]);
+      acc[4] += allneg ? -0.0 : 0.0;
+    }
+    for (int k = 0; k < 5; k++) rhs[(size_t)k * m.ncv + c] = acc[k];
+    const double cflv = dta.cfl_dev ? *dta.cfl_dev : dta.cfl;
+    if (dta.mode == 2) {
+      dtc = dta.dt_fixed;
+    } else if (dta.sum) {  // SUM_BASED (UgpWithCvCompFlow.cpp:62-99): sums in faocv order
+      double lc = 0.0;
+      for (int k = 0; k < nent; k++) lc += slot[NS * m.foc[ks + k] + 5];
+      dtc = Dev::mn(cflv * vol / lc, 1.0e20);
+    } else {
+      dtc = cflv * vol / lambdaMax;
+    }
+    dt[c] = dtc;
+  }
+  double dts[1] = {dtc};
+  block_partials<1>(dts, partials, sh, kMin, hw_blk());
+}
+
 // Entry-parallel form of k_flux: one lane per cell-face entry computes that
 // face's flux (signed for this cell) and the face's wave-speed bound; the
 // cell's owner lane adds the terms from LDS in entry order (the reference's
@@ -5369,6 +5646,18 @@ __global__ void __launch_bounds__(kBlock) k_wall_dist(int ncv, const double *__r
 }
 
 
+// the tiles' face evaluations from {entry | other entry << 16} (set-up)
+__global__ void __launch_bounds__(kBlock) k_tile_eval(DMesh m, const unsigned *__restrict__ packed,
+                                                      int4 *__restrict__ eval) {
+  const Tile T = m.tile[blockIdx.x];
+  for (int k = threadIdx.x; k < T.nw; k += blockDim.x) {
+    const unsigned w = packed[T.w0 + k];
+    const int e = T.e0 + (w & 0xffff), own = m.ecp[e].x - T.c0;
+    const int2 en = m.cfl[e];
+    eval[T.w0 + k] = make_int4(en.x, en.y, own | (en.y >= 0 ? (int)m.lnb[e] : own) << 16, (int)w);
+  }
+}
+
 // for every cell-face entry the block of its cell's column in the
 // neighbour's row (set-up; the rows are symmetric in their pattern)
 __global__ void __launch_bounds__(kBlock) k_tnoc(int ncv, const int *__restrict__ cfl_i, const int2 *__restrict__ cfl,
@@ -5795,7 +6084,19 @@ struct Ctx::Impl {
   DBuf<double> gradv;  // [ncv][12] velocity and enthalpy gradients of the viscous flux
   DBuf<int2> fcell;    // [nfa_i] device cells (icv0, icv1) of each internal face (face form of the flux, k_face_visc)
   DBuf<double> muf;    // [nfa][2] the faces' viscosities (k_face_visc)
+  DBuf<double> gg;     // [entries][5] Green-Gauss coefficients
+  int nent = 0;        // cell-face entries
+  // tiles of the gradient and inviscid flux kernels (DMesh)
+  int ntile = 0;
+  DBuf<char> tiles;
+  const unsigned *eval_packed = nullptr;
   DBuf<double> fflux;  // [nfa_i][5] face fluxes of the face form
+  // the tile forms (build_tiles) of the gradient and the inviscid flux
+  // (a duplicate neighbour pair has fewer coefficients than entries)
+  bool grad_tiled() const {
+    return par.grad_kernel == kResidCell && !par.grad_thread_sorted && !dup_blocks;
+  }
+  bool flux_tiled() const { return par.flux_kernel == kResidEntry && !dp.visc; }
   bool face_form() const { return par.flux_kernel == kResidFace && !dp.visc; }
   DBuf<int> counters;  // [0] negative pressure, [1] first-order fallbacks
   // solver (T = double or float, both allocated lazily)
@@ -5869,6 +6170,7 @@ struct Ctx::Impl {
   template <typename T>
   void enqueue_step_tail();
   hipGraphExec_t capture(void (Ctx::Impl::*enq)());
+  void build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf);
   hipStream_t cap_stream = nullptr;
   hipGraphExec_t g_head = nullptr, g_chunk = nullptr, g_tail = nullptr;
   int dev_phase = 0;  // 1: head or chunk in flight, 2: tail in flight
@@ -5933,6 +6235,105 @@ static uint64_t morton3(double x, double y, double z) {
     return (uint64_t)(u * (double)(1 << 21));
   };
   return spread(q(x)) | spread(q(y)) << 1 | spread(q(z)) << 2;
+}
+
+// Cuts the device-ordered cells (ci, cf: their entries) into tiles within the
+// limits above, in order, and lists what each tile's kernels need.
+void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf) {
+  std::vector<Tile> tl;
+  std::vector<int> hl;
+  std::vector<unsigned short> ln(std::max<size_t>(1, cf.size()));
+  std::vector<unsigned> ev;  // entry | other entry << 16
+  std::vector<uint2> tcl(std::max(1, ncv));
+  hl.reserve(ncv);
+  ev.reserve(cf.size() * 7 / 10 + 16);
+  std::vector<int> stamp(ncv, -1), hrow(ncv), fent(std::max(1, nfa), -1);
+  int c0 = 0;
+  while (c0 < ncv) {
+    const int t = (int)tl.size();
+    int c1 = c0, nev = 0, nh = 0;
+    for (; c1 < ncv && c1 - c0 < kTileCells && ci[c1 + 1] - ci[c0] <= kTileEnt; c1++) {
+      int dev = 0, dh = 0;  // what cell c1 adds; neighbours seen but not yet in the tile count as halo
+      for (int e = ci[c1]; e < ci[c1 + 1]; e++) {
+        const int nb = cf[e].y;
+        if (nb < 0 || nb < c0 || nb >= c1) dev++;
+        if (nb >= 0 && (nb < c0 || nb > c1) && stamp[nb] != t) dh++;
+      }
+      if (stamp[c1] == t) dh--;
+      if (c1 > c0 && (nev + dev > kTileEval || c1 + 1 - c0 + nh + dh > kTileRows)) break;
+      for (int e = ci[c1]; e < ci[c1 + 1]; e++)
+        if (cf[e].y >= 0) stamp[cf[e].y] = t;
+      nev += dev;
+      nh += dh;
+    }
+    if (c1 == c0) c1 = c0 + 1;  // one cell alone (at most 64 faces) always fits
+    const std::vector<int> &ki = h_dev_nbocv_i;
+    Tile T{c0, c1 - c0, (int)hl.size(), 0, ci[c0], ci[c1] - ci[c0], ki[c0], ki[c1] - ki[c0], (int)ev.size(), 0, 0, 0};
+    for (int c = c0; c < c1; c++)
+      for (int e = ci[c]; e < ci[c + 1]; e++) {
+        const int nb = cf[e].y, f = cf[e].x & 0x7fffffff;
+        const unsigned el = e - T.e0, alone = el | kNoEntry << 16;
+        if (nb < 0) {
+          ln[e] = kNoRow;
+          ev.push_back(alone);
+        } else if (nb >= c0 && nb < c1) {
+          ln[e] = (unsigned short)(nb - c0);
+          if (nb > c) {
+            fent[f] = e;
+          } else {  // the face's second entry: evaluated once, from its first side
+            const unsigned l2 = fent[f] - T.e0;
+            ev.push_back(cf[e].x >= 0 ? el | l2 << 16 : l2 | el << 16);
+          }
+        } else {
+          if (stamp[nb] != -2 - t) {
+            stamp[nb] = -2 - t;
+            hrow[nb] = (int)hl.size() - T.h0;
+            hl.push_back(nb);
+          }
+          ln[e] = (unsigned short)(c1 - c0 + hrow[nb]);
+          ev.push_back(alone);
+        }
+      }
+    // the cells by entry count, so that the lanes of a wavefront that work on
+    // one each loop about equally long
+    int cnt[66] = {0};
+    for (int c = c0; c < c1; c++) cnt[ci[c + 1] - ci[c] + 1]++;
+    for (int k = 1; k < 66; k++) cnt[k] += cnt[k - 1];
+    for (int c = c0; c < c1; c++) {
+      const int n = ci[c + 1] - ci[c];
+      int ni = 0;
+      while (ni < n && cf[ci[c] + ni].y >= 0) ni++;
+      tcl[c0 + cnt[n]++] = make_uint2((unsigned)((c - c0) | n << 8 | (ci[c] - T.e0) << 16),
+                                      (unsigned)((ki[c] - T.k0) | ni << 16));
+    }
+    T.nh = (int)hl.size() - T.h0;
+    T.nw = (int)ev.size() - T.w0;
+    tl.push_back(T);
+    c0 = c1;
+  }
+  ntile = (int)tl.size();
+  // one buffer: headers, cells, halo, neighbours, evaluations
+  size_t at[6] = {0, sizeof(Tile) * tl.size(), sizeof(uint2) * tcl.size(), sizeof(int) * hl.size(),
+                  sizeof(unsigned short) * ln.size(), sizeof(unsigned) * ev.size()};
+  for (int k = 1; k < 6; k++) at[k] = (at[k - 1] + at[k] + 15) & ~(size_t)15;
+  std::vector<char> blob(at[5]);  // what is uploaded; the evaluations' room follows it
+  auto put = [&](int k, const void *src, size_t bytes) {
+    if (bytes) std::memcpy(blob.data() + at[k], src, bytes);
+  };
+  put(0, tl.data(), sizeof(Tile) * tl.size());
+  put(1, tcl.data(), sizeof(uint2) * tcl.size());
+  put(2, hl.data(), sizeof(int) * hl.size());
+  put(3, ln.data(), sizeof(unsigned short) * ln.size());
+  put(4, ev.data(), sizeof(unsigned) * ev.size());
+  tiles.alloc(at[5] + sizeof(int4) * ev.size());
+  HIPCHECK(hipMemcpy(tiles.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
+  dm.ntile = ntile;
+  dm.tile = (const Tile *)(tiles.p + at[0]);
+  dm.tcell = (const uint2 *)(tiles.p + at[1]);
+  dm.halo = (const int *)(tiles.p + at[2]);
+  dm.lnb = (const unsigned short *)(tiles.p + at[3]);
+  dm.eval = (const int4 *)(tiles.p + at[5]);
+  eval_packed = (const unsigned *)(tiles.p + at[4]);
 }
 
 Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) : d_(new Impl) {
@@ -6213,6 +6614,8 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
     d.wave_e0.upload(we.data(), we.size());
     d.cfl_noc.upload(noc.data(), noc.size());
     d.cfl_tnoc.alloc(std::max<size_t>(1, dcf.size()));
+    d.nent = (int)dcf.size();
+    d.build_tiles(dci, dcf);
   }
   std::vector<int> bcell(std::max(1, nfa_b), 0);
   for (int f = 0; f < nfa_b; f++) bcell[f] = inv[m.cvofa[2 * (size_t)f]];
@@ -6354,6 +6757,12 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
                      d.nbocv_v.p, d.cfl_tnoc.p);
   HIPCHECK(hipGetLastError());
   d.dm.cfl_tnoc = d.cfl_tnoc.p;
+  if (!d.par.grad_ls) {
+    d.gg.alloc(5 * (size_t)std::max(1, d.nent));
+    d.dm.gg = d.gg.p;
+    hipLaunchKernelGGL(k_gg_coeff, dim3(nblk(ncv)), dim3(kBlock), 0, d.stream, d.dm, d.prim.p, d.gg.p);
+    HIPCHECK(hipGetLastError());
+  }
   if (d.par.mu_ref > 0.0) {
     d.muf.alloc(2 * (size_t)std::max(1, nfa));
     d.fcell.alloc(std::max(1, nfa - nfa_b));
@@ -6375,6 +6784,11 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
   d.dm.nwave = d.nwave;
   d.dm.foc = d.foc.p;
   d.dm.cell_perm = d.cell_perm.p;
+  if (d.ntile > 0) {
+    hipLaunchKernelGGL(k_tile_eval, dim3(d.ntile), dim3(kBlock), 0, d.stream, d.dm, d.eval_packed,
+                       const_cast<int4 *>(d.dm.eval));
+    HIPCHECK(hipGetLastError());
+  }
 
   d.dp.gamma = d.par.gamma;
   d.dp.R = d.par.R_gas;
@@ -6755,7 +7169,7 @@ void StepBatch::set(Ctx *const *ctxs, int n, void *stream) {
     const bool grad = d.par.second_order || d.dp.visc;
     const bool ent = d.par.grad_kernel == kResidEntry && !d.dp.visc;
     J.n[kShCell] = nblk(d.ncv);
-    J.n[kShGrad] = !grad ? 0 : ent ? (d.nwave + kWaves - 1) / kWaves : nblk(d.ncv);
+    J.n[kShGrad] = !grad ? 0 : ent ? (d.nwave + kWaves - 1) / kWaves : nblk(grad_fields(d.dp.visc) * (long long)d.ncv);
     // the batched flux kernel runs blocks of kWaves wavefronts
     J.n[kShFlux] = d.flux_entry() ? (d.nwave + kWaves - 1) / kWaves : nblk(d.ncv);
     J.n[kShBc] = d.nfa_b > 0 ? nblk(d.nfa_b) : 0;
@@ -7068,11 +7482,22 @@ void Ctx::Impl::launch_grad(hipStream_t s) {
   if (!par.second_order && !dp.visc) return;
   // the per-entry gradient kernel has no viscous variant
   const bool ent = par.grad_kernel == kResidEntry && !dp.visc;
-  const dim3 g(ent ? (nwave + kGradWaves - 1) / kGradWaves : nblk(ncv));
+  const dim3 g(ent ? (nwave + kGradWaves - 1) / kGradWaves : nblk(grad_fields(dp.visc) * (long long)ncv));
   if (ent) {
     const dim3 b(64 * kGradWaves);
     if (par.grad_ls) hipLaunchKernelGGL(k_grad_e<true>, g, b, 0, s, dm, dp, prim.p, bfa.p, grad.p);
     else hipLaunchKernelGGL(k_grad_e<false>, g, b, 0, s, dm, dp, prim.p, bfa.p, grad.p);
+  } else if (grad_tiled()) {
+    auto got = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(ntile), dim3(kBlock), 0, s, dm, dp, prim.p, bfa.p, grad.p, gradv.p);
+    };
+    if (dp.visc) {
+      if (par.grad_ls) got(k_grad_t<true, true>);
+      else got(k_grad_t<false, true>);
+    } else {
+      if (par.grad_ls) got(k_grad_t<true, false>);
+      else got(k_grad_t<false, false>);
+    }
   } else {
     if (dp.visc) {
       if (par.grad_ls) hipLaunchKernelGGL((k_grad<true, true>), g, dim3(kBlock), 0, s, dm, dp, prim.p, bfa.p, grad.p, gradv.p);
@@ -7118,6 +7543,7 @@ void Ctx::Impl::launch_dt_fin() {
 
 int Ctx::Impl::flux_blocks() const {
   if (face_form()) return (nwave + kWaves - 1) / kWaves;  // k_gather_e
+  if (flux_tiled()) return ntile;
   return flux_entry() ? (nwave + kFluxWaves - 1) / kFluxWaves : nblk(ncv);
 }
 
@@ -7155,36 +7581,40 @@ void Ctx::Impl::launch_flux(hipStream_t s, const double *cfl_dev) {
     }
     return;
   }
-  if (flux_entry()) {
+  if (flux_tiled()) {
+    auto got = [&](auto kern) {
+      hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, dm, dp, prim.p, grad.p, bfa.p, q.p, rhs.p, counters.p + 1, dta,
+                         dt.p, partials.p);
+    };
+    if (par.second_order) {
+      if (par.scheme == kRoe) got(k_flux_t<kRoe, true>);
+      else if (par.scheme == kAusm) got(k_flux_t<kAusm, true>);
+      else if (par.scheme == kHllcC) got(k_flux_t<kHllcC, true>);
+      else got(k_flux_t<kHllc, true>);
+    } else {
+      if (par.scheme == kRoe) got(k_flux_t<kRoe, false>);
+      else if (par.scheme == kAusm) got(k_flux_t<kAusm, false>);
+      else if (par.scheme == kHllcC) got(k_flux_t<kHllcC, false>);
+      else got(k_flux_t<kHllc, false>);
+    }
+    return;
+  }
+  if (flux_entry()) {  // viscous
     if (par.sst) {  // HLLC, viscous (the parser requires both)
       if (par.second_order) goe(k_flux_e<kHllc, true, true, true>);
       else goe(k_flux_e<kHllc, false, true, true>);
       return;
     }
-    if (dp.visc) {
-      if (par.second_order) {
-        if (par.scheme == kRoe) goe(k_flux_e<kRoe, true, true>);
-        else if (par.scheme == kAusm) goe(k_flux_e<kAusm, true, true>);
-        else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, true, true>);
-        else goe(k_flux_e<kHllc, true, true>);
-      } else {
-        if (par.scheme == kRoe) goe(k_flux_e<kRoe, false, true>);
-        else if (par.scheme == kAusm) goe(k_flux_e<kAusm, false, true>);
-        else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, false, true>);
-        else goe(k_flux_e<kHllc, false, true>);
-      }
+    if (par.second_order) {
+      if (par.scheme == kRoe) goe(k_flux_e<kRoe, true, true>);
+      else if (par.scheme == kAusm) goe(k_flux_e<kAusm, true, true>);
+      else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, true, true>);
+      else goe(k_flux_e<kHllc, true, true>);
     } else {
-      if (par.second_order) {
-        if (par.scheme == kRoe) goe(k_flux_e<kRoe, true, false>);
-        else if (par.scheme == kAusm) goe(k_flux_e<kAusm, true, false>);
-        else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, true, false>);
-        else goe(k_flux_e<kHllc, true, false>);
-      } else {
-        if (par.scheme == kRoe) goe(k_flux_e<kRoe, false, false>);
-        else if (par.scheme == kAusm) goe(k_flux_e<kAusm, false, false>);
-        else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, false, false>);
-        else goe(k_flux_e<kHllc, false, false>);
-      }
+      if (par.scheme == kRoe) goe(k_flux_e<kRoe, false, true>);
+      else if (par.scheme == kAusm) goe(k_flux_e<kAusm, false, true>);
+      else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, false, true>);
+      else goe(k_flux_e<kHllc, false, true>);
     }
   } else {
     if (par.second_order) {

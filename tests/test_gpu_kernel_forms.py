@@ -110,3 +110,34 @@ def test_sst_rows_per_entry_equal_per_cell(n, frac):
     b = values(mesh, joe + "GPU_SCAL_KERNEL = CELL\n", names)
     for k in names:
         assert np.array_equal(a[k], b[k], equal_nan=True), k
+
+
+# the gradient per cell and field against the per-entry form and against
+# itself with the cells of a tile in another thread order
+@pytest.mark.parametrize("grad", ["LEASTSQUARES", "GREENGAUSS"])
+@pytest.mark.parametrize("n,frac", [(1, 0.0), (1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0), (9, 0.5)])
+def test_gradient_forms_agree(n, frac, grad):
+    print(f"gradient forms n={n} frac={frac} {grad}", flush=True)
+    mesh, joe = box(n, frac, grad=grad)
+    names = ["GRAD_RHO", "GRAD_P", "GRAD_U", "ALPHA_RHO", "RHS_RHO", "RHS_RHOU", "RHS_RHOE"]
+    ref = values(mesh, joe + "GPU_GRAD_KERNEL = ENTRY\n", names, implicit=False)
+    for keys in ("GPU_GRAD_KERNEL = CELL\n", "GPU_GRAD_KERNEL = CELL\nGPU_GRAD_THREAD_ORDER = SORTED\n"):
+        got = values(mesh, joe + keys, names, implicit=False)
+        for k in names:
+            assert np.array_equal(got[k], ref[k], equal_nan=True), k
+
+
+# the inviscid flux by tiles (every option of it, both time steps) against the
+# per-cell form, and per-face fluxes
+@pytest.mark.parametrize("n,frac", [(1, 0.0), (1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0), (9, 0.5)])
+@pytest.mark.parametrize("scheme", ["HLLC", "ROE", "AUSM"])
+@pytest.mark.parametrize("second", [True, False])
+@pytest.mark.parametrize("extra", ["", "TIME_STEP = SUM_BASED\n", "GRAVITY 0.1 -0.2 0.3\n"])
+def test_flux_forms_agree(n, frac, scheme, second, extra):
+    print(f"flux forms n={n} frac={frac} {scheme} {second} {extra!r}", flush=True)
+    mesh, joe = box(n, frac, scheme, second_order=second)
+    names = ["RHS_RHO", "RHS_RHOU", "RHS_RHOE", "LOCAL_DT"]
+    a = values(mesh, joe + extra + "GPU_FLUX_KERNEL = ENTRY\n", names, implicit=False)
+    b = values(mesh, joe + extra + "GPU_FLUX_KERNEL = CELL\n", names, implicit=False)
+    for k in names:
+        assert np.array_equal(a[k], b[k], equal_nan=True), k
