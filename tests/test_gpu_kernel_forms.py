@@ -141,3 +141,31 @@ def test_flux_forms_agree(n, frac, scheme, second, extra):
     b = values(mesh, joe + extra + "GPU_FLUX_KERNEL = CELL\n", names, implicit=False)
     for k in names:
         assert np.array_equal(a[k], b[k], equal_nan=True), k
+
+
+def morton(x):
+    """21 bits of every coordinate of the centroids, scaled by their largest
+    extent, interleaved with x lowest."""
+    lo = x.min(0)
+    q = (np.minimum((x - lo) / (x.max(0) - lo).max(), 0.99999999) * (1 << 21)).astype(np.uint64)
+    key = np.zeros(len(x), np.uint64)
+    for b in range(21):
+        for i in range(3):
+            key |= ((q[:, i] >> np.uint64(b)) & np.uint64(1)) << np.uint64(3 * b + i)
+    return key
+
+
+# cells along the Morton curve, equal keys in their own order: either side of
+# the size from which the sort goes by digits (65536), with the centroids as
+# they are and moved to the corners of an 8^3 grid, so that many share a key
+@pytest.mark.parametrize("n,grid", [(2, None), (40, None), (41, None), (40, 8), (41, 8)])
+def test_cell_order_is_the_stable_morton_order(n, grid):
+    print(f"cell order n={n} grid={grid}", flush=True)
+    mm, joe = cases.box_case(n, frac=0.0, seed=n)
+    dump = joemi.Mesh.from_faces(mm).as_dump()
+    x = dump["X_CV"].reshape(-1, 3)
+    if grid:
+        x[:] = np.floor(x * grid) / grid
+    mesh = joemi.Mesh.from_ugp(dump)
+    pos = joemi.Solver(mesh, joe + "GPU_CELL_ORDER = MORTON\n").get("CELL_ORDER").astype(np.int64)
+    assert np.array_equal(np.argsort(pos), np.argsort(morton(x[:mesh.ncv]), kind="stable"))
