@@ -1852,30 +1852,48 @@ __global__ void __launch_bounds__(kBlock) k_jac(DMesh m, DParams P, const double
 // few waves its registers allow, so one matrix per lane, formed row by row
 // straight into LDS (jac_hllc_rows), is worth more than the arithmetic it
 // saves: 146-160 registers and three waves per SIMD where two matrices held
-// whole took 256 and one. 386k-cell split box, FP64: 392 -> 208 us; 687k-cell
-// SST plate: 1531 -> 696 us; the 6x6 form (200 registers, 18.8 KB of LDS per
-// wavefront, two waves) 454 -> 386 us at 250k cells.
+// whole took 256 and one; the sums and the stores read LDS for several values
+// at once, since a read waited for by itself costs a hundred cycles and there
+// are sixty (2M-cell SA plate, 6x6 FP32: 2514 -> 1764 us). 386k-cell split box,
+// FP64: 392 -> 192 us; 687k-cell SST plate: 1531 -> 566 us. The coupled viscous
+// form takes 202 registers and 18.9 KB of LDS per wavefront: two waves.
 // ---------------------------------------------------------------------------
-// the entries of a coupled viscous block (visc_coupled_jac) that may be
-// nonzero: [1+i][0], [1+i][1+i] for i < 3 and row 4; -1 for the others
-__device__ __forceinline__ int vc_index(int k) {
-  switch (k) {
-    case 5: return 0;
-    case 6: return 1;
-    case 10: return 2;
-    case 12: return 3;
-    case 15: return 4;
-    case 18: return 5;
-    case 20: return 6;
-    case 21: return 7;
-    case 22: return 8;
-    case 23: return 9;
-    case 24: return 10;
-    default: return -1;
+// The entries of a coupled viscous block (visc_coupled_jac) that may be
+// nonzero: [1+i][0], [1+i][1+i] for i < 3 and row 4. Component k's place among
+// them, kVcN (a slot that holds 0.0: a sum that starts from 0.0 is never -0.0,
+// so adding it changes nothing) for the others.
+constexpr int kVcN = 11;
+constexpr unsigned kVcMask = 1u << 5 | 1u << 6 | 1u << 10 | 1u << 12 | 1u << 15 | 1u << 18 | 31u << 20;
+__device__ __forceinline__ constexpr int vc_slot(int k) {
+  return kVcMask >> k & 1 ? __builtin_popcount(kVcMask & ((1u << k) - 1)) : kVcN;
+}
+constexpr int kMaxOwned = 7;  // components of the diagonal block per lane (cells have at least 4 faces)
+
+// the sums over a cell's entries, in their order, of the components pos,
+// pos + nent, ... of their slots (S: the first one's; CV: each value followed
+// by the component's viscous one); an entry's reads are issued together
+template <int NS, bool CV>
+__device__ __forceinline__ void own_sums(const double *S, int pos, int nent, double *D) {
+  int at[kMaxOwned];
+#pragma unroll
+  for (int q = 0; q < kMaxOwned; q++) {
+    D[q] = 0.0;
+    at[q] = min(pos + q * nent, 24);  // past the last: summed and not used
+  }
+  for (int j = 0; j < nent; j++, S += NS) {
+    double v[kMaxOwned], w[kMaxOwned];
+#pragma unroll
+    for (int q = 0; q < kMaxOwned; q++) {
+      v[q] = S[at[q]];
+      if (CV) w[q] = S[25 + vc_slot(at[q])];
+    }
+#pragma unroll
+    for (int q = 0; q < kMaxOwned; q++) {
+      D[q] += v[q];
+      if (CV) D[q] += w[q];
+    }
   }
 }
-constexpr int kVcN = 11;
-constexpr int kMaxOwned = 7;  // components of the diagonal block per lane (cells have at least 4 faces)
 
 // SST: the cells' (or the boundary's) turbulent kinetic energy in the HLLC
 // Jacobian (kineCV / kineFA, JoeWithModels.cpp:3034-3037, 3202-3206, 3490-3495)
@@ -1888,10 +1906,8 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
                                         const double *__restrict__ gradv) {
   constexpr bool CPL = SCHEME == kHllcC;
   constexpr bool CV = VISC && CPL;
-  constexpr int NS = CV ? 25 + kVcN : 25;
+  constexpr int NS = CV ? 25 + kVcN + 1 : 25;  // odd: lanes' slots on different banks
   __shared__ double lds[64 * W * NS];
-  __shared__ signed char vsg[64 * W];  // the entry's viscous block: 0 none, +1 added, -1 subtracted
-  __shared__ int toff[64 * W];         // the entry's off-diagonal block, -1 without one
   double *slot = lds + NS * threadIdx.x;
   const EntryLane L = entry_lane<W>(m, B);
   const double gam = P.gamma;
@@ -1978,7 +1994,6 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         slot[5 * (i + 1) + 4] = a2 * n[i] * area;
       }
     }
-    signed char vs = 0;
     if (CV) {  // the same face's viscous block next (JoeWithModels.cpp:5096-5104)
       if (internal) {
         const VSide vo = vside_cell(P, pc, gradv + 12 * (size_t)c);
@@ -1995,11 +2010,9 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         double VF[5], tau[3], keff;
         visc_coupled(P, a, b, mul, mut, ufa, area, n, smag, sV, alpha, VF, tau, keff, P.sa != 0);
         visc_coupled_jac(P, J, s0 ? 0 : 1, vsel(s0, a, b), mul + mut, keff, tau, ufa, area, alpha, smag);
-        for (int k = 0; k < 25; k++) {
-          const int vi = vc_index(k);
-          if (vi >= 0) slot[25 + vi] = s0 ? J[k / 5][k % 5] : -J[k / 5][k % 5];
-        }
-        vs = s0 ? 1 : -1;
+#pragma unroll
+        for (int k = 0; k < 25; k++)
+          if (vc_slot(k) < kVcN) slot[25 + vc_slot(k)] = s0 ? J[k / 5][k % 5] : -J[k / 5][k % 5];
       } else if (z->bc != kBcSymmetry) {  // none on symmetry faces
         const double *gvo = gradv + 12 * (size_t)c;
         const VSide vo = vside_cell(P, pc, gvo);
@@ -2013,40 +2026,25 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
         double VF[5], tau[3], keff;
         visc_coupled(P, lv, vb, mul, mut, vb.u, area, n, smag, sArg, alpha, VF, tau, keff, P.sa != 0);
         visc_coupled_jac(P, J, 0, lv, mul + mut, keff, tau, vb.u, area, alpha, smag);
-        for (int k = 0; k < 25; k++) {
-          const int vi = vc_index(k);
-          if (vi >= 0) slot[25 + vi] = J[k / 5][k % 5];
-        }
-        vs = 1;
+#pragma unroll
+        for (int k = 0; k < 25; k++)
+          if (vc_slot(k) < kVcN) slot[25 + vc_slot(k)] = J[k / 5][k % 5];
+      } else {
+#pragma unroll
+        for (int k = 0; k < kVcN; k++) slot[25 + k] = 0.0;
       }
+      slot[25 + kVcN] = 0.0;
     }
-    vsg[threadIdx.x] = vs;
   }
   toff[threadIdx.x] = L.e >= 0 ? m.cfl_tnoc[L.e] : -1;
   __syncthreads();
   // the cell's diagonal block, summed in entry order by the cell's lanes
   double Dk[kMaxOwned];
   const int first = threadIdx.x - pos;
-  if (L.e >= 0) {
-    int q = 0;
-    for (int k = pos; k < 25; k += nent, q++) {
-      double d = 0.0;
-      for (int j = 0; j < nent; j++) {
-        const double *sj = lds + NS * (first + j);
-        d += sj[k];
-        if (CV) {
-          const int sg = vsg[first + j];
-          if (sg != 0) {
-            const int vi = vc_index(k);
-            d += vi >= 0 ? sj[25 + vi] : (sg > 0 ? 0.0 : -0.0);
-          }
-        }
-      }
-      Dk[q] = d;
-    }
-  }
+  if (L.e >= 0) own_sums<NS, CV>(lds + NS * first, pos, nent, Dk);
   if (VISC && !CPL) {  // viscous blocks after every Euler block (JoeWithModels.cpp:3680-3697, 3789-3796, 3835-3842)
     __syncthreads();
+    bool vs = false;  // the entry has a viscous block
     if (L.e >= 0) {
       const int2 en = m.cfl[L.e];
       const int f = en.x & 0x7fffffff;
@@ -2058,7 +2056,6 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
       if (SST) vo.k = P.sst_phi[c];
       double Fu[3], FE;
       VFace vf;
-      signed char vs = 0;
       if (en.y >= 0) {
         const double *pn = prim + 8 * (size_t)en.y;
         VSide vn = vside_cell(P, pn, gradv + 12 * (size_t)en.y);
@@ -2087,7 +2084,7 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
             slot[5 * i + j] = v;
             J[i][j] = (double)(T)((double)(T)(0.0 - inv) - v);  // the off-diagonal value
           }
-        vs = 1;
+        vs = true;
       } else {
         const ZoneDev &z = m.zones[-en.y - 1];
         if (z.bc != kBcSymmetry) {
@@ -2114,32 +2111,31 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
           visc_jac<SST>(P, J, -1.0, vo, mul, mut, vf, vb.u, area, smag);
           for (int i = 1; i < 5; i++)
             for (int j = 0; j < 5; j++) slot[5 * i + j] = -J[i][j];
-          vs = 1;
+          vs = true;
         }
       }
-      vsg[threadIdx.x] = vs;
     }
+    const unsigned long long vsm = __ballot(vs) >> (first & 63);  // from the cell's first entry on
     __syncthreads();
-    if (L.e >= 0) {
-      int q = 0;
-      for (int k = pos; k < 25; k += nent, q++) {
-        if (k < 5) continue;  // rows 1-4 only
-        double d = Dk[q];
-        for (int j = 0; j < nent; j++)
-          if (vsg[first + j]) d += lds[NS * (first + j) + k];
-        Dk[q] = d;
+    if (L.e >= 0)
+      for (int j = 0; j < nent; j++) {
+        if (!(vsm >> j & 1)) continue;
+        const double *sj = lds + NS * (first + j);
+#pragma unroll
+        for (int q = 0; q < kMaxOwned; q++) {
+          const int k = pos + q * nent;
+          if (k >= 5 && k < 25) Dk[q] += sj[k];  // rows 1-4 only
+        }
       }
-    }
   }
   // the off-diagonal blocks: the slots' values negated, less the viscous ones
   if (VISC) {
     __syncthreads();
-    if (L.e >= 0 && toff[threadIdx.x] >= 0) {
+    if (toff >= 0) {
 #pragma unroll
       for (int k = 0; k < 25; k++) {
         if (CPL) {
-          const int vi = vc_index(k);
-          if (vi >= 0) slot[k] = -(double)(T)((double)(T)(0.0 - slot[k]) - slot[25 + vi]);
+          if (vc_slot(k) < kVcN) slot[k] = -(double)(T)((double)(T)(0.0 - slot[k]) - slot[25 + vc_slot(k)]);
         } else if (k >= 5) {
           slot[k] = -J[k / 5][k % 5];
         }
@@ -2151,21 +2147,24 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
     constexpr int NR = 5 * NB;  // the flow rows of a block; with the scalar their sixth column is zero
     const int lane = threadIdx.x & 63, wb = threadIdx.x - lane;
     int en = lane / NR, k = lane % NR;
-    for (int it = 0; it < NR; it++) {
-      const int tn = toff[wb + en];
-      if (tn >= 0) {
-        const double *sj = lds + NS * (wb + en);
-        T v;
-        if (NB == 6) v = k % 6 == 5 ? (T)0.0 : (T)(0.0 - sj[k - k / 6]);
-        else v = (T)(0.0 - sj[k]);
-        A[NB * NB * (size_t)tn + k] = v;
+    for (int it = 0; it < NR; it += 5) {  // five at a time, so that their LDS reads are in flight together
+      int tn[5], kk[5];
+      double v[5];
+#pragma unroll
+      for (int u = 0; u < 5; u++) {
+        tn[u] = __shfl(toff, en);
+        kk[u] = k;
+        v[u] = lds[NS * (wb + en) + (NB == 6 ? k - k / 6 : k)];
+        k += 64 % NR;
+        en += 64 / NR;
+        if (k >= NR) {
+          k -= NR;
+          en++;
+        }
       }
-      k += 64 % NR;
-      en += 64 / NR;
-      if (k >= NR) {
-        k -= NR;
-        en++;
-      }
+#pragma unroll
+      for (int u = 0; u < 5; u++)
+        if (tn[u] >= 0) A[NB * NB * (size_t)tn[u] + kk[u]] = NB == 6 && kk[u] % 6 == 5 ? (T)0.0 : (T)(0.0 - v[u]);
     }
   }
   if (L.e < 0) return;
@@ -2173,8 +2172,10 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
   const double vol = m.vol[c];
   const double tmp = step_mode ? vol / (dt[c]) : 0.0;
   T *dgl = A + NB * NB * (size_t)m.nbocv_i[c];
-  int q = 0;
-  for (int k = pos; k < 25; k += nent, q++) {
+#pragma unroll
+  for (int q = 0; q < kMaxOwned; q++) {
+    const int k = pos + q * nent;
+    if (k >= 25) break;
     const int i = k / 5, j = k % 5;
     double d = Dk[q];
     if (P.gravity_on) {
