@@ -2036,7 +2036,7 @@ __device__ __forceinline__ void d_jac_e(const Blk &B, DMesh m, DParams P, const 
       slot[25 + kVcN] = 0.0;
     }
   }
-  toff[threadIdx.x] = L.e >= 0 ? m.cfl_tnoc[L.e] : -1;
+  const int toff = L.e >= 0 ? m.cfl_tnoc[L.e] : -1;  // the entry's off-diagonal block, -1 without one
   __syncthreads();
   // the cell's diagonal block, summed in entry order by the cell's lanes
   double Dk[kMaxOwned];
