@@ -3632,25 +3632,81 @@ __device__ __forceinline__ void block_partials(double (&v)[NV], double *partials
   block_partials<NV>(v, partials, sh, op, hw_blk());
 }
 
-// fixed-order combination of nb partials; valid in thread 0
-__device__ double fin_slot(const double *__restrict__ p, int nb, int op, double *sh) {
-  const double id = op == kSum ? 0.0 : (op == kMax ? -__builtin_huge_val() : __builtin_huge_val());
-  // four independent chains per thread keep four loads in flight
-  double x0 = id, x1 = id, x2 = id, x3 = id;
-  const int st = blockDim.x;
-  int b = threadIdx.x;
-  for (; b + 3 * st < nb; b += 4 * st) {
-    x0 = rcomb(x0, p[b], op);
-    x1 = rcomb(x1, p[b + st], op);
-    x2 = rcomb(x2, p[b + 2 * st], op);
-    x3 = rcomb(x3, p[b + 3 * st], op);
+// Fixed-order combination of nb partials of NV sums (or maxima, minima: op),
+// `stride` apart, in every thread. The order is that of a block of kFinBlock
+// threads; a smaller one (a divisor of it, whole wavefronts) has its thread t
+// play that block's threads t, t + blockDim.x, ..., so the bits do not depend
+// on the launch. All values' loads, shuffles and barriers go together. sh
+// holds 16 NV doubles.
+constexpr int kFinBlock = 1024;
+
+template <int NV>
+__device__ __forceinline__ void fin_slots(const double *__restrict__ p, size_t stride, int nb, const int (&op)[NV],
+                                          double *sh, double (&out)[NV]) {
+  const int st = kFinBlock, lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  double id[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+    id[k] = op[k] == kSum ? 0.0 : (op[k] == kMax ? -__builtin_huge_val() : __builtin_huge_val());
+  __syncthreads();  // sh may still be read by a previous call
+  for (int r = 0; r < kFinBlock / (int)blockDim.x; r++) {
+    double x[NV];
+    if (r * (int)blockDim.x >= nb) {  // no partials for these waves
+#pragma unroll
+      for (int k = 0; k < NV; k++) x[k] = id[k];
+    } else {
+      // four independent chains per value keep four loads in flight
+      double x0[NV], x1[NV], x2[NV], x3[NV];
+#pragma unroll
+      for (int k = 0; k < NV; k++) x0[k] = x1[k] = x2[k] = x3[k] = id[k];
+      int b = threadIdx.x + r * blockDim.x;
+      for (; b + 3 * st < nb; b += 4 * st) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+          const double *q = p + k * stride + b;
+          x0[k] = rcomb(x0[k], q[0], op[k]);
+          x1[k] = rcomb(x1[k], q[st], op[k]);
+          x2[k] = rcomb(x2[k], q[2 * st], op[k]);
+          x3[k] = rcomb(x3[k], q[3 * st], op[k]);
+        }
+      }
+      for (; b < nb; b += st) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) x0[k] = rcomb(x0[k], p[k * stride + b], op[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < NV; k++) x[k] = rcomb(rcomb(x0[k], x1[k], op[k]), rcomb(x2[k], x3[k], op[k]), op[k]);
+      for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) x[k] = rcomb(x[k], __shfl_down(x[k], off, 64), op[k]);
+      }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) sh[k * 16 + wid + r * nw] = x[k];
+    }
   }
-  for (; b < nb; b += st) x0 = rcomb(x0, p[b], op);
-  double v[1] = {rcomb(rcomb(x0, x1, op), rcomb(x2, x3, op), op)};
   __syncthreads();
-  block_reduce<1>(v, sh, op);
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    double v = sh[k * 16];
+#pragma unroll
+    for (int w = 1; w < kFinBlock / 64; w++) v = rcomb(v, sh[k * 16 + w], op[k]);
+    out[k] = v;
+  }
+}
+
+__device__ double fin_slot(const double *__restrict__ p, int nb, int op, double *sh) {
+  const int ops[1] = {op};
+  double v[1];
+  fin_slots<1>(p, 0, nb, ops, sh, v);
   return v[0];
 }
+
+// threads of a block that finishes nb partials: the waves past them would only
+// hold it up (61 partials, the kernel's mean over a step: 5.6 us with sixteen
+// waves, 3.5 with four)
+inline int fin_threads(int nb) { return nb <= kBlock ? kBlock : kFinBlock; }
 
 enum FinOp {
   kFinDt = 0, kFinL1 = 1, kFinAlpha = 2, kFinOmega = 3, kFinResid0 = 4, kFinResid = 5,
@@ -3660,9 +3716,9 @@ enum FinOp {
   kFinConfirm = 9   // kFinResid on the true residual, for solves that wait for it (done 3)
 };
 
-// one block: finishes a reduction and applies the scalar update of its owner
-constexpr int kFinBlock = 1024;
+// one block: finishes a reduction and applies the scalar update of its owner;
 // slot k of the partials at partials + k * stride (nb values each)
+constexpr int kFinShared = 16 * 2;
 __device__ void fin_body(int nb, int op, const double *__restrict__ partials, size_t stride, SolverScalars *S,
                          double *sh) {
   if ((op == kFinAlpha || op == kFinOmega || op == kFinResid) && (S->done || S->stop)) return;
@@ -3672,13 +3728,14 @@ __device__ void fin_body(int nb, int op, const double *__restrict__ partials, si
     double m = fin_slot(partials, nb, kMin, sh);
     if (t0) S->dt_min = m;
   } else if (op == kFinL1) {
+    const int sums[2] = {kSum, kSum};
     for (int k = 0; k < 5; k++) {
-      double v = fin_slot(partials + (size_t)k * stride, nb, kSum, sh);
-      if (t0) S->resid[k] = v;
-    }
-    for (int k = 0; k < 5; k++) {
-      double v = fin_slot(partials + (size_t)(5 + k) * stride, nb, kSum, sh);
-      if (t0) S->resid_l2[k] = sqrt(v);
+      double v[2];  // L1 and squared L2 of field k
+      fin_slots<2>(partials + k * stride, 5 * stride, nb, sums, sh, v);
+      if (t0) {
+        S->resid[k] = v[0];
+        S->resid_l2[k] = sqrt(v[1]);
+      }
     }
   } else if (op == kFinL1S) {
     double v = fin_slot(partials, nb, kSum, sh);
@@ -3694,12 +3751,15 @@ __device__ void fin_body(int nb, int op, const double *__restrict__ partials, si
       S->alpha = S->rho / gamma;
     }
   } else if (op == kFinOmega) {  // :2808-2810
-    double st = fin_slot(partials, nb, kSum, sh);
-    double tt = fin_slot(partials + stride, nb, kSum, sh);
-    if (t0) S->omega = st / (tt + 1.0E-20);
+    const int sums[2] = {kSum, kSum};
+    double v[2];  // s.t, t.t
+    fin_slots<2>(partials, stride, nb, sums, sh, v);
+    if (t0) S->omega = v[0] / (v[1] + 1.0E-20);
   } else {  // residual: stop test (:2847-2856) and the next iteration's rho, beta (:2736-2749)
-    double rho_next = fin_slot(partials, nb, kSum, sh);
-    double mxv = fin_slot(partials + stride, nb, kMax, sh);
+    const int ops[2] = {kSum, kMax};
+    double v[2];
+    fin_slots<2>(partials, stride, nb, ops, sh, v);
+    const double rho_next = v[0], mxv = v[1];
     if (t0) {
       if (op == kFinResid0 || op == kFinResid0J) {
         S->res0_max = mxv;
@@ -3732,7 +3792,7 @@ __device__ void fin_body(int nb, int op, const double *__restrict__ partials, si
 
 __global__ void __launch_bounds__(kFinBlock) k_fin(int nb, int op, const double *__restrict__ partials,
                                                 SolverScalars *S) {
-  __shared__ double sh[16];
+  __shared__ double sh[kFinShared];
   fin_body(nb, op, partials, (size_t)nb, S, sh);
 }
 
@@ -3750,33 +3810,40 @@ __global__ void __launch_bounds__(256) k_min_pre(const double *__restrict__ in, 
   if (threadIdx.x == 0) out[blockIdx.x] = v[0];
 }
 
-// fin_slot of a kFinBlock-thread block computed by a smaller block (a divisor
-// of kFinBlock, whole wavefronts): thread t plays the full block's threads
-// t, t + blockDim.x, ..., each wave's lanes in the same shuffle tree, and the
-// sixteen wave results are combined in the same order, so the value is the
-// same bits as k_fin's. Valid in every thread; sh holds 16 doubles.
-__device__ double fin_slot_v(const double *__restrict__ p, int nb, int op, double *sh) {
-  const double id = op == kSum ? 0.0 : (op == kMax ? -__builtin_huge_val() : __builtin_huge_val());
-  const int st = kFinBlock, lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  __syncthreads();  // sh may still be read by a previous call
-  for (int r = 0; r < kFinBlock / (int)blockDim.x; r++) {
-    double x0 = id, x1 = id, x2 = id, x3 = id;
-    int b = threadIdx.x + r * blockDim.x;
-    for (; b + 3 * st < nb; b += 4 * st) {
-      x0 = rcomb(x0, p[b], op);
-      x1 = rcomb(x1, p[b + st], op);
-      x2 = rcomb(x2, p[b + 2 * st], op);
-      x3 = rcomb(x3, p[b + 3 * st], op);
-    }
-    for (; b < nb; b += st) x0 = rcomb(x0, p[b], op);
-    double x = rcomb(rcomb(x0, x1, op), rcomb(x2, x3, op), op);
-    for (int off = 32; off > 0; off >>= 1) x = rcomb(x, __shfl_down(x, off, 64), op);
-    if (lane == 0) sh[wid + r * nw] = x;
+// What bounds a small solve is the chain of its launches, nine of 2 to 4 us
+// each per iteration, two thirds of it waits. A solve with at most this many
+// partials therefore has no k_fin for alpha and omega:
+// every block of the kernel that uses the value finishes it by itself (two
+// launches of nine fewer per iteration), the first one stores it. A block
+// then reads at most 8 KB per sum, one value per thread of k_fin's; with more
+// blocks and more partials each the reads grow with their product. k_x_rec's
+// omega always has its k_fin: it leaves partials where the others are read.
+// 3072-cell bump, 25 steps (three to six iterations each): 9170 -> 8050 us,
+// and 7590 with fin_threads and both sums of a stop test read together.
+constexpr int kFinInline = kFinBlock;
+
+// alpha = rho / gamma, UgpWithCv.cpp:2775-2782
+__device__ __forceinline__ double fin_alpha(const double *__restrict__ partials, int nb, SolverScalars *S, bool first,
+                                            double *sh) {
+  double gamma = fin_slot(partials, nb, kSum, sh);
+  if (fabs(gamma) < 1.0E-20) gamma = 1.0E-20;
+  const double alpha = S->rho / gamma;
+  if (first && threadIdx.x == 0) {
+    S->gamma = gamma;
+    S->alpha = alpha;
   }
-  __syncthreads();
-  double v = sh[0];
-  for (int w = 1; w < kFinBlock / 64; w++) v = rcomb(v, sh[w], op);
-  return v;
+  return alpha;
+}
+
+// omega = (s.t) / (t.t + 1e-20), :2808-2810; the two slots `stride` apart
+__device__ __forceinline__ double fin_omega(const double *__restrict__ partials, int nb, size_t stride,
+                                            SolverScalars *S, bool first, double *sh) {
+  const int sums[2] = {kSum, kSum};
+  double v[2];  // s.t, t.t
+  fin_slots<2>(partials, stride, nb, sums, sh, v);
+  const double omega = v[0] / (v[1] + 1.0E-20);
+  if (first && threadIdx.x == 0) S->omega = omega;
+  return omega;
 }
 
 // Residual kernel: one cell per thread (flux_cell), block minima of the local
@@ -4799,15 +4866,17 @@ __global__ void __launch_bounds__(kBlock) k_spmv_dot(int ncv, const int *__restr
   block_partials<2>(v, partials, sh, kSum);
 }
 
-// s = res - alpha v; shat = LU^-1 s (with BJ = false only s)
+// s = res - alpha v; shat = LU^-1 s (with BJ = false only s). nfin > 0: alpha
+// finished here from that many partials (kFinInline); so omega in k_x
 template <typename T, int NB, bool BJ = true>
 __global__ void __launch_bounds__(kBlock) k_s(int ncv, const T *__restrict__ LU, const T *__restrict__ res,
                                               const T *__restrict__ v, T *__restrict__ s, T *__restrict__ shat,
-                                              const SolverScalars *S) {
+                                              SolverScalars *S, const double *__restrict__ fin, int nfin) {
+  __shared__ double sh[16];
   if (S->done || S->stop) return;
+  const T alpha = (T)(nfin > 0 ? fin_alpha(fin, nfin, S, blockIdx.x == 0, sh) : S->alpha);
   int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= ncv) return;
-  const T alpha = (T)S->alpha;
   T t[NB];
   for (int k = 0; k < NB; k++) {
     size_t o = NB * (size_t)c + k;
@@ -4823,11 +4892,15 @@ __global__ void __launch_bounds__(kBlock) k_s(int ncv, const T *__restrict__ LU,
 // phi += alpha phat + omega shat
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_x(int n5, T *__restrict__ phi, const T *__restrict__ phat,
-                                              const T *__restrict__ shat, const SolverScalars *S) {
+                                              const T *__restrict__ shat, SolverScalars *S,
+                                              const double *__restrict__ fin, int nfin) {
+  __shared__ double sh[32];
   if (S->done || S->stop) return;
+  const T alpha = (T)S->alpha;
+  const T omega = (T)(nfin > 0 ? fin_omega(fin, nfin, nfin, S, blockIdx.x == 0, sh) : S->omega);
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n5) return;
-  phi[k] += (T)S->alpha * phat[k] + (T)S->omega * shat[k];
+  phi[k] += alpha * phat[k] + omega * shat[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -5035,7 +5108,7 @@ void bcg_prologue(const BcgSys &y) {
   const int gb = (ncv + cells_per_block<NB>() - 1) / cells_per_block<NB>();
   hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), bl, 0, y.stream, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi, rhs_, res,
                      res0, y.zero_guess ? (int)kResidZero : (int)kResidFirst, y.partials, y.S);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, y.stream, gb, (int)kFinResid0, y.partials, y.S);
+  hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(gb)), 0, y.stream, gb, (int)kFinResid0, y.partials, y.S);
 }
 
 // count BiCGStab iterations (van der Vorst, UgpWithCv.cpp:2725-2856); each
@@ -5054,6 +5127,7 @@ void bcg_iterations(const BcgSys &y, int count) {
     *vv = (T *)y.v[5], *phat = (T *)y.v[6], *s = (T *)y.v[7], *shat = (T *)y.v[8], *t = (T *)y.v[9];
   const int gb = (ncv + cells_per_block<NB>() - 1) / cells_per_block<NB>();
   hipStream_t st = y.stream;
+  const int nfin = gb <= kFinInline ? gb : 0;
   const bool ilu = y.ilu_sub > 0;
   const int nsub = ilu ? (ncv + y.ilu_sub - 1) / y.ilu_sub : 0;
   auto ilu_solve = [&](const T *r, T *z) {
@@ -5069,31 +5143,35 @@ void bcg_iterations(const BcgSys &y, int count) {
     }
     hipLaunchKernelGGL((k_spmv_dot<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, phat, vv,
                        res0, y.partials, y.S);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, gb, (int)kFinAlpha, y.partials, y.S);
+    if (nfin == 0)
+      hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(gb)), 0, st, gb, (int)kFinAlpha, y.partials, y.S);
     if (ilu) {
-      hipLaunchKernelGGL((k_s<T, NB, false>), dim3(nblk(ncv)), dim3(kBlock), 0, st, ncv, LU, res, vv, s, shat, y.S);
+      hipLaunchKernelGGL((k_s<T, NB, false>), dim3(nblk(ncv)), dim3(kBlock), 0, st, ncv, LU, res, vv, s, shat, y.S,
+                         y.partials, nfin);
       ilu_solve(s, shat);
     } else {
-      hipLaunchKernelGGL((k_s<T, NB>), dim3(nblk(ncv)), dim3(kBlock), 0, st, ncv, LU, res, vv, s, shat, y.S);
+      hipLaunchKernelGGL((k_s<T, NB>), dim3(nblk(ncv)), dim3(kBlock), 0, st, ncv, LU, res, vv, s, shat, y.S,
+                         y.partials, nfin);
     }
     hipLaunchKernelGGL((k_spmv_dot<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, shat, t, s,
                        y.partials, y.S);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, gb, (int)kFinOmega, y.partials, y.S);
+    if (nfin == 0 || y.rec_resid)
+      hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(gb)), 0, st, gb, (int)kFinOmega, y.partials, y.S);
     if (y.rec_resid) {
       hipLaunchKernelGGL((k_x_rec<T, NB>), dim3(nblk(ncv)), dim3(kBlock), 0, st, ncv, LU, phi, phat, shat, s, t, res,
                          res0, y.partials, y.S);
     } else {
-      hipLaunchKernelGGL(k_x<T>, dim3(nblk(n)), dim3(kBlock), 0, st, n, phi, phat, shat, y.S);
+      hipLaunchKernelGGL(k_x<T>, dim3(nblk(n)), dim3(kBlock), 0, st, n, phi, phat, shat, y.S, y.partials, nfin);
       hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi,
                          rhs_, res, res0, (int)kResidIter, y.partials, y.S);
     }
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, y.rec_resid ? nblk(ncv) : gb, (int)kFinResid,
-                       y.partials, y.S);
+    const int gr = y.rec_resid ? nblk(ncv) : gb;
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(gr)), 0, st, gr, (int)kFinResid, y.partials, y.S);
   }
   if (y.confirm) {
     hipLaunchKernelGGL((k_resid<T, NB>), dim3(gb), dim3(kBlock), 0, st, ncv, y.nbocv_i, y.nbocv_v, A, LU, phi, rhs_,
                        res, res0, (int)kResidConfirm, y.partials, y.S);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, st, gb, (int)kFinConfirm, y.partials, y.S);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(gb)), 0, st, gb, (int)kFinConfirm, y.partials, y.S);
   }
 }
 
@@ -5158,15 +5236,7 @@ __global__ void __launch_bounds__(kBlock) kb_ps(const KrylovJob *__restrict__ jo
   SolverScalars *S = (SolverScalars *)J.S;
   if (S->done || S->stop) return;
   double alpha = 0.0;
-  if (which == 1) {  // UgpWithCv.cpp:2775-2782
-    double gamma = fin_slot_v(partials + J.b5, J.nb5, kSum, sh);
-    if (fabs(gamma) < 1.0E-20) gamma = 1.0E-20;
-    alpha = S->rho / gamma;
-    if ((int)blockIdx.x == J.b1 && threadIdx.x == 0) {
-      S->gamma = gamma;
-      S->alpha = alpha;
-    }
-  }
+  if (which == 1) alpha = fin_alpha(partials + J.b5, J.nb5, S, (int)blockIdx.x == J.b1, sh);
   const int c = (blockIdx.x - J.b1) * blockDim.x + threadIdx.x;
   if (c >= J.ncv) return;
   const T *res = (const T *)J.v[2], *vv = (const T *)J.v[5], *LU = (const T *)J.LU;
@@ -5228,10 +5298,7 @@ __global__ void __launch_bounds__(kBlock) kb_x_rec(const KrylovJob *__restrict__
   const KrylovJob &J = jobs[map1[blockIdx.x]];
   SolverScalars *S = (SolverScalars *)J.S;
   if (S->done || S->stop) return;
-  const double st = fin_slot_v(partials + J.b5, J.nb5, kSum, sh);  // UgpWithCv.cpp:2808-2810
-  const double tt = fin_slot_v(partials + J.b5 + grid5, J.nb5, kSum, sh);
-  const double omega = st / (tt + 1.0E-20);
-  if ((int)blockIdx.x == J.b1 && threadIdx.x == 0) S->omega = omega;
+  const double omega = fin_omega(partials + J.b5, J.nb5, grid5, S, (int)blockIdx.x == J.b1, sh);
   __syncthreads();
   if (!J.rec) {
     const int c = (blockIdx.x - J.b1) * blockDim.x + threadIdx.x;
@@ -5253,7 +5320,7 @@ __global__ void __launch_bounds__(kBlock) kb_x_rec(const KrylovJob *__restrict__
 __global__ void __launch_bounds__(kFinBlock) kb_fin(const KrylovJob *__restrict__ jobs, int op,
                                                     const double *__restrict__ partials, int grid5,
                                                     const double *__restrict__ partials1, int grid1) {
-  __shared__ double sh[16];
+  __shared__ double sh[kFinShared];
   const KrylovJob &J = jobs[blockIdx.x];
   if (op == kFinResid && J.rec)
     fin_body(J.nb1, op, partials1 + J.b1, (size_t)grid1, (SolverScalars *)J.S, sh);
@@ -5411,7 +5478,7 @@ __global__ void ks_publish(const StepJob *__restrict__ jobs) {
 
 // k_fin of each solve's partials of one launch shape
 __global__ void __launch_bounds__(kFinBlock) ks_fin(const StepJob *__restrict__ jobs, int op, int shape) {
-  __shared__ double sh[16];
+  __shared__ double sh[kFinShared];
   const StepJob &J = jobs[blockIdx.x];
   fin_body(J.n[shape], op, J.partials, (size_t)J.n[shape], J.scal, sh);
 }
@@ -7559,9 +7626,9 @@ void Ctx::Impl::launch_dt_fin() {
   if (nb > 4 * kMinPre) {
     const int nb2 = (nb + kMinPre - 1) / kMinPre;
     hipLaunchKernelGGL(k_min_pre, dim3(nb2), dim3(256), 0, stream, partials.p, nb, partials.p + nb);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb2, (int)kFinDt, partials.p + nb, scal.p);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb2)), 0, stream, nb2, (int)kFinDt, partials.p + nb, scal.p);
   } else {
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinDt, partials.p, scal.p);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinDt, partials.p, scal.p);
   }
 }
 
@@ -7742,7 +7809,7 @@ void Ctx::Impl::scalar_step(const T *dq) {
   const int nb = nblk(ncv);
   hipLaunchKernelGGL(k_sc_resid, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, AS.p, x, b, res, res0, 1, partials.p,
                      scal_s.p);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinResid0J, partials.p, scal_s.p);
+  hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinResid0J, partials.p, scal_s.p);
   const int max_it = kSaMaxIter + 1;
   int launched = 0;
   while (launched < max_it) {
@@ -7751,15 +7818,15 @@ void Ctx::Impl::scalar_step(const T *dq) {
       hipLaunchKernelGGL(k_sc_p, g, bl, 0, stream, ncv, nbocv_i.p, AS.p, res, vv, p, phat, scal_s.p);
       hipLaunchKernelGGL(k_sc_spmv_dot, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, AS.p, phat, vv, res0, partials.p,
                          scal_s.p);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinAlpha, partials.p, scal_s.p);
+      hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinAlpha, partials.p, scal_s.p);
       hipLaunchKernelGGL(k_sc_s, g, bl, 0, stream, ncv, nbocv_i.p, AS.p, res, vv, sv, shat, scal_s.p);
       hipLaunchKernelGGL(k_sc_spmv_dot, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, AS.p, shat, tv, sv, partials.p,
                          scal_s.p);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinOmega, partials.p, scal_s.p);
+      hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinOmega, partials.p, scal_s.p);
       hipLaunchKernelGGL(k_sc_x, g, bl, 0, stream, ncv, x, phat, shat, scal_s.p);
       hipLaunchKernelGGL(k_sc_resid, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, AS.p, x, b, res, res0, 0,
                          partials.p, scal_s.p);
-      hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinResid, partials.p, scal_s.p);
+      hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinResid, partials.p, scal_s.p);
     }
     launched += chunk;
     HIPCHECK(hipMemcpyAsync(h_scal_s, scal_s.p, sizeof(SolverScalars), hipMemcpyDeviceToHost, stream));
@@ -7792,7 +7859,7 @@ void Ctx::Impl::sst_scalar_step(const T *dq) {
                        kSstPhiZeroRel, 0);
     hipLaunchKernelGGL(k_sc_resid, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, as, x, b, res, res0, 1, partials.p,
                        scal_s.p);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinResid0J, partials.p, scal_s.p);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinResid0J, partials.p, scal_s.p);
     const int max_it = kSstMaxIter + 1;
     int launched = 0;
     while (launched < max_it) {
@@ -7801,15 +7868,15 @@ void Ctx::Impl::sst_scalar_step(const T *dq) {
         hipLaunchKernelGGL(k_sc_p, g, bl, 0, stream, ncv, nbocv_i.p, as, res, vv, p, phat, scal_s.p);
         hipLaunchKernelGGL(k_sc_spmv_dot, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, as, phat, vv, res0, partials.p,
                            scal_s.p);
-        hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinAlpha, partials.p, scal_s.p);
+        hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinAlpha, partials.p, scal_s.p);
         hipLaunchKernelGGL(k_sc_s, g, bl, 0, stream, ncv, nbocv_i.p, as, res, vv, sv, shat, scal_s.p);
         hipLaunchKernelGGL(k_sc_spmv_dot, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, as, shat, tv, sv, partials.p,
                            scal_s.p);
-        hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinOmega, partials.p, scal_s.p);
+        hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinOmega, partials.p, scal_s.p);
         hipLaunchKernelGGL(k_sc_x, g, bl, 0, stream, ncv, x, phat, shat, scal_s.p);
         hipLaunchKernelGGL(k_sc_resid, g, bl, 0, stream, ncv, nbocv_i.p, nbocv_v.p, as, x, b, res, res0, 0,
                            partials.p, scal_s.p);
-        hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nb, (int)kFinResid, partials.p, scal_s.p);
+        hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nb)), 0, stream, nb, (int)kFinResid, partials.p, scal_s.p);
       }
       launched += chunk;
       HIPCHECK(hipMemcpyAsync(h_scal_s, scal_s.p, sizeof(SolverScalars), hipMemcpyDeviceToHost, stream));
@@ -7956,7 +8023,8 @@ void Ctx::Impl::enqueue_step_tail() {
   hipLaunchKernelGGL(k_update<T>, dim3(nblk(ncv)), dim3(kBlock), 0, stream, ncv, q.p, v[1].p);
   launch_state_bc();
   hipLaunchKernelGGL(k_l1, dim3(nblk(ncv)), dim3(kBlock), 0, stream, ncv, rhs.p, partials.p);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nblk(ncv), (int)kFinL1, partials.p, scal.p);
+  hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nblk(ncv))), 0, stream, nblk(ncv),
+                       (int)kFinL1, partials.p, scal.p);
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, stream, scal.p, mail_d);
 }
 
@@ -8137,20 +8205,24 @@ void Ctx::Impl::update() {
 // residual L1 sums of the step just taken (JoeWithModels.cpp:1119-1136) and its report
 void Ctx::Impl::finish_step(StepInfo &info, int it, int st) {
   hipLaunchKernelGGL(k_l1, dim3(nblk(ncv)), dim3(kBlock), 0, stream, ncv, rhs.p, partials.p);
-  hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nblk(ncv), (int)kFinL1, partials.p, scal.p);
+  hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nblk(ncv))), 0, stream, nblk(ncv),
+                       (int)kFinL1, partials.p, scal.p);
   if (par.sa) {
     // the segregated loop reports the scalar residual over the mean-flow
     // relaxation (JoeWithModels.cpp:1132-1134), the coupled loop as it is (:4443-4453)
     hipLaunchKernelGGL(k_l1s, dim3(nblk(ncv)), dim3(kBlock), 0, stream, ncv, rhs_s.p,
                        coupled_sa() ? 1.0 : par.under_relax, partials.p);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nblk(ncv), (int)kFinL1S, partials.p, scal.p);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nblk(ncv))), 0, stream, nblk(ncv),
+                       (int)kFinL1S, partials.p, scal.p);
   }
   if (par.sst) {  // kine's and omega's residuals over the mean-flow relaxation (:1132-1134)
     hipLaunchKernelGGL(k_l1s, dim3(nblk(ncv)), dim3(kBlock), 0, stream, ncv, rhs_s.p, par.under_relax, partials.p);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nblk(ncv), (int)kFinL1S, partials.p, scal.p);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nblk(ncv))), 0, stream, nblk(ncv),
+                       (int)kFinL1S, partials.p, scal.p);
     hipLaunchKernelGGL(k_l1s, dim3(nblk(ncv)), dim3(kBlock), 0, stream, ncv, rhs_s.p + ncv, par.under_relax,
                        partials.p);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(kFinBlock), 0, stream, nblk(ncv), (int)kFinL1S2, partials.p, scal.p);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(fin_threads(nblk(ncv))), 0, stream, nblk(ncv),
+                       (int)kFinL1S2, partials.p, scal.p);
   }
   HIPCHECK(hipMemcpyAsync(h_scal, scal.p, sizeof(SolverScalars), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));

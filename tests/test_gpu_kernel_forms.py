@@ -47,10 +47,11 @@ def test_jacobian_per_entry_equals_per_cell(n, frac, precision, scheme, kind):
 
 # the block BiCGStab against its own stop test: 1 cell .. several blocks of
 # either launch shape with the true residual, and on both sides of the size
-# from which it takes the recurrence's and confirms it (14k cells); a zero and
-# a near guess, tolerances it reaches and one it cannot
+# from which it takes the recurrence's and confirms it (14k cells); its sums
+# finished from 256 and 257 partials (13056 cells, one more), 1024 and 1025
+# (52224); a zero and a near guess, tolerances it reaches and one it cannot
 @pytest.mark.parametrize("dims", [(1, 1, 1), (2, 1, 1), (7, 3, 2), (4, 13, 1), (8, 8, 8), (23, 23, 23), (25, 25, 25),
-                                  (3, 71, 73)])
+                                  (3, 71, 73), (64, 12, 17), (7, 7, 267), (64, 24, 34), (11, 47, 102)])
 def test_block_solver_true_residual_at_the_stop(dims):
     print(f"block solver {dims}", flush=True)
     n = int(np.prod(dims))
