@@ -6164,7 +6164,12 @@ struct Ctx::Impl {
   bool grad_tiled() const {
     return par.grad_kernel == kResidCell && !par.grad_thread_sorted && !dup_blocks;
   }
-  bool flux_tiled() const { return par.flux_kernel == kResidEntry && !dp.visc; }
+  // From two tiles per compute unit (about 36k cells). Below that the chip is
+  // not full and a launch is as long as one block's chain of loads, which is
+  // longer in k_flux_t. A residual by tiles against by entry, us: first order
+  // 3.3k cells 16.8, 15.5; 13k 16.9, 16.5; 107k 31.8, 38.5; second order 3.3k
+  // 28.9, 27.7; 5.9k 27.4, 26.1.
+  bool flux_tiled() const { return par.flux_kernel == kResidEntry && !dp.visc && ntile >= 512; }
   bool face_form() const { return par.flux_kernel == kResidFace && !dp.visc; }
   DBuf<int> counters;  // [0] negative pressure, [1] first-order fallbacks
   // solver (T = double or float, both allocated lazily)
@@ -7690,13 +7695,25 @@ void Ctx::Impl::launch_flux(hipStream_t s, const double *cfl_dev) {
     }
     return;
   }
-  if (flux_entry()) {  // viscous
+  if (flux_entry()) {  // viscous, or too few cells for tiles
     if (par.sst) {  // HLLC, viscous (the parser requires both)
       if (par.second_order) goe(k_flux_e<kHllc, true, true, true>);
       else goe(k_flux_e<kHllc, false, true, true>);
       return;
     }
-    if (par.second_order) {
+    if (!dp.visc) {
+      if (par.second_order) {
+        if (par.scheme == kRoe) goe(k_flux_e<kRoe, true, false>);
+        else if (par.scheme == kAusm) goe(k_flux_e<kAusm, true, false>);
+        else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, true, false>);
+        else goe(k_flux_e<kHllc, true, false>);
+      } else {
+        if (par.scheme == kRoe) goe(k_flux_e<kRoe, false, false>);
+        else if (par.scheme == kAusm) goe(k_flux_e<kAusm, false, false>);
+        else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, false, false>);
+        else goe(k_flux_e<kHllc, false, false>);
+      }
+    } else if (par.second_order) {
       if (par.scheme == kRoe) goe(k_flux_e<kRoe, true, true>);
       else if (par.scheme == kAusm) goe(k_flux_e<kAusm, true, true>);
       else if (par.scheme == kHllcC) goe(k_flux_e<kHllcC, true, true>);

@@ -128,9 +128,10 @@ def test_gradient_forms_agree(n, frac, grad):
             assert np.array_equal(got[k], ref[k], equal_nan=True), k
 
 
-# the inviscid flux by tiles (every option of it, both time steps) against the
-# per-cell form, and per-face fluxes
-@pytest.mark.parametrize("n,frac", [(1, 0.0), (1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0), (9, 0.5)])
+# the inviscid flux (every option of it, both time steps) against the per-cell
+# form: by entry, and from 512 tiles on (the last three sizes) by tiles
+@pytest.mark.parametrize("n,frac", [(1, 0.0), (1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0), (9, 0.5),
+                                    (36, 0.0), (24, 0.5), (20, 1.0)])
 @pytest.mark.parametrize("scheme", ["HLLC", "ROE", "AUSM"])
 @pytest.mark.parametrize("second", [True, False])
 @pytest.mark.parametrize("extra", ["", "TIME_STEP = SUM_BASED\n", "GRAVITY 0.1 -0.2 0.3\n"])
