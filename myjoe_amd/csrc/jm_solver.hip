@@ -134,8 +134,8 @@ struct SolverScalars {
   double resid_s;  // L1 of the transported scalar's residual (Spalart-Allmaras; SST's kine)
   double resid_s2;  // SST: omega's
   // done: 0 running, 1 converged, 2 iteration limit, 3 the recurrence's
-  // residual has met the stop test and the true residual is to confirm it
-  // (confirm: FP64 block solves)
+  // residual has met the stop test, or the solve is at its last iteration,
+  // and the true residual is to take the test (confirm: FP64 block solves)
   int iter, done, maxiter, confirm;
   double zero_abs, zero_rel;
   // pseudo-time step counter and CFL of the device-driven (graph) step
@@ -3770,13 +3770,15 @@ __device__ void fin_body(int nb, int op, const double *__restrict__ partials, si
         S->done = (op == kFinResid0J && mxv <= S->zero_abs) ? 1 : 0;  // UgpWithCv.cpp:2356-2361
       } else {
         S->res_max = mxv;
-        if ((mxv <= S->zero_abs) || (mxv / (S->res0_max + 1.0E-12) <= S->zero_rel))
-          S->done = op == kFinResid && S->confirm ? 3 : 1;
+        const bool met = (mxv <= S->zero_abs) || (mxv / (S->res0_max + 1.0E-12) <= S->zero_rel);
+        if (op == kFinResid && S->confirm && (met || S->iter + 1 >= S->max_launch))
+          S->done = 3;  // the true residual decides, at the last iteration too
         else
-          S->done = S->iter > S->maxiter ? 2 : 0;
+          S->done = met ? 1 : (S->iter > S->maxiter ? 2 : 0);
       }
-      // the host-polled loop launches at most max_launch iterations; a
-      // device-driven step stops at the same point (iter counts them)
+      // a solve ends after its max_launch - 1 iterations, counted here and not
+      // by launches: those between a stop test that waits for its
+      // confirmation and the end of the chunk do nothing
       if ((op == kFinResid || op == kFinConfirm) && !S->done && S->iter + 1 >= S->max_launch) S->stop = 1;
       if (!S->done) {
         S->iter += 1;
@@ -5176,21 +5178,22 @@ void bcg_iterations(const BcgSys &y, int count) {
 }
 
 // a whole solve, host-polled: the flag is read between chunks (2, then 4
-// iterations) into hs (any host memory: the copy is waited for); iterations
-// past convergence are no-ops, so the chunking does not change the result
+// iterations) into hs (any host memory: the copy is waited for) until the
+// device has set it. Iterations past convergence are no-ops, and a chunk of a
+// solve that goes on does at least one, so the chunking changes neither the
+// result nor where the solve ends
 template <typename T, int NB>
 void bcg_solve(const BcgSys &y, SolverScalars *hs, int &iters, int &status) {
   bcg_prologue<T, NB>(y);
   const int max_it = y.maxiter + 1;
-  int launched = 0;
-  while (launched < max_it) {
-    int chunk = std::min(launched == 0 ? 2 : 4, max_it - launched);
+  for (int launched = 0; max_it > 0;) {
+    const int chunk = std::min(launched == 0 ? 2 : 4, std::max(1, max_it - launched));
     bcg_iterations<T, NB>(y, chunk);
     launched += chunk;
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipMemcpyAsync(hs, y.S, sizeof(SolverScalars), hipMemcpyDeviceToHost, y.stream));
     HIPCHECK(hipStreamSynchronize(y.stream));
-    if (hs->done) break;
+    if (hs->done || hs->stop) break;
   }
   iters = hs->iter;
   status = hs->done;
@@ -7156,16 +7159,18 @@ static void krylov_batch_iterations(hipStream_t st, const KrylovBatchBuf &buf, i
 
 // The batch set up last, with host polling between chunks of iterations: the
 // first chunk is the previous call's count less two (consecutive steps of the
-// same solves take similar counts), then chunks of two. Launches after a
-// solve's stop return at once, so the chunking changes no result.
+// same solves take similar counts), then chunks of two, until every solve has
+// set its flag. Launches after a solve's stop return at once and a chunk does
+// at least one iteration of each that goes on, so the chunking changes
+// neither a result nor where a solve ends.
 void run_krylov_batch(int precision, void *stream, KrylovBatchBuf &buf) {
   if (buf.njobs <= 0) return;
   hipStream_t st = (hipStream_t)stream;
   if (precision == 0) krylov_batch_prologue<double>(st, buf);
   else krylov_batch_prologue<float>(st, buf);
   int launched = 0, chunk = std::max(2, buf.last_launched - 2);
-  while (launched < buf.max_it) {
-    chunk = std::min(chunk, buf.max_it - launched);
+  while (buf.max_it > 0) {
+    chunk = std::min(chunk, std::max(1, buf.max_it - launched));
     if (precision == 0) krylov_batch_iterations<double>(st, buf, chunk);
     else krylov_batch_iterations<float>(st, buf, chunk);
     launched += chunk;

@@ -57,3 +57,44 @@ def test_batched_server_takes_the_recurrence_for_fp32_solves():
     srv.wait(t)
     srv.release(t)
     srv.close()
+
+
+# FP64 solves of 16 MB and more take the recurrence's residual and confirm the
+# stop test on the true one. A tolerance the confirmation passes at once, two
+# near the rounding of the true residual, where the recurrence meets the test
+# and the confirmation fails and the chunk's other launches do nothing, and
+# limits that are reached before: the ordinary step, the graph step and both
+# servers do the same iterations, and a solve that does not converge ends at
+# its limit, not before. (The geometry is scaled so that the solver's absolute
+# guards, 1e-20 beside t.t, lie below the rounding.)
+@pytest.mark.parametrize("max_iter,rel", [(30, 1e-2), (60, 1e-15), (60, 3e-16), (7, 1e-12), (1, 1e-2), (0, 1e-2)])
+def test_confirmed_solves_end_at_the_same_iteration(max_iter, rel):
+    print(f"confirmed solves {max_iter} {rel}", flush=True)
+    n = 3
+    mm, joe = cases.bump_case(240, 80, nsteps=n, ls=f"MAX_ITER={max_iter} ABS_RESID=1.0e-300 REL_RESID={rel}")
+    mm.x_no *= 1e4
+    mesh = joemi.Mesh.from_faces(mm)
+    info, state = [], []
+    for graph in (False, True):
+        s = joemi.Solver(mesh, joe)
+        s.init_uniform()
+        steps = [s.step_graph() if graph else s.step() for _ in range(n)]
+        info.append([(i.lin_iters, i.lin_status, list(i.resid)) for i in steps])
+        state.append(s.state())
+    print(info[0], flush=True)
+    assert info[0] == info[1]
+    for it, st, _ in info[0]:
+        # a solve at its limit has counted one iteration more (limit 0: one is done)
+        assert st == 1 or (st == 0 and it == max_iter + 1) or (st == 2 and max_iter == 0 and it == 1)
+    for batched in (False, True):
+        srv = joemi.Server(1 << 30, 2, batched=batched)
+        t = srv.submit(mesh, joe)
+        srv.wait(t)
+        st, rep = srv.result(t)
+        assert rep.status == joemi.Server.DONE and rep.steps == n and list(rep.resid) == info[0][-1][2]
+        state.append(st)
+        srv.release(t)
+        srv.close()
+    for other in state[1:]:
+        for a, b in zip(state[0], other):
+            assert np.array_equal(a, b)
