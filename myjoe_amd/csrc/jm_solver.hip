@@ -5069,7 +5069,7 @@ struct BcgSys {
   int ilu_sub = 0;
   void *F = nullptr, *Dinv = nullptr;
   // the residual of each iteration by the recurrence s - omega t instead of
-  // rhs - A phi (FP32 solves unless asked otherwise; FP64 solves of
+  // rhs - A phi (unless asked otherwise: FP32 solves, FP64 solves of
   // kRecMinBytes and more); with confirm (FP64) the stop test it meets is
   // taken again on the true residual, so a solve ends on the reference's own
   // criterion
@@ -5874,8 +5874,8 @@ void parse_params(const std::string &joe_in, const Mesh &m, SolverParams &p, std
       throw std::invalid_argument("GPU_GRAD_THREAD_ORDER = " + o + " (SORTED, NATIVE)");
     p.grad_thread_sorted = o == "SORTED";
   }
-  {  // the FP32 BiCGStab's residual: RECURRENCE (s - omega t) or TRUE (rhs - A phi, as the reference);
-     // FP64 solves always take the reference's
+  {  // the BiCGStab's residual: RECURRENCE (s - omega t; FP64: from kRecMinBytes on, the stop
+     // test confirmed on the true residual) or TRUE (rhs - A phi, as the reference)
     const std::string o = pm.str("GPU_KRYLOV_RESIDUAL", "RECURRENCE");
     if (o != "TRUE" && o != "RECURRENCE") throw std::invalid_argument("GPU_KRYLOV_RESIDUAL = " + o + " (TRUE, RECURRENCE)");
     p.krylov_recurrence = o == "RECURRENCE";
@@ -6201,6 +6201,8 @@ struct Ctx::Impl {
   // Spalart-Allmaras scalar (its row and column in every block)
   int nbs = 5;
   bool coupled_sa() const { return nbs == 6; }
+  // whether an FP64 solve takes the recurrence's residual, confirmed at the stop
+  bool confirmed64() const { return par.krylov_recurrence && krylov_rec64(nnz, nbs); }
   // the Jacobian, preconditioner and Krylov vectors of the block system in
   // precision T (nvec work vectors)
   template <typename T>
@@ -7264,7 +7266,7 @@ void StepBatch::set(Ctx *const *ctxs, int n, void *stream) {
     J.cfl_after = d.par.cfl_after;
     J.cfl_interval = d.par.cfl_interval;
     J.ls_maxiter = d.par.ls_maxiter;
-    J.confirm = d.precision == 0 && krylov_rec64(d.nnz, 5);
+    J.confirm = d.precision == 0 && d.confirmed64();
     // the grids of the solve's own launches (launch_grad, launch_flux,
     // launch_jac, launch_state_bc)
     const bool grad = d.par.second_order || d.dp.visc;
@@ -7445,7 +7447,7 @@ void Ctx::batch_job(KrylovJob &job) {
   Impl &d = *d_;
   job.ncv = d.ncv;
   job.maxiter = d.par.ls_maxiter;
-  job.confirm = d.precision == 0 && krylov_rec64(d.nnz, 5);
+  job.confirm = d.precision == 0 && d.confirmed64();
   job.rec = d.precision != 0 || job.confirm;  // FP32 solves: the server takes no other form
   job.nbocv_i = d.nbocv_i.p;
   job.nbocv_v = d.nbocv_v.p;
@@ -7984,7 +7986,7 @@ BcgSys Ctx::Impl::bcg_sys() {
   y.partials = partials.p;
   y.S = scal.p;
   y.stream = stream;
-  y.confirm = std::is_same<T, double>::value && krylov_rec64(nnz, nbs);
+  y.confirm = std::is_same<T, double>::value && confirmed64();
   y.rec_resid = y.confirm || (par.krylov_recurrence && !std::is_same<T, double>::value);
   y.zero_guess = true;  // the Jacobian kernels (or k_time_term) leave phi = 0 with the right-hand side
   if (par.ilu_sub > 0) {

@@ -1,10 +1,11 @@
-"""The FP32 BiCGStab's residual by its recurrence (GPU_KRYLOV_RESIDUAL =
-RECURRENCE, the default for FP32 solves): r = s - omega t, where the
-reference recomputes rhs - A phi every iteration (UgpWithCv.cpp:2812-2846),
-one product with A fewer per iteration. It changes the linear solves' path
-only: a mixed-precision steady solve reaches the same steady state as with
-the true residual (GPU_KRYLOV_RESIDUAL = TRUE), and the FP64 solve, which
-always takes the reference's form, is not affected by the key."""
+"""The BiCGStab's residual by its recurrence (GPU_KRYLOV_RESIDUAL =
+RECURRENCE, the default): r = s - omega t, where the reference recomputes
+rhs - A phi every iteration (UgpWithCv.cpp:2812-2846), one product with A
+fewer per iteration. It changes the linear solves' path only: a
+mixed-precision steady solve reaches the same steady state as with the true
+residual (GPU_KRYLOV_RESIDUAL = TRUE). FP64 solves take it from 16 MB of A on
+and confirm the stop test on the true residual; smaller ones take the
+reference's form whatever the key says."""
 import numpy as np
 import pytest
 
@@ -31,6 +32,7 @@ def test_recurrence_residual_reaches_the_same_steady_state():
 
 
 def test_recurrence_key_leaves_the_fp64_solve_alone():
+    # 192 cells: below the size from which FP64 solves take the recurrence
     mm, joe = cases.bump_case(24, 8, nsteps=5)
     mesh = joemi.Mesh.from_faces(mm)
     out = []
@@ -45,8 +47,7 @@ def test_recurrence_key_leaves_the_fp64_solve_alone():
 
 def test_batched_server_takes_the_recurrence_for_fp32_solves():
     # the batched FP32 BiCGStab takes the recurrence: a mixed request asking
-    # for the true residual is refused; FP64 requests take the true residual
-    # whatever the key says
+    # for the true residual is refused, an FP64 one served
     mm, joe = cases.bump_case(24, 8, nsteps=5)
     mesh = joemi.Mesh.from_faces(mm)
     srv = joemi.Server(1 << 30, 2, batched=True)
@@ -98,3 +99,38 @@ def test_confirmed_solves_end_at_the_same_iteration(max_iter, rel):
     for other in state[1:]:
         for a, b in zip(state[0], other):
             assert np.array_equal(a, b)
+
+
+# above that size the key decides: TRUE is the reference's form in every kind
+# of step, so its iterates part from the recurrence's by rounding (a tolerance
+# that takes some twenty iterations), and only by that
+def test_fp64_solves_take_the_true_residual_when_asked():
+    print("fp64 true residual", flush=True)
+    mm, joe = cases.bump_case(240, 80, nsteps=2, ls="MAX_ITER=60 ABS_RESID=1.0e-300 REL_RESID=1e-11")
+    mm.x_no *= 1e4
+    mesh = joemi.Mesh.from_faces(mm)
+    out = {}
+    for text in (joe + "GPU_KRYLOV_RESIDUAL = TRUE\n", joe):
+        states = []
+        for graph in (False, True):
+            s = joemi.Solver(mesh, text)
+            s.init_uniform()
+            for _ in range(2):
+                info = s.step_graph() if graph else s.step()
+                assert info.lin_status == 1 and info.lin_iters > 10
+            states.append(s.state())
+        srv = joemi.Server(1 << 30, 2, batched=True)
+        t = srv.submit(mesh, text)
+        srv.wait(t)
+        states.append(srv.result(t)[0])
+        srv.release(t)
+        srv.close()
+        for other in states[1:]:
+            for a, b in zip(states[0], other):
+                assert np.array_equal(a, b)
+        out[text] = np.concatenate([np.ravel(x) for x in states[0]])
+    a, b = out.values()
+    d = np.max(np.abs(a - b)) / np.max(np.abs(a))
+    print(f"true against recurrence {d:.1e}", flush=True)
+    # both stop on a true residual 1e-11 below the first
+    assert 0.0 < d <= 1e-10
