@@ -260,6 +260,9 @@ jm_status jm_sync(jm_ctx *c);
  * row), A[nnz][5][5], rhs[ncv][5], phi[ncv][5] (the initial guess in, the
  * solution out). The reference's callers (JoeWithModels::runBackwardEuler via
  * solveCoupledLinSysNS, JoeWithModels.cpp:1026) pass dq = 0 as the guess.
+ * From 13982 cells on the iterations take their residual by its recurrence,
+ * s - omega t, and the stop test it meets is taken again on rhs - A phi;
+ * smaller systems take rhs - A phi throughout, as the reference.
  * Runs on stream (NULL: the default stream) and returns when done; the work
  * space (block LU, eight vectors, partials) is allocated for the call.
  * iters / status (1 converged, 2 hit max_iter) may be NULL. */

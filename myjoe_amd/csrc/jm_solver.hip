@@ -8742,9 +8742,10 @@ int64_t Ctx::get(const std::string &name, double *out) {
 
 // ---------------------------------------------------------------------------
 // solveCvVectorR5Bcgstab (UgpWithCv.cpp:2660-2876) on a 5x5 block system the
-// caller holds on the device, with the same kernels and launch sequence as
-// the context's own linear solve. The work space (block LU, eight vectors,
-// partials, solver scalars) is carved from one device buffer.
+// caller holds on the device, with the kernels of the context's own FP64
+// linear solve (from a guess that need not be zero; which residual the
+// iterations take: bcg_on_workspace). The work space (block LU, eight
+// vectors, partials, solver scalars) is carved from one device buffer.
 // ---------------------------------------------------------------------------
 namespace {
 // doubles of work space a solve of ncv cells takes
@@ -8768,8 +8769,11 @@ BcgSys bcg_on_workspace(const BlockSolve &bs, double *ws, hipStream_t stream) {
   y.A = bs.A;
   y.v[0] = (void *)bs.rhs;
   y.v[1] = bs.phi;
-  // the row pointers are on the device: six blocks a row, a mean of hexahedra
-  // and tetrahedra, stand for A's size
+  // The row pointers are on the device, so the choice of the residual's form
+  // goes by the number of cells: six blocks a row, a mean of hexahedra and
+  // tetrahedra, stand for A's size (13982 cells), where a context counts its
+  // own blocks. Reading their number first took 20 to 30 us more of a call's
+  // 270 to 1040 us (1.4k to 20k cells).
   y.rec_resid = y.confirm = krylov_rec64(6LL * bs.ncv, 5);
   size_t o = 0;
   y.S = (SolverScalars *)(ws + o);  // first, so it keeps the buffer's alignment
