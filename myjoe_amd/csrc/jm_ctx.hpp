@@ -31,6 +31,7 @@ enum CellOrder : int { kOrderNative = 0, kOrderGrouped = 1, kOrderMorton = 2, kO
 // residual kernels: one lane per cell-face entry, one thread per cell, or
 // (inviscid flux only) one thread per internal face plus an entry gather
 enum ResidKernels : int { kResidEntry = 0, kResidCell = 1, kResidFace = 2 };
+enum TileKernels : int { kTilesAuto = 0, kTilesAlways = 1, kTilesNever = 2 };
 
 // Parameters of UgpWithCvCompFlow::init / runBackwardEuler read from Joe.in.
 struct SolverParams {
@@ -71,6 +72,7 @@ struct SolverParams {
   int ilu_sub = 0;
   // the per-cell gradient's lanes take a tile's cells by face count (GPU_GRAD_THREAD_ORDER)
   bool grad_thread_sorted = false;
+  int tiles = kTilesAuto;  // GPU_TILE_KERNELS
   // the BiCGStab's residual by the recurrence s - omega t (GPU_KRYLOV_RESIDUAL = RECURRENCE;
   // FP64 solves large enough only)
   bool krylov_recurrence = true;
@@ -203,7 +205,9 @@ struct StepInfo {
 
 class Ctx {
  public:
-  Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream);
+  // batched: for a batched server (batch_prepare and what follows it): it does
+  // not make what only a step of its own reads
+  Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream, bool batched = false);
   ~Ctx();
   Ctx(const Ctx &) = delete;
   Ctx &operator=(const Ctx &) = delete;

@@ -203,7 +203,7 @@ void Server::admit_loop() {
       std::lock_guard<std::mutex> hg(hip_mu_);
       if (hipStreamCreateWithFlags(&a.stream, hipStreamNonBlocking) != hipSuccess)
         throw std::runtime_error("HIP stream creation failed");
-      a.ctx.reset(new Ctx(*r->mesh, r->joe_in, r->precision, a.stream));
+      a.ctx.reset(new Ctx(*r->mesh, r->joe_in, r->precision, a.stream, batched_));
       if (r->init.empty()) {
         a.ctx->init_uniform();
       } else {

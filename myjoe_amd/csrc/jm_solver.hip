@@ -164,6 +164,32 @@ constexpr int kTileEval = kBlock, kTileCells = 80, kTileRows = 188, kTileEnt = 4
 // a cell in DMesh::tcell: {cell of the tile | entries << 8 | first entry << 16,
 // first LS coefficient | internal entries << 16}
 constexpr unsigned kNoRow = 0xffff, kNoEntry = 0xffff;
+
+// From which size a context takes the tile forms (GPU_TILE_KERNELS = AUTO).
+// The flux: from two tiles per compute unit on (33k hexahedra, 41k
+// tetrahedra). Below that the chip is not full and a launch is as long as one
+// block's chain of loads, which is longer in k_flux_t. HLLC by entry and by
+// tiles, us: 18k hexahedra 9.0, 9.0; 39k 13.6, 11.2; 512k 122, 86; 25k
+// tetrahedra 8.5, 8.9; 48k 11.5, 11.0; 511k 75, 63.
+constexpr int kTileMinFlux = 512;
+// The gradient: k_grad's wavefronts loop as long as their longest cell, so a
+// mesh whose cells all have as many faces keeps it up to larger sizes; a
+// Green-Gauss entry has five coefficients to stage where a least-squares one
+// has three, a viscous gradient one field more to share a row among. k_grad
+// and k_grad_t, us, least squares: mixed 20k cells 8.8, 9.4; 28k 10.7, 10.2;
+// 223k 43.7, 33.5; hexahedra 85k 16.6, 17.5; 176k 30.0, 28.8; 2M 435, 285;
+// tetrahedra 197k 24.9, 24.7. Green-Gauss: mixed 37k 11.9, 12.1; 78k 20.7,
+// 18.6; hexahedra 176k 33.3, 38.4; 512k 126, 116; tetrahedra 511k 66, 72;
+// 1.3M 228, 205. Viscous (with k_face_visc): mixed 9k 12.4, 12.8; 14k 13.9,
+// 13.1; hexahedra 39k 17.2, 17.0; 85k 32.5, 30.9; 176k 51.6, 47.5;
+// tetrahedra 105k 27.3, 29.1; 197k 42.0, 39.7; Green-Gauss, hexahedra 85k
+// 33.4, 34.9; 176k 56.3, 53.5; tetrahedra 197k 44.9, 44.2.
+inline int tile_min_grad(bool uniform, bool ls, bool visc) {
+  if (!uniform) return (ls ? 24000 : 40000) / (visc ? 2 : 1);
+  return ls ? 150000 : (visc ? 200000 : 500000);
+}
+// smaller meshes are not cut into tiles at all
+constexpr int kTileMinCells = 16384;
 constexpr int kRedSlots = 8;  // partial-sum slots per block for fused reductions
 inline int nblk(long long n, int b = kBlock) { return (int)((n + b - 1) / b); }
 
@@ -421,9 +447,10 @@ __device__ __forceinline__ double bj_face(double alfa, double phi, double phifa,
 // values of each neighbour's row, the coefficient and offset of an entry is
 // one address for all of them, and each lane keeps only its own field's
 // gradient and bounds (44 registers; a thread holding all fields needed 120).
-// The batched server's form, and of meshes with duplicate neighbour pairs; a
-// solve of its own takes k_grad_t. 5.9k cells: 23 us with a thread per cell,
-// 10 so; 3.1M cells: 614 and 670, bound by the vector memory unit.
+// The batched server's form, and that of smaller meshes (tile_min_grad); a
+// larger solve of its own takes k_grad_t.
+// 5.9k cells: 23 us with a thread per cell, 7.5 so; 3.1M cells: 614 and 670,
+// bound by the vector memory unit.
 // ---------------------------------------------------------------------------
 // enthalpy of a cell state (calcStateVariables: T = p / (rho R),
 // h = gamma R / (gamma - 1) T; UgpWithCvCompFlow.h:1680-1690)
@@ -5874,6 +5901,13 @@ void parse_params(const std::string &joe_in, const Mesh &m, SolverParams &p, std
       throw std::invalid_argument("GPU_GRAD_THREAD_ORDER = " + o + " (SORTED, NATIVE)");
     p.grad_thread_sorted = o == "SORTED";
   }
+  {  // the tile forms of the per-cell gradient and of the inviscid per-entry flux (this build's
+     // option; results do not depend on it): by size, or wherever the mesh and the other options allow
+    const std::string o = pm.str("GPU_TILE_KERNELS", "AUTO");
+    if (o != "AUTO" && o != "ALWAYS" && o != "NEVER")
+      throw std::invalid_argument("GPU_TILE_KERNELS = " + o + " (AUTO, ALWAYS, NEVER)");
+    p.tiles = o == "AUTO" ? kTilesAuto : (o == "ALWAYS" ? kTilesAlways : kTilesNever);
+  }
   {  // the BiCGStab's residual: RECURRENCE (s - omega t; FP64: from kRecMinBytes on, the stop
      // test confirmed on the true residual) or TRUE (rhs - A phi, as the reference)
     const std::string o = pm.str("GPU_KRYLOV_RESIDUAL", "RECURRENCE");
@@ -6145,7 +6179,10 @@ struct Ctx::Impl {
   std::vector<int> fnew;              // reference face -> device face
   std::vector<int> h_dev_nbocv_i, h_ref_nbocv_i;
   bool dup_blocks = false;
-  int min_faces = 1 << 30;  // fewest faces of a cell
+  int min_faces = 1 << 30, max_faces = 0;  // fewest and most faces of a cell
+  // every row of nbocv is the cell and one neighbour per internal face
+  // (duplicate pairs included), as the reference builds it
+  bool rows_by_face = true;
   // the per-entry Jacobian kernel: needs no duplicate neighbour pairs (their
   // shared block is accumulated in entry order by k_jac) and at least four
   // faces per cell (its lanes own at most seven components of a block)
@@ -6157,22 +6194,12 @@ struct Ctx::Impl {
   DBuf<double> muf;    // [nfa][2] the faces' viscosities (k_face_visc)
   DBuf<double> gg;     // [entries][5] Green-Gauss coefficients
   int nent = 0;        // cell-face entries
-  // tiles of the gradient and inviscid flux kernels (DMesh)
+  // tiles of the gradient and inviscid flux kernels (DMesh), and whether this
+  // context runs those forms (build_tiles)
   int ntile = 0;
   DBuf<char> tiles;
-  const unsigned *eval_packed = nullptr;
+  bool grad_tiled = false, flux_tiled = false;
   DBuf<double> fflux;  // [nfa_i][5] face fluxes of the face form
-  // the tile forms (build_tiles) of the gradient and the inviscid flux
-  // (a duplicate neighbour pair has fewer coefficients than entries)
-  bool grad_tiled() const {
-    return par.grad_kernel == kResidCell && !par.grad_thread_sorted && !dup_blocks;
-  }
-  // From two tiles per compute unit (about 36k cells). Below that the chip is
-  // not full and a launch is as long as one block's chain of loads, which is
-  // longer in k_flux_t. A residual by tiles against by entry, us: first order
-  // 3.3k cells 16.8, 15.5; 13k 16.9, 16.5; 107k 31.8, 38.5; second order 3.3k
-  // 28.9, 27.7; 5.9k 27.4, 26.1.
-  bool flux_tiled() const { return par.flux_kernel == kResidEntry && !dp.visc && ntile >= 512; }
   bool face_form() const { return par.flux_kernel == kResidFace && !dp.visc; }
   DBuf<int> counters;  // [0] negative pressure, [1] first-order fallbacks
   // solver (T = double or float, both allocated lazily)
@@ -6248,7 +6275,8 @@ struct Ctx::Impl {
   template <typename T>
   void enqueue_step_tail();
   hipGraphExec_t capture(void (Ctx::Impl::*enq)());
-  void build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf);
+  void build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf, bool batched, DBuf<char> &setup,
+                   const unsigned *&packed);
   hipStream_t cap_stream = nullptr;
   hipGraphExec_t g_head = nullptr, g_chunk = nullptr, g_tail = nullptr;
   int dev_phase = 0;  // 1: head or chunk in flight, 2: tail in flight
@@ -6316,18 +6344,23 @@ static uint64_t morton3(double x, double y, double z) {
 }
 
 // Cuts the device-ordered cells (ci, cf: their entries) into tiles within the
-// limits above, in order, and lists what each tile's kernels need.
-void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf) {
+// limits above, in order, and lists what the tile kernels that this context
+// runs need; none for a context that runs none (a batched solve's kernels are
+// per cell and per entry). setup holds what k_tile_eval reads: the packed
+// evaluations, and the neighbours' rows if no kernel keeps them.
+void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf, bool batched, DBuf<char> &setup,
+                            const unsigned *&packed) {
+  const bool any = par.tiles == kTilesAlways;
+  if (batched || par.tiles == kTilesNever || (!any && ncv < kTileMinCells)) return;
+  const bool visc = par.mu_ref > 0.0;
+  // (a tile has room for one least-squares coefficient per cell and entry)
+  grad_tiled = (par.second_order || visc) && par.grad_kernel == kResidCell && (rows_by_face || !par.grad_ls) &&
+               (any || ncv >= tile_min_grad(min_faces == max_faces, par.grad_ls, visc));
+  flux_tiled = par.flux_kernel == kResidEntry && !visc;
+  if (!grad_tiled && !flux_tiled) return;
   std::vector<Tile> tl;
-  std::vector<int> hl;
-  std::vector<unsigned short> ln(std::max<size_t>(1, cf.size()));
-  std::vector<unsigned> ev;  // entry | other entry << 16
-  std::vector<uint2> tcl(std::max(1, ncv));
-  hl.reserve(ncv);
-  ev.reserve(cf.size() * 7 / 10 + 16);
-  std::vector<int> stamp(ncv, -1), hrow(ncv), fent(std::max(1, nfa), -1);
-  int c0 = 0;
-  while (c0 < ncv) {
+  std::vector<int> stamp(ncv, -1);
+  for (int c0 = 0; c0 < ncv;) {
     const int t = (int)tl.size();
     int c1 = c0, nev = 0, nh = 0;
     for (; c1 < ncv && c1 - c0 < kTileCells && ci[c1 + 1] - ci[c0] <= kTileEnt; c1++) {
@@ -6345,23 +6378,43 @@ void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> 
       nh += dh;
     }
     if (c1 == c0) c1 = c0 + 1;  // one cell alone (at most 64 faces) always fits
-    const std::vector<int> &ki = h_dev_nbocv_i;
-    Tile T{c0, c1 - c0, (int)hl.size(), 0, ci[c0], ci[c1] - ci[c0], ki[c0], ki[c1] - ki[c0], (int)ev.size(), 0, 0, 0};
+    Tile T{};
+    T.c0 = c0;
+    T.nc = c1 - c0;
+    tl.push_back(T);
+    c0 = c1;
+  }
+  if (!any && (int)tl.size() < kTileMinFlux) flux_tiled = false;
+  if (!grad_tiled && !flux_tiled) return;
+  ntile = (int)tl.size();
+  std::vector<int> hl, hrow(ncv), fent;
+  std::vector<unsigned short> ln(std::max<size_t>(1, cf.size()));
+  std::vector<unsigned> ev;  // entry | other entry << 16
+  std::vector<uint2> tcl;
+  hl.reserve(ncv);
+  if (flux_tiled) {
+    ev.reserve(cf.size() * 7 / 10 + 16);
+    fent.assign(std::max(1, nfa), -1);
+  }
+  if (grad_tiled) tcl.resize(std::max(1, ncv));
+  const std::vector<int> &ki = h_dev_nbocv_i;
+  for (int t = 0; t < ntile; t++) {
+    Tile &T = tl[t];
+    const int c0 = T.c0, c1 = c0 + T.nc;
+    T.h0 = (int)hl.size();
+    T.e0 = ci[c0];
+    T.ne = ci[c1] - ci[c0];
+    T.k0 = ki[c0];
+    T.nk = ki[c1] - ki[c0];
+    T.w0 = (int)ev.size();
     for (int c = c0; c < c1; c++)
       for (int e = ci[c]; e < ci[c + 1]; e++) {
-        const int nb = cf[e].y, f = cf[e].x & 0x7fffffff;
-        const unsigned el = e - T.e0, alone = el | kNoEntry << 16;
+        const int nb = cf[e].y;
+        const bool in = nb >= c0 && nb < c1;
         if (nb < 0) {
           ln[e] = kNoRow;
-          ev.push_back(alone);
-        } else if (nb >= c0 && nb < c1) {
+        } else if (in) {
           ln[e] = (unsigned short)(nb - c0);
-          if (nb > c) {
-            fent[f] = e;
-          } else {  // the face's second entry: evaluated once, from its first side
-            const unsigned l2 = fent[f] - T.e0;
-            ev.push_back(cf[e].x >= 0 ? el | l2 << 16 : l2 | el << 16);
-          }
         } else {
           if (stamp[nb] != -2 - t) {
             stamp[nb] = -2 - t;
@@ -6369,9 +6422,21 @@ void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> 
             hl.push_back(nb);
           }
           ln[e] = (unsigned short)(c1 - c0 + hrow[nb]);
-          ev.push_back(alone);
+        }
+        if (!flux_tiled) continue;
+        const unsigned el = e - T.e0;
+        if (!in) {
+          ev.push_back(el | kNoEntry << 16);
+        } else if (nb > c) {
+          fent[cf[e].x & 0x7fffffff] = e;
+        } else {  // the face's second entry: evaluated once, from its first side
+          const unsigned l2 = fent[cf[e].x & 0x7fffffff] - T.e0;
+          ev.push_back(cf[e].x >= 0 ? el | l2 << 16 : l2 | el << 16);
         }
       }
+    T.nh = (int)hl.size() - T.h0;
+    T.nw = (int)ev.size() - T.w0;
+    if (!grad_tiled) continue;
     // the cells by entry count, so that the lanes of a wavefront that work on
     // one each loop about equally long
     int cnt[66] = {0};
@@ -6384,34 +6449,38 @@ void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> 
       tcl[c0 + cnt[n]++] = make_uint2((unsigned)((c - c0) | n << 8 | (ci[c] - T.e0) << 16),
                                       (unsigned)((ki[c] - T.k0) | ni << 16));
     }
-    T.nh = (int)hl.size() - T.h0;
-    T.nw = (int)ev.size() - T.w0;
-    tl.push_back(T);
-    c0 = c1;
   }
-  ntile = (int)tl.size();
-  // one buffer: headers, cells, halo, neighbours, evaluations
-  size_t at[6] = {0, sizeof(Tile) * tl.size(), sizeof(uint2) * tcl.size(), sizeof(int) * hl.size(),
-                  sizeof(unsigned short) * ln.size(), sizeof(unsigned) * ev.size()};
-  for (int k = 1; k < 6; k++) at[k] = (at[k - 1] + at[k] + 15) & ~(size_t)15;
-  std::vector<char> blob(at[5]);  // what is uploaded; the evaluations' room follows it
+  // one buffer of headers, halo, and what each kernel reads: cells and
+  // neighbours (gradient), room for the evaluations (flux); setup: what only
+  // k_tile_eval reads
+  size_t at[5] = {0, sizeof(Tile) * tl.size(), sizeof(int) * hl.size(), sizeof(uint2) * tcl.size(),
+                  grad_tiled ? sizeof(unsigned short) * ln.size() : 0};
+  for (int k = 1; k < 5; k++) at[k] = (at[k - 1] + at[k] + 15) & ~(size_t)15;
+  std::vector<char> blob(at[4]);  // what is uploaded; the evaluations' room follows it
   auto put = [&](int k, const void *src, size_t bytes) {
     if (bytes) std::memcpy(blob.data() + at[k], src, bytes);
   };
   put(0, tl.data(), sizeof(Tile) * tl.size());
-  put(1, tcl.data(), sizeof(uint2) * tcl.size());
-  put(2, hl.data(), sizeof(int) * hl.size());
-  put(3, ln.data(), sizeof(unsigned short) * ln.size());
-  put(4, ev.data(), sizeof(unsigned) * ev.size());
-  tiles.alloc(at[5] + sizeof(int4) * ev.size());
+  put(1, hl.data(), sizeof(int) * hl.size());
+  put(2, tcl.data(), sizeof(uint2) * tcl.size());
+  if (grad_tiled) put(3, ln.data(), sizeof(unsigned short) * ln.size());
+  tiles.alloc(at[4] + sizeof(int4) * ev.size());
   HIPCHECK(hipMemcpy(tiles.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
   dm.ntile = ntile;
   dm.tile = (const Tile *)(tiles.p + at[0]);
-  dm.tcell = (const uint2 *)(tiles.p + at[1]);
-  dm.halo = (const int *)(tiles.p + at[2]);
+  dm.halo = (const int *)(tiles.p + at[1]);
+  dm.tcell = (const uint2 *)(tiles.p + at[2]);
   dm.lnb = (const unsigned short *)(tiles.p + at[3]);
-  dm.eval = (const int4 *)(tiles.p + at[5]);
-  eval_packed = (const unsigned *)(tiles.p + at[4]);
+  dm.eval = (const int4 *)(tiles.p + at[4]);
+  if (!flux_tiled) return;
+  const size_t nln = grad_tiled ? 0 : sizeof(unsigned short) * ln.size(), nev = sizeof(unsigned) * ev.size();
+  setup.alloc(nev + nln);
+  HIPCHECK(hipMemcpy(setup.p, ev.data(), nev, hipMemcpyHostToDevice));
+  if (nln) {
+    HIPCHECK(hipMemcpy(setup.p + nev, ln.data(), nln, hipMemcpyHostToDevice));
+    dm.lnb = (const unsigned short *)(setup.p + nev);
+  }
+  packed = (const unsigned *)setup.p;
 }
 
 // perm (the identity) ordered by key, equal keys in their order: pairs kept
@@ -6437,8 +6506,10 @@ static void sort_by_key(const std::vector<uint64_t> &key, std::vector<int> &perm
   for (size_t i = 0; i < n; i++) perm[i] = a[i].second;
 }
 
-Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) : d_(new Impl) {
+Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream, bool batched) : d_(new Impl) {
   Impl &d = *d_;
+  DBuf<char> tile_setup;  // until the device is waited for at the end
+  const unsigned *tile_packed = nullptr;
   d.precision = precision;
   d.stream = (hipStream_t)stream;
   parse_params(joe_in, m, d.par, d.zbc);
@@ -6512,6 +6583,8 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
       slot_of.push_back(0);
     }
     d.min_faces = std::min(d.min_faces, (int)cf.size() - ci[c]);
+    d.max_faces = std::max(d.max_faces, (int)cf.size() - ci[c]);
+    if (m.nbocv_i[c + 1] - m.nbocv_i[c] != 1 + (int)fi.size()) d.rows_by_face = false;
   }
   ci[ncv] = (int)cf.size();
   // SST runs the per-entry Jacobian only
@@ -6716,7 +6789,7 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
     d.cfl_noc.upload(noc.data(), noc.size());
     d.cfl_tnoc.alloc(std::max<size_t>(1, dcf.size()));
     d.nent = (int)dcf.size();
-    d.build_tiles(dci, dcf);
+    d.build_tiles(dci, dcf, batched, tile_setup, tile_packed);
   }
   std::vector<int> bcell(std::max(1, nfa_b), 0);
   for (int f = 0; f < nfa_b; f++) bcell[f] = inv[m.cvofa[2 * (size_t)f]];
@@ -6885,8 +6958,8 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
   d.dm.nwave = d.nwave;
   d.dm.foc = d.foc.p;
   d.dm.cell_perm = d.cell_perm.p;
-  if (d.ntile > 0) {
-    hipLaunchKernelGGL(k_tile_eval, dim3(d.ntile), dim3(kBlock), 0, d.stream, d.dm, d.eval_packed,
+  if (d.flux_tiled) {
+    hipLaunchKernelGGL(k_tile_eval, dim3(d.ntile), dim3(kBlock), 0, d.stream, d.dm, tile_packed,
                        const_cast<int4 *>(d.dm.eval));
     HIPCHECK(hipGetLastError());
   }
@@ -6929,6 +7002,7 @@ Ctx::Ctx(const Mesh &m, const std::string &joe_in, int precision, void *stream) 
   d.dp.sst_alfa[1] = 0.0828 / 0.09 - 0.856 * std::pow(0.41, 2.0) / std::sqrt(0.09);
   d.cfl = d.par.cfl;
   HIPCHECK(hipDeviceSynchronize());
+  if (!d.grad_tiled) d.dm.lnb = nullptr;  // in tile_setup
 }
 
 Ctx::~Ctx() {
@@ -7590,7 +7664,7 @@ void Ctx::Impl::launch_grad(hipStream_t s) {
     const dim3 b(64 * kGradWaves);
     if (par.grad_ls) hipLaunchKernelGGL(k_grad_e<true>, g, b, 0, s, dm, dp, prim.p, bfa.p, grad.p);
     else hipLaunchKernelGGL(k_grad_e<false>, g, b, 0, s, dm, dp, prim.p, bfa.p, grad.p);
-  } else if (grad_tiled()) {
+  } else if (grad_tiled) {
     auto got = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(ntile), dim3(kBlock), 0, s, dm, dp, prim.p, bfa.p, grad.p, gradv.p);
     };
@@ -7646,7 +7720,7 @@ void Ctx::Impl::launch_dt_fin() {
 
 int Ctx::Impl::flux_blocks() const {
   if (face_form()) return (nwave + kWaves - 1) / kWaves;  // k_gather_e
-  if (flux_tiled()) return ntile;
+  if (flux_tiled) return ntile;
   return flux_entry() ? (nwave + kFluxWaves - 1) / kFluxWaves : nblk(ncv);
 }
 
@@ -7684,7 +7758,7 @@ void Ctx::Impl::launch_flux(hipStream_t s, const double *cfl_dev) {
     }
     return;
   }
-  if (flux_tiled()) {
+  if (flux_tiled) {
     auto got = [&](auto kern) {
       hipLaunchKernelGGL(kern, g, dim3(kBlock), 0, s, dm, dp, prim.p, grad.p, bfa.p, q.p, rhs.p, counters.p + 1, dta,
                          dt.p, partials.p);

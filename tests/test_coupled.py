@@ -159,20 +159,21 @@ def test_gpu_coupled_matches_reference(fixture):
     print(f"coupled {fixture}", flush=True)
     g = load(fixture)
     mesh = joemi.Mesh.from_faces(MESHES[_mesh_key(fixture).split("_")[0]]())
-    s = joemi.Solver(mesh, joe_text(g))
-    s.set_state(g["RHO"], g["RHOU"], g["RHOE"])
     sa = "_sa" in fixture
-    if sa:
-        s.set_scalar(g["NUSA"])
-    s.calc_rhs(True)
     exact = total = 0
-    for k in FIELDS + (["GRAD_ENTHALPY", "MUL_FA"] if "visc" in fixture else []) + \
-            (SA_DEVICE_FIELDS + ["MUT_FA"] if sa else []):
-        if k not in g:
-            continue
-        e, n = compare(s.get(k), g[k], 1e-12, f"{fixture}:{k}")
-        exact += e
-        total += n
+    for extra in ("", "GPU_TILE_KERNELS = ALWAYS\n"):  # by size, and by tiles
+        s = joemi.Solver(mesh, joe_text(g) + extra)
+        s.set_state(g["RHO"], g["RHOU"], g["RHOE"])
+        if sa:
+            s.set_scalar(g["NUSA"])
+        s.calc_rhs(True)
+        for k in FIELDS + (["GRAD_ENTHALPY", "MUL_FA"] if "visc" in fixture else []) + \
+                (SA_DEVICE_FIELDS + ["MUT_FA"] if sa else []):
+            if k not in g:
+                continue
+            e, n = compare(s.get(k), g[k], 1e-12, f"{fixture}:{extra.strip()}:{k}")
+            exact += e
+            total += n
     print(f"{fixture}: {exact}/{total} bit-exact")
 
 

@@ -135,6 +135,33 @@ def test_cell_kernels_match_reference(fixture):
             compare(s.get(k), g[k], 1e-12, f"cell:{fixture}:{k}")
 
 
+@pytest.mark.parametrize("fixture", RHS_FIXTURES)
+def test_tile_kernels_match_reference(fixture):
+    # meshes of this size take the per-entry flux and the gradient per cell
+    # and field; with the tile forms asked for, the same bits
+    print(f"tile kernels {fixture}", flush=True)
+    g = load("rhs_" + fixture)
+    mesh = joemi.Mesh.from_faces(MESHES[fixture.split("_")[0]]())
+    sa, sst = "_sa" in fixture, "_sst" in fixture
+    fields = (FIELDS + (["GRAD_ENTHALPY", "MUL_FA"] if "visc" in fixture else []) + (SA_GPU_FIELDS if sa else [])
+              + (SST_GPU_FIELDS if sst else []))
+    out = []
+    for tiles in ("ALWAYS", "NEVER"):
+        s = joemi.Solver(mesh, joe_text(g) + f"GPU_TILE_KERNELS = {tiles}\n")
+        s.set_state(g["RHO"], g["RHOU"], g["RHOE"])
+        if sa:
+            s.set_scalar(g["NUSA"])
+        if sst:
+            s.set_scalar(g["KINE"], "kine")
+            s.set_scalar(g["OMEGA"], "omega")
+        s.calc_rhs(True)
+        out.append({k: s.get(k) for k in fields + ["COUNTERS"] if k in g or k == "COUNTERS"})
+    for k, v in out[0].items():
+        assert np.array_equal(v, out[1][k], equal_nan=True), k
+        if k in g:
+            compare(v, g[k], 1e-12, f"tiles:{fixture}:{k}")
+
+
 @pytest.mark.parametrize("fixture", ["bump24_hllc", "box4_hllc_gg", "box4_roe_first", "box4_ausm_alt_ana_gg",
                                      "box4_roe_alt_ana", "box4_hllc_alt_new", "box4_hllc_dtsum"])
 def test_face_flux_form_matches_reference(fixture):

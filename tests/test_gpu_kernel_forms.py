@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 
 from myjoe_amd import cases, joemi
+from oracle.oracle import Oracle
+from tests.helpers import compare
 
 pytestmark = pytest.mark.gpu
 
@@ -113,8 +115,8 @@ def test_sst_rows_per_entry_equal_per_cell(n, frac):
         assert np.array_equal(a[k], b[k], equal_nan=True), k
 
 
-# the gradient per cell and field against the per-entry form and against
-# itself with the cells of a tile in another thread order
+# the gradient per cell and field, the same with the cells in another thread
+# order, and the gradient by tiles, against the per-entry form
 @pytest.mark.parametrize("grad", ["LEASTSQUARES", "GREENGAUSS"])
 @pytest.mark.parametrize("n,frac", [(1, 0.0), (1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0), (9, 0.5)])
 def test_gradient_forms_agree(n, frac, grad):
@@ -122,14 +124,16 @@ def test_gradient_forms_agree(n, frac, grad):
     mesh, joe = box(n, frac, grad=grad)
     names = ["GRAD_RHO", "GRAD_P", "GRAD_U", "ALPHA_RHO", "RHS_RHO", "RHS_RHOU", "RHS_RHOE"]
     ref = values(mesh, joe + "GPU_GRAD_KERNEL = ENTRY\n", names, implicit=False)
-    for keys in ("GPU_GRAD_KERNEL = CELL\n", "GPU_GRAD_KERNEL = CELL\nGPU_GRAD_THREAD_ORDER = SORTED\n"):
+    cell = "GPU_GRAD_KERNEL = CELL\n"
+    for keys in (cell + "GPU_TILE_KERNELS = NEVER\n", cell + "GPU_TILE_KERNELS = ALWAYS\n",
+                 cell + "GPU_TILE_KERNELS = NEVER\nGPU_GRAD_THREAD_ORDER = SORTED\n"):
         got = values(mesh, joe + keys, names, implicit=False)
         for k in names:
             assert np.array_equal(got[k], ref[k], equal_nan=True), k
 
 
-# the inviscid flux (every option of it, both time steps) against the per-cell
-# form: by entry, and from 512 tiles on (the last three sizes) by tiles
+# the inviscid flux (every option of it, both time steps) by entry, by tiles
+# and as the size decides (the last three by tiles) against the per-cell form
 @pytest.mark.parametrize("n,frac", [(1, 0.0), (1, 1.0), (2, 0.5), (3, 0.0), (5, 0.5), (4, 1.0), (9, 0.5),
                                     (36, 0.0), (24, 0.5), (20, 1.0)])
 @pytest.mark.parametrize("scheme", ["HLLC", "ROE", "AUSM"])
@@ -139,10 +143,81 @@ def test_flux_forms_agree(n, frac, scheme, second, extra):
     print(f"flux forms n={n} frac={frac} {scheme} {second} {extra!r}", flush=True)
     mesh, joe = box(n, frac, scheme, second_order=second)
     names = ["RHS_RHO", "RHS_RHOU", "RHS_RHOE", "LOCAL_DT"]
-    a = values(mesh, joe + extra + "GPU_FLUX_KERNEL = ENTRY\n", names, implicit=False)
     b = values(mesh, joe + extra + "GPU_FLUX_KERNEL = CELL\n", names, implicit=False)
-    for k in names:
-        assert np.array_equal(a[k], b[k], equal_nan=True), k
+    for tiles in ("NEVER", "ALWAYS", "AUTO"):
+        a = values(mesh, joe + extra + f"GPU_FLUX_KERNEL = ENTRY\nGPU_TILE_KERNELS = {tiles}\n", names, implicit=False)
+        for k in names:
+            assert np.array_equal(a[k], b[k], equal_nan=True), (tiles, k)
+
+
+def duplicate_pairs(mm, every=5):
+    """Every few internal quadrilaterals as two triangles between the same
+    cells: duplicate neighbour pairs."""
+    nodes, cells, zone, ptr, quads = [], [], [], [0], 0
+    for f in range(mm.nfa):
+        parts = [mm.face_nodes[mm.face_ptr[f]:mm.face_ptr[f + 1]]]
+        if mm.face_cells[f, 1] >= 0 and len(parts[0]) == 4:
+            quads += 1
+            if quads % every == 0:
+                parts = [parts[0][[0, 1, 2]], parts[0][[0, 2, 3]]]
+        for nd in parts:
+            nodes.append(nd)
+            ptr.append(ptr[-1] + len(nd))
+            cells.append(mm.face_cells[f])
+            zone.append(mm.face_zone[f])
+    mm.face_ptr, mm.face_nodes = np.array(ptr, mm.face_ptr.dtype), np.concatenate(nodes).astype(mm.face_nodes.dtype)
+    mm.face_cells, mm.face_zone = np.array(cells, mm.face_cells.dtype), np.array(zone, mm.face_zone.dtype)
+    return mm
+
+
+# the tile forms under every option that reaches them (schemes and the coupled
+# flux, both gradients, viscous runs (gradient only), every SYMM_BC, every
+# boundary kind, duplicate neighbour pairs): the same bits as without tiles
+TILE_FIELDS = ["GRAD_RHO", "GRAD_P", "GRAD_U", "ALPHA_RHO", "RHS_RHO", "RHS_RHOU", "RHS_RHOE", "LOCAL_DT", "FLUX_FA",
+               "COUNTERS"]
+
+
+@pytest.mark.parametrize("n,frac,dup", [(1, 1.0, False), (5, 0.5, False), (13, 0.5, False), (7, 0.0, True),
+                                        (9, 0.3, True)])
+@pytest.mark.parametrize("kind", ["HLLC", "ROE", "AUSM", "coupled", "laminar", "coupled laminar"])
+def test_tile_forms_under_every_option(n, frac, dup, kind):
+    print(f"tile forms n={n} frac={frac} dup={dup} {kind}", flush=True)
+    mm, _ = cases.box_case(n, frac=frac, seed=n)
+    mesh = joemi.Mesh.from_faces(duplicate_pairs(mm) if dup else mm)
+    scheme = kind if kind in ("ROE", "AUSM") else "HLLC"
+    for grad in ("LEASTSQUARES", "GREENGAUSS"):
+        for bcs in (cases.BOX_BCS, cases.BOX_BCS_ALT):
+            for symm in ("ORIGINAL_NUMERIC", "NEW_NUMERIC", "ANALYTICAL"):
+                for second in (True, False):
+                    joe = cases.box_joe_in(scheme, second, grad, bcs=bcs, symm_bc=symm)
+                    if "coupled" in kind:
+                        joe = cases.coupled(joe, keep_symm_bc=True)
+                    names = TILE_FIELDS
+                    if "laminar" in kind:
+                        joe = joe.replace("MU_REF = 0.0", "MU_REF = 0.01\nMU_MODE = POWERLAW\nMU_POWER_LAW = 0.7")
+                        names = names + ["GRAD_ENTHALPY"]
+                    a = values(mesh, joe + "GPU_TILE_KERNELS = ALWAYS\n", names, implicit=False)
+                    b = values(mesh, joe + "GPU_TILE_KERNELS = NEVER\n", names, implicit=False)
+                    for k in names:
+                        assert np.array_equal(a[k], b[k], equal_nan=True), (grad, symm, second, k)
+
+
+def test_duplicate_pairs_match_the_oracle():
+    print("duplicate pairs", flush=True)
+    for grad in ("LEASTSQUARES", "GREENGAUSS"):
+        mm, joe = cases.box_case(5, frac=0.3, seed=2, grad=grad)
+        nfa = mm.nfa
+        mm = duplicate_pairs(mm)
+        assert mm.nfa > nfa
+        mesh = joemi.Mesh.from_faces(mm)
+        o = Oracle(mesh.as_dump(), joe)
+        o.set_state(*cases.random_state(mesh.ncv, 5))
+        o.residual(True)
+        names = TILE_FIELDS[:-1] + ["A"]
+        for tiles in ("ALWAYS", "NEVER"):
+            got = values(mesh, joe + f"GPU_TILE_KERNELS = {tiles}\n", names)
+            for k in names:
+                compare(got[k], o.get(k), 1e-12, f"duplicates:{tiles}:{k}")
 
 
 def morton(x):
