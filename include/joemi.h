@@ -317,8 +317,10 @@ jm_status jm_mesh_quality(const jm_mesh *m, double *min_sdotn, int *neg_subtets)
  * to jm_server_submit must stay alive until the ticket is released. Results
  * are bit-identical to a solve run alone.
  * ------------------------------------------------------------------------- */
-/* device bytes a context for this mesh holds once it has stepped (the
- * server's admission estimate) */
+/* a bound on the device bytes that a context for this mesh holds once it has
+ * stepped, whatever its options but for TURB_MODEL and GPU_PRECONDITIONER =
+ * ILU0, which add to it. The server admits each request by the same count for
+ * the request's own options, so no more than this without those two. */
 jm_status jm_ctx_footprint(const jm_mesh *m, int precision, int64_t *bytes);
 
 typedef struct jm_server jm_server;

@@ -259,9 +259,10 @@ class Ctx {
   void batch_job(KrylovJob &job);
   StepInfo batch_result();
   int precision() const;
-  // device bytes a context for this mesh holds once it has stepped
+  // a bound on the device bytes a context for this mesh holds once it has
+  // stepped: of these options, and of any but a turbulence model's and ILU0's
+  static size_t footprint(const Mesh &m, int precision, const SolverParams &p, bool batched);
   static size_t footprint(const Mesh &m, int precision);
-  static size_t footprint(const Mesh &m, int precision, bool sa);
   int run(int max_steps, double *hist, bool graph = false);
   // doneSolver (JoeWithModels.h:42-95) after a step, plus RESID_ENERG_REL
   bool done_solver(const StepInfo &s);

@@ -117,7 +117,8 @@ int Server::submit(const Mesh *mesh, const std::string &joe_in, int precision, c
   r->mesh = mesh;
   r->joe_in = joe_in;
   r->precision = precision;
-  r->footprint = Ctx::footprint(*mesh, precision);
+  r->footprint = Ctx::footprint(*mesh, precision, p, batched_);
+  r->footprint64 = Ctx::footprint(*mesh, 0, p, batched_);
   if (r->footprint > budget_) throw std::invalid_argument("solve does not fit the server's memory budget");
   if (rho) {
     const size_t n = mesh->ncv;
@@ -271,7 +272,7 @@ bool Server::retry_in_fp64(Active &a, const StepInfo &s) {
   bool finite = true;
   for (int k = 0; k < 5; k++) finite = finite && std::isfinite(s.resid[k]);
   if (finite) return false;
-  const size_t fp = Ctx::footprint(*r->mesh, 0);
+  const size_t fp = r->footprint64;
   if (fp > budget_) return false;  // the FP64 solve could never be admitted
   release_ctx(a);
   std::lock_guard<std::mutex> g(mu_);

@@ -28,7 +28,7 @@ class Server {
     const Mesh *mesh = nullptr;  // owned by the caller until the solve is released
     std::string joe_in;
     int precision = 0;
-    size_t footprint = 0;
+    size_t footprint = 0, footprint64 = 0;  // at its precision, in FP64
     std::vector<double> init;  // optional initial state (rho, rhou[3], rhoE), reference numbering
     int status = kQueued;
     int fp64_retries = 0;     // 1 once a mixed-precision solve that went non-finite was queued again in FP64

@@ -6277,6 +6277,7 @@ struct Ctx::Impl {
   hipGraphExec_t capture(void (Ctx::Impl::*enq)());
   void build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf, bool batched, DBuf<char> &setup,
                    const unsigned *&packed);
+  size_t device_bytes() const;  // in this context's buffers
   hipStream_t cap_stream = nullptr;
   hipGraphExec_t g_head = nullptr, g_chunk = nullptr, g_tail = nullptr;
   int dev_phase = 0;  // 1: head or chunk in flight, 2: tail in flight
@@ -7019,30 +7020,55 @@ Ctx::~Ctx() {
   if (d.h_scal_s) (void)hipHostFree(d.h_scal_s);
 }
 
-// Device bytes a context holds once it has stepped (mesh, state, Jacobian,
-// preconditioner, Krylov vectors, reduction partials).
-size_t Ctx::footprint(const Mesh &m, int precision) {
-  const size_t ncv = m.ncv, nfa = m.nfa, nfa_b = m.nfa_b, nnz = m.nbocv_s();
-  const size_t ent = 2 * (nfa - nfa_b) + nfa_b;
-  const size_t sJ = precision == 0 ? 8 : 4;
+// At least the device bytes that a context of these options holds once it has
+// stepped: what the constructor and ensure_solver allocate (device_bytes
+// counts it), the tiles by a bound. A tile kernel's list entries are counted as
+// if every entry had an evaluation (16 bytes) and a halo cell (4) of its own,
+// beside its neighbour (2); a tile's header (48) goes by the wavefronts, two
+// of which cover more than 64 entries and which are never fewer than the tiles.
+size_t Ctx::footprint(const Mesh &m, int precision, const SolverParams &p, bool batched) {
+  const size_t n = m.ncv, nfa = m.nfa, nfa_b = std::max<size_t>(1, m.nfa_b), nfa_i = m.nfa - m.nfa_b, nnz = m.nbocv_s();
+  const size_t ent = 2 * nfa_i + m.nfa_b, sJ = precision == 0 ? 8 : 4, nb = p.coupled && p.sa ? 6 : 5;
+  const bool visc = p.mu_ref > 0.0, face = p.flux_kernel == kResidFace && !visc, turb = p.sa || p.sst;
   size_t b = 0;
-  b += nfa * (8 + 3) * 8;  // fgeo; fnorm, or without it muf, fcell and cfl_tnoc
-  b += nnz * (3 * 8 + 4) + nfa_b * (3 * 8 + 4 + 4);  // lsg, nbocv_v, bfa_lsg, bfa_cell, bfa_zone
-  b += (ncv + 1) * 4 * 2 + ncv * 4;                // cfl_i, nbocv_i, wave table
-  b += ent * (8 + 4 + 8 + 24);                     // entries, their blocks, their cells and positions, limiter offsets
-  b += ncv * (5 + 8 + 16 + 5 + 1 + 1) * 8;         // q, prim, grad, rhs, dt, vol
-  b += nfa_b * (8 + 5) * 8;                        // bfa, hook
-  b += (nnz + ncv) * 25 * sJ + 10 * ncv * 5 * sJ;  // A, LU, Krylov vectors
-  b += 8 * ((size_t)nblk(5 * (long long)ncv) + 64) * 8;
+  b += nfa * 8 * 8 + (!p.grad_ls || turb ? nfa * 3 * 8 : 0);       // fgeo, fnorm
+  b += nnz * (24 + 4) + nfa_b * (24 + 4 + 4) + n * 8;              // lsg, nbocv_v; bfa_lsg, bfa_cell, bfa_zone; vol
+  b += 3 * (n + 1) * 4 + (p.grad_thread_sorted ? n * 4 : 0);       // cfl_i, nbocv_i, wave_e0; cell_perm
+  b += ent * (8 + 8 + 4 + 4 + 24);                                 // cfl_e, ecp, cfl_noc, cfl_tnoc, cfl_r0
+  b += (turb || p.dt_sum ? ent * 4 : 0) + (p.grad_ls ? 0 : ent * 5 * 8);  // foc, gg
+  b += n * (5 + 8 + 16 + 5 + 1) * 8 + nfa_b * (8 + 5) * 8;         // q, prim, grad, rhs, dt; bfa, hook
+  b += visc ? n * 12 * 8 + nfa * 2 * 8 + nfa_i * 8 : 0;            // gradv, muf, fcell
+  b += face ? nfa_i * (8 + 5 * 8) : 0;                             // fcell, fflux
+  if (!batched && p.tiles != kTilesNever && (p.tiles == kTilesAlways || m.ncv >= kTileMinCells))
+    b += n * 8 + ent * (2 + 4 + 2) + (visc ? 0 : ent * 16);        // tcell; lnb, halo, headers; eval
+  b += nb * nb * (nnz + n) * sJ + 10 * nb * n * sJ;                // A, LU, Krylov vectors
+  b += p.ilu_sub > 0 ? nb * nb * (nnz + n) * sJ : 0;               // ILU factors
+  b += 8 * std::max<size_t>(8 * ((size_t)nblk(5 * (long long)n) + 64), n + n / kMinPre + 65);  // partials
+  if (p.sa) b += (2 + kAuxN) * n * 8 + nfa_b * 8 + (p.coupled ? 0 : 6 * nnz * 8 + 10 * n * 8);  // phi, rhs, aux, profile, AS, sw
+  if (p.sst) b += (6 + kSstN + 10) * n * 8 + 2 * nfa_b * 8 + 12 * nnz * 8;  // phi, rhs, dscal, aux, sw, bfa, AS
   return b + (1 << 20);
 }
 
-size_t Ctx::footprint(const Mesh &m, int precision, bool sa) {
-  size_t b = footprint(m, precision);
-  if (sa) {
-    const size_t ncv = m.ncv, nnz = m.nbocv_s(), ent = 2 * (size_t)(m.nfa - m.nfa_b) + m.nfa_b;
-    b += ncv * (1 + kAuxN + 1 + 10) * 8 + nnz * 6 * 8 + ent * 4;  // nuSA, fields, rhs, Krylov, AScal, faocv map
-  }
+// for any options but a turbulence model's and ILU0's
+size_t Ctx::footprint(const Mesh &m, int precision) {
+  SolverParams p;
+  p.mu_ref = 1.0;
+  p.grad_ls = false;
+  p.dt_sum = true;
+  const size_t v = footprint(m, precision, p, false);
+  p.mu_ref = 0.0;
+  return std::max(v, footprint(m, precision, p, false));
+}
+
+size_t Ctx::Impl::device_bytes() const {
+  size_t b = 0;
+  auto add = [&](const auto &x) { b += x.n * sizeof(*x.p); };
+  auto all = [&](const auto &...x) { (add(x), ...); };
+  all(fgeo, fnorm, lsg, bfa_lsg, vol, cfl_i, cfl_noc, cfl_tnoc, nbocv_i, nbocv_v, bfa_cell, bfa_zone, cfl_e, ecp, wave_e0,
+      cfl_r0, zones, q, prim, grad, bfa, rhs, dt, hook, gradv, fcell, muf, gg, tiles, fflux, counters);
+  all(A64, LU64, A32, LU32, F64, Dinv64, F32, Dinv32, partials, scal, sa_phi, sa_aux, sa_prof, rhs_s, AS, sst_phi, sst_aux,
+      sst_bfa, sst_dscal, scal_s, foc, cell_perm, src);
+  for (int k = 0; k < 10; k++) all(v64[k], v32[k], sw[k]);
   return b;
 }
 
@@ -8733,6 +8759,10 @@ int64_t Ctx::get(const std::string &name, double *out) {
     const int k = name == "MUL_FA" ? 0 : 1;
     for (size_t f = 0; f < nf; f++) out[f] = h[2 * (size_t)d.fnew[f] + k];
     return (int64_t)nf;
+  }
+  if (name == "DEVICE_BYTES") {  // that the context's buffers hold now (jm_ctx_footprint bounds it)
+    if (out) out[0] = (double)d.device_bytes();
+    return 1;
   }
   if (name == "COUNTERS") {  // negative pressures, first-order fallbacks
     if (out) {
