@@ -29,19 +29,25 @@ HBM_PEAK_GBS = 8000.0
 METRIC = "steady solves/min + p50/p99 latency vs plain FP64 GPU loop; residual Mcell-it/s"
 
 
-def algorithmic_bytes(ncv, nfa, nfa_b, nnz):
+def algorithmic_bytes(ncv, nfa, nfa_b, nnz, grad_tiles=True, flux_tiles=True):
     """Compulsory HBM bytes of each residual kernel (every array it needs read
-    or written once): prim rows 64 B (rho u v w p x_cv), limited-gradient
-    rows 120 B (+8 alpha), face rows 56 B (unit normal, area, x_fa), boundary
-    rows 40 B (rho u v w p), face-list entries 8 B, LS coefficients 24 B."""
+    or written once): prim rows 64 B (rho u v w p x_cv), gradient rows 128 B
+    (15 and alpha), face rows 56 B (unit normal, area, x_fa), boundary rows
+    40 B (rho u v w p), face-list entries 8 B, LS coefficients and limiter
+    offsets 24 B. By tiles (k_grad_t, k_flux_t): instead of the face-list
+    entries a cell's 8 B and an entry's 2 B in the gradient and 16 B per face
+    in the flux (a face between two tiles has two; those and the halo's rows
+    are not counted)."""
     nfa_i = nfa - nfa_b
     nfoc = 2 * nfa_i + nfa_b
+    grad = ncv * (64 + 8 + 128) + nnz * 24 + nfoc * 24 + nfa_b * (8 + 40 + 24)
+    # fluxes + local time step: + rhou (24 B) and dt (8 B) per cell
+    flux = ncv * (64 + 128 + 4 + 8 + 40 + 24 + 8) + nfa * 56 + nfa_b * 40
     return {
         "k_state": ncv * (40 + 40),
         "k_bc": nfa_b * (64 + 56 + 8 + 56),
-        "k_grad": ncv * (64 + 4 + 4 + 128) + nnz * 24 + nfoc * 8 + nfa_i * 56 + nfa_b * (40 + 24),
-        # fluxes + local time step: + rhou (24 B) and dt (8 B) per cell
-        "k_flux": ncv * (64 + 120 + 4 + 8 + 40 + 24 + 8) + nfoc * 8 + nfa * 56 + nfa_b * 40,
+        "k_grad": grad + nfoc * (2 if grad_tiles else 8),
+        "k_flux": flux + (nfa * 16 if flux_tiles else nfoc * 8),
         # Jacobian assembly, FP64 blocks: A written once, per cell its prim
         # row, entry range, diagonal index; per entry the face entry and the
         # block index; face rows; boundary rows
@@ -548,7 +554,10 @@ def main():
 
     head = args.schemes.split(",")[0]
     kt = kernels[head]
-    ab = algorithmic_bytes(mesh.ncv, mesh.nfa, mesh.nfa_b, mesh.nnz)
+    # by tiles: the default forms on a mesh that is large enough for them
+    tiled = mesh.ncv >= 41000
+    ab = algorithmic_bytes(mesh.ncv, mesh.nfa, mesh.nfa_b, mesh.nnz, tiled and args.grad_kernel != "ENTRY",
+                           tiled and args.flux_kernel in (None, "ENTRY"))
     dom = max(("k_grad", "k_flux", "k_state"), key=lambda k: kt.get(k, 0.0))
     achieved = ab[dom] / (kt[dom] * 1e-3) / 1e9
     resid_bytes = ab["k_state"] + ab["k_bc"] + ab["k_grad"] + ab["k_flux"]

@@ -157,7 +157,8 @@ jm_status jm_calc_rhs(jm_ctx *c, int flags);
  * MUT_FA, each face's laminar and eddy viscosity [nfa] (mul_fa of
  * calcMaterialProperties, UgpWithCvCompFlow.h:1701-1753; mut_fa of
  * calcRansTurbViscMuet, TurbModel_SA.h:74-128, TurbModel_KOMSST.h:100-158), zero when the case is
- * inviscid or has no turbulence model. out may be NULL to query *count. */
+ * inviscid or has no turbulence model. DEVICE_BYTES: what the context's device
+ * buffers hold now. out may be NULL to query *count. */
 jm_status jm_get(jm_ctx *c, const char *name, double *out, int64_t *count);
 
 /* One pass of the runBackwardEuler loop (JoeWithModels.cpp:975-1158): CFL
@@ -167,7 +168,7 @@ jm_status jm_get(jm_ctx *c, const char *name, double *out, int64_t *count);
 typedef struct {
   int step;            /* step counter after this call */
   int lin_iters;       /* BiCGStab iterations */
-  int lin_status;      /* 1 converged, 2 hit MAX_ITER (reference "done" codes) */
+  int lin_status;      /* 1 converged; 0 (2 with MAX_ITER = 0) ended at MAX_ITER, lin_iters then one more than were done */
   double cfl;          /* CFL used */
   double dt_min;       /* minimum local time step */
   double resid[5];     /* L1 residuals of rho, rhou(3), rhoE */
@@ -265,7 +266,7 @@ jm_status jm_sync(jm_ctx *c);
  * smaller systems take rhs - A phi throughout, as the reference.
  * Runs on stream (NULL: the default stream) and returns when done; the work
  * space (block LU, eight vectors, partials) is allocated for the call.
- * iters / status (1 converged, 2 hit max_iter) may be NULL. */
+ * iters / status (as jm_step_info's lin_iters and lin_status) may be NULL. */
 jm_status jm_block_bcgstab(int ncv, const int *nbocv_i, const int *nbocv_v, const double *A, const double *rhs,
                            double *phi, double zero_abs, double zero_rel, int max_iter, void *stream, int *iters,
                            int *status);

@@ -14,8 +14,8 @@
 // per round, on the group's stream: each kernel of the step before the
 // linear solve launched once for all solves of a kernel configuration
 // (StepBatch::pre), the block-Jacobi BiCGStab of all of them (each kernel
-// launched once for all solves, nine per iteration whatever their number,
-// with a host poll between chunks of iterations), then the update and
+// launched once for all solves, six or seven per iteration whatever their
+// number, with a host poll between chunks of iterations), then the update and
 // refresh, again one launch per kernel (StepBatch::post), and one
 // synchronisation. The tables are rebuilt only when a solve joins or
 // leaves. A solve's result is the same bits as its ordinary step's.

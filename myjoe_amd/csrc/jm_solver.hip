@@ -166,30 +166,39 @@ constexpr int kTileEval = kBlock, kTileCells = 80, kTileRows = 188, kTileEnt = 4
 constexpr unsigned kNoRow = 0xffff, kNoEntry = 0xffff;
 
 // From which size a context takes the tile forms (GPU_TILE_KERNELS = AUTO).
-// The flux: from two tiles per compute unit on (33k hexahedra, 41k
-// tetrahedra). Below that the chip is not full and a launch is as long as one
-// block's chain of loads, which is longer in k_flux_t. HLLC by entry and by
-// tiles, us: 18k hexahedra 9.0, 9.0; 39k 13.6, 11.2; 512k 122, 86; 25k
+// Making their lists costs a context 1.8 ms at 28k cells and 2.5 at 48k, so a
+// form is taken where it wins by a microsecond or more, not where it first
+// does.
+// The flux: from two tiles per compute unit on (33k hexahedra, 36k cells of
+// mixed shapes, 41k tetrahedra). Below that the chip is not full and a launch
+// is as long as one block's chain of loads, which is longer in k_flux_t. HLLC
+// by entry and by tiles, us: mixed 14k cells 8.6, 7.8; 48k 13.9, 11.9; 757k
+// 146, 112; 18k hexahedra 9.0, 9.0; 39k 13.6, 11.2; 512k 122, 86; 25k
 // tetrahedra 8.5, 8.9; 48k 11.5, 11.0; 511k 75, 63.
-constexpr int kTileMinFlux = 512;
+// (A mesh is cut to count its tiles only if it has this many entries: 512
+// tiles of hexahedra have 198k, of mixed shapes 173k, of tetrahedra 164k.)
+constexpr int kTileMinFlux = 512, kTileMinEnt = 160000;
 // The gradient: k_grad's wavefronts loop as long as their longest cell, so a
 // mesh whose cells all have as many faces keeps it up to larger sizes; a
 // Green-Gauss entry has five coefficients to stage where a least-squares one
 // has three, a viscous gradient one field more to share a row among. k_grad
 // and k_grad_t, us, least squares: mixed 20k cells 8.8, 9.4; 28k 10.7, 10.2;
-// 223k 43.7, 33.5; hexahedra 85k 16.6, 17.5; 176k 30.0, 28.8; 2M 435, 285;
-// tetrahedra 197k 24.9, 24.7. Green-Gauss: mixed 37k 11.9, 12.1; 78k 20.7,
-// 18.6; hexahedra 176k 33.3, 38.4; 512k 126, 116; tetrahedra 511k 66, 72;
-// 1.3M 228, 205. Viscous (with k_face_visc): mixed 9k 12.4, 12.8; 14k 13.9,
-// 13.1; hexahedra 39k 17.2, 17.0; 85k 32.5, 30.9; 176k 51.6, 47.5;
-// tetrahedra 105k 27.3, 29.1; 197k 42.0, 39.7; Green-Gauss, hexahedra 85k
-// 33.4, 34.9; 176k 56.3, 53.5; tetrahedra 197k 44.9, 44.2.
+// 48k 13.2, 11.3; 223k 43.7, 33.5; hexahedra 85k 16.6, 17.5; 176k 30.0, 28.8;
+// 2M 435, 285; tetrahedra 197k 24.9, 24.7; 511k 55.6, 50.3. Green-Gauss: mixed
+// 37k 11.9, 12.1; 48k 14.9, 13.8; hexahedra 176k 33.3, 38.4; 512k 126, 116;
+// tetrahedra 511k 66, 72; 1.3M 228, 205. Viscous (with k_face_visc): mixed 14k
+// 13.9, 13.1; 28k 16.4, 15.0; Green-Gauss 37k 21.5, 17.4; hexahedra 85k 32.5,
+// 30.9; 176k 51.6, 47.5; tetrahedra 105k 27.3, 29.1; 197k 42.0, 39.7;
+// Green-Gauss, hexahedra 85k 33.4, 34.9; 176k 56.3, 53.5; tetrahedra 197k
+// 44.9, 44.2.
 inline int tile_min_grad(bool uniform, bool ls, bool visc) {
-  if (!uniform) return (ls ? 24000 : 40000) / (visc ? 2 : 1);
+  if (!uniform) return visc ? 20000 : (ls ? 32000 : 40000);
   return ls ? 150000 : (visc ? 200000 : 500000);
 }
-// smaller meshes are not cut into tiles at all
-constexpr int kTileMinCells = 16384;
+// whether a context of this size may take either
+inline bool tiles_possible(size_t ncv, size_t nent) {
+  return ncv >= (size_t)tile_min_grad(false, true, true) || nent >= (size_t)kTileMinEnt;
+}
 constexpr int kRedSlots = 8;  // partial-sum slots per block for fused reductions
 inline int nblk(long long n, int b = kBlock) { return (int)((n + b - 1) / b); }
 
@@ -5110,9 +5119,15 @@ struct BcgSys {
 // solve. Implicit step of the split box, true residual against recurrence:
 // 223k cells 1598 -> 1469 us, 115k 901 -> 828, 28k 462 -> 432, 5.9k 377 -> 358.
 // Below 16 MB (14k cells of five-by-five blocks) the product costs no more
-// than its launch and the 20-40 us left are the fused update's; there the
-// solve keeps the reference's form and its bits, which small cases are
-// compared on over hundreds of steps.
+// than its launch and what is left is the fused update's 5 %; small systems
+// keep the reference's form, so that a solve follows the reference's over
+// hundreds of steps (with the recurrence a small SST case parted from the
+// oracle by 2.9e-8, where the oracle's own answer to one ulp in its input is
+// 1.2e-8). Distance of a 7-point block system's solution from the same iterate
+// in 80 bits, true residual against recurrence: 16k cells, reduction 1e-2
+// 2.8e-16, 3.2e-16; 1e-4 7.2e-16, 3.3e-16; 1e-6 1.0e-13, 3.5e-16; 84k cells,
+// 1e-6, 7.6e-14, 3.7e-16: the true residual's rounding is relative to the
+// right-hand side, the recurrence's to the residual.
 constexpr size_t kRecMinBytes = size_t(16) << 20;
 inline bool krylov_rec64(long long nnz, int nb) { return (size_t)nnz * nb * nb * sizeof(double) >= kRecMinBytes; }
 
@@ -5230,7 +5245,8 @@ void bcg_solve(const BcgSys &y, SolverScalars *hs, int &iters, int &status) {
 // Batched block-Jacobi BiCGStab for serving: the kernels above, each launched
 // once for every active solve (a block -> solve map per grid shape, each
 // solve keeping its own blocks, partials and solver scalars), so a batch
-// costs nine launches per iteration whatever the number of solves. Every
+// costs six launches per iteration whatever the number of solves (seven with
+// one that takes the true residual). Every
 // solve is cut into blocks exactly as its own solve would be and its
 // partials are finished by one block in the same order, so its result is the
 // same bits as the per-solve solver's.
@@ -6352,12 +6368,12 @@ static uint64_t morton3(double x, double y, double z) {
 void Ctx::Impl::build_tiles(const std::vector<int> &ci, const std::vector<int2> &cf, bool batched, DBuf<char> &setup,
                             const unsigned *&packed) {
   const bool any = par.tiles == kTilesAlways;
-  if (batched || par.tiles == kTilesNever || (!any && ncv < kTileMinCells)) return;
+  if (batched || par.tiles == kTilesNever) return;
   const bool visc = par.mu_ref > 0.0;
   // (a tile has room for one least-squares coefficient per cell and entry)
   grad_tiled = (par.second_order || visc) && par.grad_kernel == kResidCell && (rows_by_face || !par.grad_ls) &&
                (any || ncv >= tile_min_grad(min_faces == max_faces, par.grad_ls, visc));
-  flux_tiled = par.flux_kernel == kResidEntry && !visc;
+  flux_tiled = par.flux_kernel == kResidEntry && !visc && (any || nent >= kTileMinEnt);
   if (!grad_tiled && !flux_tiled) return;
   std::vector<Tile> tl;
   std::vector<int> stamp(ncv, -1);
@@ -7039,7 +7055,7 @@ size_t Ctx::footprint(const Mesh &m, int precision, const SolverParams &p, bool 
   b += n * (5 + 8 + 16 + 5 + 1) * 8 + nfa_b * (8 + 5) * 8;         // q, prim, grad, rhs, dt; bfa, hook
   b += visc ? n * 12 * 8 + nfa * 2 * 8 + nfa_i * 8 : 0;            // gradv, muf, fcell
   b += face ? nfa_i * (8 + 5 * 8) : 0;                             // fcell, fflux
-  if (!batched && p.tiles != kTilesNever && (p.tiles == kTilesAlways || m.ncv >= kTileMinCells))
+  if (!batched && p.tiles != kTilesNever && (p.tiles == kTilesAlways || tiles_possible(n, ent)))
     b += n * 8 + ent * (2 + 4 + 2) + (visc ? 0 : ent * 16);        // tcell; lnb, halo, headers; eval
   b += nb * nb * (nnz + n) * sJ + 10 * nb * n * sJ;                // A, LU, Krylov vectors
   b += p.ilu_sub > 0 ? nb * nb * (nnz + n) * sJ : 0;               // ILU factors
@@ -7244,7 +7260,7 @@ static void krylov_batch_iterations(hipStream_t st, const KrylovBatchBuf &buf, i
   const KrylovJob *jd = buf.jobs_d;
   double *pt = buf.partials_d, *pt1 = pt + 2 * (size_t)buf.g5;
   const int g5 = buf.g5, g1 = buf.g1, nj = buf.njobs;
-  for (int k = 0; k < count; k++) {  // six launches: alpha and omega are finished in kb_ps and kb_x_rec
+  for (int k = 0; k < count; k++) {  // alpha and omega are finished in kb_ps and kb_x_rec
     hipLaunchKernelGGL(kb_ps<T>, dim3(g1), dim3(kBlock), 0, st, jd, m1, 0, pt, g5);
     hipLaunchKernelGGL(kb_spmv_dot<T>, dim3(g5), dim3(kBlock), 0, st, jd, m5, 0, pt);
     hipLaunchKernelGGL(kb_ps<T>, dim3(g1), dim3(kBlock), 0, st, jd, m1, 1, pt, g5);
@@ -8218,7 +8234,7 @@ std::string Ctx::time_kernels(int reps, double *ms) {
 // Mean ms of the parts of an implicit step: the residual (state, BC,
 // gradients, fluxes and dt; with the coupled scalar its row), the Jacobian
 // assembly of a step (blocks, V/dt, relaxed right-hand side), the block LU
-// of the preconditioner, and one BiCGStab iteration (its nine kernels) with
+// of the preconditioner, and one BiCGStab iteration (seven to nine kernels) with
 // the stop tests switched off so that every timed iteration runs.
 std::string Ctx::time_step_kernels(int reps, double *ms) {
   Impl &d = *d_;
@@ -8916,8 +8932,8 @@ void block_bcgstab(const BlockSolve &bs, int &iters, int &status) {
 // is a stand-in, not a device address): each device's address is looked up
 // once with hipGetSymbolAddress, with that device current, and kept. Every
 // call on a device shares its array and leaves the last call's contents in
-// it; bcg_prologue clears what must start at zero (p, v) with fill kernels
-// and writes the solver scalars, LU and residuals before they are read, so
+// it; bcg_prologue clears what must start at zero (p, v: k_start) and
+// writes the solver scalars, LU and residuals before they are read, so
 // nothing carries over. Calls that overlap on one device race.
 // ---------------------------------------------------------------------------
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];

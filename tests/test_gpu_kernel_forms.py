@@ -98,7 +98,8 @@ def test_block_solver_true_residual_at_the_stop(dims):
         phi = t(guess)
         it, st = joemi.block_bcgstab(*d, phi, zero_abs=0.0, zero_rel=1e-30, max_iter=60)
         # stalled by those guards, |t| near 1e-10: at the solution to ten times that
-        assert st in (0, 1, 2) and np.max(np.abs(phi.numpy() - x)) <= 1e-9 * np.max(np.abs(x))
+        assert (st == 1 and it <= 60) or (st == 0 and it == 61)  # its limit, not before
+        assert np.max(np.abs(phi.numpy() - x)) <= 1e-9 * np.max(np.abs(x))
 
 
 # the scalar rows per entry (their off-diagonal entries written from the other
